@@ -18,6 +18,7 @@ LIB = os.path.join(HERE, "liblkgpu.so")
 
 SOURCES = [
     "lk_kernels.hip",
+    "lk_potrf.hip",
     "lk_nested.hip",
     "lk_loo.hip",
     "lk_noalloc.hip",

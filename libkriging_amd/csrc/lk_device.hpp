@@ -56,16 +56,57 @@ __device__ inline double readlane_d(double v, int lane) {
   return __hiloint2double(hi, lo);
 }
 
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+// Cross-lane reductions in the vector registers: rotations inside the 16-lane
+// rows (DPP row_ror), then the rows and the halves exchanged by
+// v_permlane16_swap / v_permlane32_swap.  A butterfly of __shfl_xor is two LDS
+// permutes and their latency per step.  Every lane gets the same value.
+template <int N>
+__device__ inline double row_ror(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x120 + N, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x120 + N, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+// (even, odd) rows' / halves' values of v in both
+__device__ inline void rows_swap16(double v, double& a, double& b) {
+  const unsigned lo = __double2loint(v), hi = __double2hiint(v);
+  const auto l2 = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  const auto h2 = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  a = __hiloint2double(h2[0], l2[0]);
+  b = __hiloint2double(h2[1], l2[1]);
+}
+__device__ inline void halves_swap32(double v, double& a, double& b) {
+  const unsigned lo = __double2loint(v), hi = __double2hiint(v);
+  const auto l2 = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  const auto h2 = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  a = __hiloint2double(h2[0], l2[0]);
+  b = __hiloint2double(h2[1], l2[1]);
+}
+
+// sum over the 16 lanes of a row
+__device__ inline double row16_sum(double v) {
+  v += row_ror<8>(v);
+  v += row_ror<4>(v);
+  v += row_ror<2>(v);
+  v += row_ror<1>(v);
   return v;
 }
 
+__device__ inline double wave_sum(double v) {
+  double a, b;
+  rows_swap16(row16_sum(v), a, b);
+  halves_swap32(a + b, a, b);
+  return a + b;
+}
+
 __device__ inline double wave_max(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-  return v;
+  v = fmax(v, row_ror<8>(v));
+  v = fmax(v, row_ror<4>(v));
+  v = fmax(v, row_ror<2>(v));
+  v = fmax(v, row_ror<1>(v));
+  double a, b;
+  rows_swap16(v, a, b);
+  halves_swap32(fmax(a, b), a, b);
+  return fmax(a, b);
 }
 
 // lower-triangular tile index t -> (i, j), i >= j, row-major over i

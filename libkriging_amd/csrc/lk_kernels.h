@@ -112,11 +112,7 @@ __host__ __device__ inline int red_rstar_off(int nblk) { return 4 * nblk + nblk 
 // cond(L_kk) up to the factor 64 (written by the diagonal-block kernel, read
 // by the panel kernel)
 __host__ __device__ inline int red_cond_off(int nblk) { return red_rstar_off(nblk) + PMAX * PMAX; }
-// per row block r >= 1 and column c of the blocks left of it: sum_i |L(i, c)|
-// over the block's rows, written by the panel kernel (r * npad + c), read
-// for ||L||_1 by k_solve_x
-__host__ __device__ inline int red_lcol_off(int nblk) { return red_cond_off(nblk) + nblk; }
-__host__ __device__ inline size_t red_size(int nblk) { return (size_t)red_lcol_off(nblk) + (size_t)nblk * nblk * NB; }
+__host__ __device__ inline size_t red_size(int nblk) { return (size_t)red_cond_off(nblk) + nblk; }
 // Panels whose diagonal block's condition estimate exceeds this get one step
 // of iterative refinement: multiplying by the explicit inverse of an
 // ill-conditioned block is not backward stable, the refined product is.
@@ -134,8 +130,10 @@ struct Batch {
 
 // Launchers (each returns the hipGetLastError of the launch).
 hipError_t launch_build(const Batch& b);
-hipError_t launch_potrf_diag(const Batch& b, int k);
-hipError_t launch_potrf_panel(const Batch& b, int k);
+// the diagonal blocks k .. k + nb - 1 (nb 1 or 2) and the tile between them
+hipError_t launch_potrf_chain(const Batch& b, int k, int nb);
+// their columns in every row block below them
+hipError_t launch_potrf_rows(const Batch& b, int k, int nb);
 // A(r, c) -= sum_{k in [kb, ke)} L(r, k) L(c, k)^T, tile columns c in [c0, c1]
 // (c1 < 0: to the last column), rows r >= c
 hipError_t launch_potrf_update(const Batch& b, int kb, int ke, int c0, int c1);
@@ -143,6 +141,9 @@ hipError_t launch_potrf_update(const Batch& b, int kb, int ke, int c0, int c1);
 hipError_t launch_potrf_update_trailing(const Batch& b, int kb, int ke, int c0);
 // the same update of a one-slot batch by `workgroups` persistent workgroups
 hipError_t launch_potrf_update_persistent(const Batch& b, int kb, int ke, int c0, int c1, int workgroups);
+// L^-1 inside the 256 x 256 diagonal blocks (the diagonal inverses given)
+hipError_t launch_trtri_base(const Batch& b);
+// recursive doubling from there: s = 4, 8, ... blocks, two products each
 hipError_t launch_trtri_level(const Batch& b, int s, int step);
 hipError_t launch_solve_fy(const Batch& b);
 hipError_t launch_gls(const Batch& b);

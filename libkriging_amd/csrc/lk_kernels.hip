@@ -11,7 +11,8 @@
 // src/lib/Kriging.cpp:214-338, and KrigingImpl::populate_Model,
 // src/lib/KrigingImpl.cpp:73-125):
 //   build           R = factor * k(x_i - x_j; theta), unit (+jitter) diagonal
-//   potrf diag/panel/update   blocked right-looking Cholesky, FP64 MFMA
+//   potrf chain/rows/update   blocked right-looking Cholesky, FP64 MFMA
+//                   (chain and rows in lk_potrf.hip)
 //   trtri           L^-1 by recursive doubling, FP64 MFMA
 //   solve_fy, gls, solve_e, solve_x   F* = L^-1 F, y* = L^-1 y, GLS beta,
 //                   E* = L^-1 (y - F beta), x = L^-T E*, |L|_1, |L^-1|_1
@@ -134,432 +135,6 @@ __global__ __launch_bounds__(TPB) void k_build(const Slot* __restrict__ slots, c
     case K_EXP: fill(std::integral_constant<int, K_EXP>{}); break;
     case K_MATERN32: fill(std::integral_constant<int, K_MATERN32>{}); break;
     default: fill(std::integral_constant<int, K_MATERN52>{}); break;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// (2a) Cholesky of the diagonal block k and its inverse, one 512-thread
-// workgroup per slot: waves 0-3 run the factor sweep, waves 4-7 the inverse
-// sweep.  Both go 4 columns / rows at a time (16 sequential steps instead of
-// 64): a 4 x 4 diagonal sub-block is factored redundantly by every factor
-// lane (lane = row) from LDS broadcasts, each lane solves its row's 4 L
-// values, and the rank-4 update of the later columns runs on MFMA
-// (V_MFMA_F64_16X16X4_F64, one 16 x 16 tile per instruction): its operands
-// are one value per lane from LDS instead of a broadcast read per updated
-// element, which kept the LDS return path the bound of the step.  Factor
-// wave w holds columns 16w .. 16w+15 of the block as four 16 x 16 MFMA
-// tiles; inverse wave w holds rows 16w .. 16w+15 of X = L_kk^-1 the same
-// way.  Pivot square roots come from v_rsq_f64 refined by one third-order
-// step.  Writes L_kk to A and L_kk^-1 to the same block of W (both with
-// zero strict upper part), the partial log-det, and flags a non-positive /
-// NaN pivot (dpotrf failure, LinearAlgebra.cpp:71).
-// ---------------------------------------------------------------------------
-__device__ inline void pivot_sqrt(double a, double& root, double& rroot) {
-  // y = v_rsq_f64(a) (relative error below 2^-22), then one third-order
-  // step: with e = 1 - a y^2, a^-1/2 = y (1 - e)^-1/2 = y (1 + e/2 + 3e^2/8
-  // + O(e^3)); two dependent operations fewer than two Newton steps
-  const double y = __builtin_amdgcn_rsq(a);
-  const double t = a * y;
-  const double e = fma(-t, y, 1.0);
-  const double p = fma(e, 0.375, 0.5);
-  const double iv = fma(y * e, p, y);
-  double s = a * iv;
-  const double r = fma(-s, s, a);
-  root = fma(r, 0.5 * iv, s);
-  rroot = iv;
-}
-
-// columns (factor) / rows (inverse) per step of the diagonal-block sweeps:
-// the K of one MFMA
-constexpr int DCW = 4;
-
-struct DiagLds {
-  // LDS layouts keep a wave's 64 lanes on consecutive doubles for every
-  // per-lane access (stride 1 writes / reads, or one broadcast address)
-  double P[2][DCW * NB];  // current values of the step's columns, [column][row]
-  double Q[4][DCW * NB];  // their L values, [column][row], one copy per factor wave
-  double L[NB * (NB + 2)];  // L_kk column-major, stride NB + 2 (16-byte aligned column pairs)
-  double X[NB * (NB + 1)];  // L_kk^-1 rows staged for coalesced stores, stride NB + 1
-  double R[2][DCW * NB];    // the step's rows of L_kk^-1 in the inverse sweep, [row][column]
-  double Z[DCW * NB];       // the inverse owner's accumulated step rows, [row][column]
-  double diag[NB], rinv[NB];
-};
-
-// MFMA tile layouts (lane l, register e; the instruction returns D(a, b) with
-// a = (l >> 4) + 4e, b = l & 15 for D = P Q, P (16 x 4) given as lane l ->
-// P(l & 15, l >> 4) and Q (4 x 16) as lane l -> Q(l >> 4, l & 15)):
-//   factor tile rb of wave W: element (16 rb + (l & 15), 16 W + (l >> 4) + 4e)
-//     (D transposed: the update's P is the wave's columns, Q the tile's rows)
-//   inverse tile cb of wave W: element (16 W + (l >> 4) + 4e, 16 cb + (l & 15))
-
-// Before the barrier of step p: the owner of the step's columns publishes
-// their current values (tile register e = (j0 & 15) / 4 holds column
-// j0 + (l >> 4) of the tile's 16 rows).  Rows above 16 W are not written:
-// no lane reads them (their L values are forced to zero).
-template <int W>
-__device__ inline void factor_publish(int p, const d4 (&T)[4], DiagLds& sh, int l) {
-  const int j0 = DCW * p;
-  if (W == j0 / 16) {
-    double* P = sh.P[p & 1];
-    const int e = (j0 & 15) / 4;
-#pragma unroll
-    for (int rb = W; rb < 4; ++rb) P[(l >> 4) * NB + 16 * rb + (l & 15)] = T[rb][e];
-  }
-}
-
-// After the barrier: the DCW x DCW diagonal sub-block (factored by every lane
-// from LDS broadcasts), this row's L values in the step's columns, then the
-// rank-DCW update of the wave's columns right of the step on MFMA; the owner
-// also writes the step's columns of L (zero above the diagonal) to sh.L, and
-// wave 0 their diagonal and reciprocal, which the inverse sweep reads two
-// steps later.
-template <int W>
-__device__ inline bool factor_step(int p, d4 (&T)[4], DiagLds& sh, int l) {
-  bool ok = true;
-  const int j0 = DCW * p;
-  const double* P = sh.P[p & 1];
-  double* Q = sh.Q[W];
-  // DCW x DCW diagonal sub-block, factored by every lane (left-looking)
-  double L4[DCW][DCW], iv[DCW];
-#pragma unroll
-  for (int r = 0; r < DCW; ++r)
-#pragma unroll
-    for (int c = 0; c <= r; ++c) L4[r][c] = P[c * NB + j0 + r];
-#pragma unroll
-  for (int c = 0; c < DCW; ++c) {
-    double d = L4[c][c];
-#pragma unroll
-    for (int m = 0; m < c; ++m) d = fma(-L4[c][m], L4[c][m], d);
-    ok = ok && (d > 0.0);
-    pivot_sqrt(d, L4[c][c], iv[c]);
-#pragma unroll
-    for (int r = c + 1; r < DCW; ++r) {
-      double t = L4[r][c];
-#pragma unroll
-      for (int m = 0; m < c; ++m) t = fma(-L4[r][m], L4[c][m], t);
-      L4[r][c] = t * iv[c];
-    }
-  }
-  // this row's L values in columns j0 .. j0+DCW-1
-  double x[DCW];
-  {
-    double v[DCW];
-#pragma unroll
-    for (int s = 0; s < DCW; ++s) v[s] = P[s * NB + l];
-#pragma unroll
-    for (int s = 0; s < DCW; ++s) {
-      double t = v[s];
-#pragma unroll
-      for (int m = 0; m < s; ++m) t = fma(-x[m], L4[s][m], t);
-      x[s] = t * iv[s];
-    }
-    // rows inside the block reproduce L4 below the diagonal (same
-    // operations); the diagonal takes the corrected root, rows above the
-    // step are zero (their published values are not meaningful).  Entries
-    // above the diagonal inside the block are left as computed: they only
-    // reach the strict upper part of the tiles' columns, which no
-    // lower-part value reads and the stores zero.
-#pragma unroll
-    for (int s = 0; s < DCW; ++s) {
-      x[s] = (l == j0 + s) ? L4[s][s] : x[s];
-      x[s] = (l < j0) ? 0.0 : x[s];
-    }
-  }
-  if (W == j0 / 16) {
-#pragma unroll
-    for (int s = 0; s < DCW; ++s) sh.L[(j0 + s) * (NB + 2) + l] = (l >= j0 + s) ? x[s] : 0.0;
-  }
-  // every wave computed the same x for all 64 rows: each keeps its own copy
-  // and reads the MFMA operands back without a workgroup barrier (one
-  // wave's LDS operations complete in order; the fences keep the compiler
-  // from moving the reads above the writes)
-#pragma unroll
-  for (int s = 0; s < DCW; ++s) Q[s * NB + l] = x[s];
-  if (W == 0 && l == 0) {
-#pragma unroll
-    for (int s = 0; s < DCW; ++s) {
-      sh.diag[j0 + s] = L4[s][s];
-      sh.rinv[j0 + s] = iv[s];
-    }
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  // tile rb -= X_rb X_W^T over the wave's columns right of the step (the
-  // P operand is zero for the columns up to j0 + DCW - 1, which stay)
-  if (W >= j0 / 16 && 16 * W + 15 >= j0 + DCW) {
-    const int c = 16 * W + (l & 15);
-    const double pv = (c >= j0 + DCW) ? -Q[(l >> 4) * NB + c] : 0.0;
-#pragma unroll
-    for (int rb = W; rb < 4; ++rb) {
-      const double qv = Q[(l >> 4) * NB + 16 * rb + (l & 15)];
-      T[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(pv, qv, T[rb], 0, 0, 0);
-    }
-  }
-  return ok;
-}
-
-// One step of the inverse sweep for wave W (owns rows 16W .. 16W+15 of
-// X = L_kk^-1), split at its barrier.  Step p solves rows j0 = DCW p ..
-// j0 + DCW - 1 (owner; lane = column) after reading the wave's MFMA operand
-// L(16W + (l & 15), j0 + (l >> 4)) for the update that follows the barrier.
-template <int W>
-__device__ inline void inverse_solve(int p, const d4 (&U)[4], double& pv, DiagLds& sh, int l) {
-  const int j0 = DCW * p;
-  double* Rr = sh.R[p & 1];
-  {
-    const int i = 16 * W + (l & 15);
-    pv = (i >= j0 + DCW) ? sh.L[(j0 + (l >> 4)) * (NB + 2) + i] : 0.0;
-  }
-  if (W == j0 / 16) {
-    // the step's rows of the accumulated sums: lane group s holds row j0 + s
-    // (register (j0 & 15) / 4 of each tile); regroup to lane = column
-    const int e = (j0 & 15) / 4;
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb) sh.Z[(l >> 4) * NB + 16 * cb + (l & 15)] = (cb <= W) ? U[cb][e] : 0.0;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    double x[DCW];
-#pragma unroll
-    for (int s = 0; s < DCW; ++s) {
-      double t = ((l == j0 + s) ? 1.0 : 0.0) - sh.Z[s * NB + l];
-#pragma unroll
-      for (int m = 0; m < s; ++m) t = fma(-sh.L[(j0 + m) * (NB + 2) + j0 + s], x[m], t);
-      x[s] = t * sh.rinv[j0 + s];
-      Rr[s * NB + l] = x[s];
-      sh.X[(j0 + s) * (NB + 1) + l] = x[s];
-    }
-  }
-}
-
-// After the barrier: tile cb += L(rows of the wave, step columns) X(step
-// rows, columns of the tile) for the wave's rows below the step (zero P
-// rows elsewhere); tiles right of the wave's rows stay zero (X is lower
-// triangular)
-template <int W>
-__device__ inline void inverse_update(int p, d4 (&U)[4], double pv, const DiagLds& sh, int l) {
-  const int j0 = DCW * p;
-  if (16 * W + 15 < j0 + DCW) return;
-  const double* Rr = sh.R[p & 1];
-#pragma unroll
-  for (int cb = 0; cb <= W; ++cb) {
-    const double qv = Rr[(l >> 4) * NB + 16 * cb + (l & 15)];
-    U[cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(pv, qv, U[cb], 0, 0, 0);
-  }
-}
-
-// The two sweeps pipelined over the workgroup's 8 waves: waves 0-3 run the
-// factor sweep, waves 4-7 the inverse sweep two steps behind it (step p of
-// the inverse reads the L columns and reciprocals that factor step p wrote,
-// one barrier earlier).  Every wave passes the same NB / DCW + 2 barriers.
-// With the factor given (factor mode), sh.L, sh.diag and sh.rinv are filled
-// before the sweep and the factor waves only keep the barrier count.
-template <int W8>
-__device__ inline bool diag_sweeps(d4 (&T)[4], DiagLds& sh, int l, bool factor_given) {
-  constexpr bool FW = W8 < 4;
-  constexpr int W = FW ? W8 : W8 - 4;
-  constexpr int NR = NB / DCW;
-  bool ok = true;
-  d4 U[4];
-#pragma unroll
-  for (int cb = 0; cb < 4; ++cb) U[cb] = d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-  for (int r = 0; r < NR + 2; ++r) {
-    double pv = 0.0;
-    if (FW) {
-      if (r < NR && !factor_given) factor_publish<W>(r, T, sh, l);
-    } else if (r >= 2) {
-      inverse_solve<W>(r - 2, U, pv, sh, l);
-    }
-    __syncthreads();
-    if (FW) {
-      if (r < NR && !factor_given) ok = factor_step<W>(r, T, sh, l) && ok;
-    } else if (r >= 2) {
-      inverse_update<W>(r - 2, U, pv, sh, l);
-    }
-  }
-  return ok;
-}
-
-constexpr int DIAG_TPB = 2 * TPB;  // 8 waves: 4 factor, 4 inverse
-
-__global__ __launch_bounds__(DIAG_TPB) void k_potrf_diag(const Slot* __restrict__ slots,
-                                                         const SlotParams* __restrict__ params,
-                                                         SlotOut* __restrict__ out, int k) {
-  const int b = blockIdx.x;
-  const Slot S = slots[b];
-  if (!slot_live(params[b], out[b]) || k >= S.nblk) return;
-  const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
-  const bool fw = w < 4;  // factor wave (else inverse wave w - 4)
-  const int k0 = k * NB;
-  const int ld = S.npad;
-  double* Ab = S.A + (size_t)k0 * ld + k0;
-  double* Wb = S.W + (size_t)k0 * ld + k0;
-  __shared__ DiagLds sh;
-  __shared__ int sbad;
-  __shared__ double smax[2][4];
-  if (tid == 0) sbad = 0;
-  const bool given = params[b].mode == MODE_FACTOR;
-
-  d4 T[4];
-#pragma unroll
-  for (int rb = 0; rb < 4; ++rb) T[rb] = d4{0.0, 0.0, 0.0, 0.0};
-  if (fw) {
-    if (given) {
-      // the block is already L_kk: its columns, diagonal and reciprocals for
-      // the inverse sweep; a non-positive or NaN diagonal entry is a failure
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int c = 16 * w + q;
-        const double v = Ab[(size_t)c * ld + l];
-        sh.L[c * (NB + 2) + l] = (l >= c) ? v : 0.0;
-        if (l == c) {
-          sh.diag[c] = v;
-          sh.rinv[c] = 1.0 / v;
-        }
-      }
-    } else {
-      // the wave's tiles on and below the diagonal (rows from 16 w)
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-        if (rb >= w)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) T[rb][e] = Ab[(size_t)(16 * w + (l >> 4) + 4 * e) * ld + 16 * rb + (l & 15)];
-    }
-  }
-  __syncthreads();
-  bool ok;
-  switch (w) {
-    case 0: ok = diag_sweeps<0>(T, sh, l, given); break;
-    case 1: ok = diag_sweeps<1>(T, sh, l, given); break;
-    case 2: ok = diag_sweeps<2>(T, sh, l, given); break;
-    case 3: ok = diag_sweeps<3>(T, sh, l, given); break;
-    case 4: ok = diag_sweeps<4>(T, sh, l, given); break;
-    case 5: ok = diag_sweeps<5>(T, sh, l, given); break;
-    case 6: ok = diag_sweeps<6>(T, sh, l, given); break;
-    default: ok = diag_sweeps<7>(T, sh, l, given); break;
-  }
-  if (given && fw && l < 16) ok = sh.diag[16 * w + l] > 0.0;
-  // every factor lane saw every pivot; in factor mode a lane checks one
-  // diagonal entry: any failure is shared through LDS before the uniform exit
-  if (fw && !ok) sbad = 1;
-  __syncthreads();
-  if (sbad) {
-    if (tid == 0) out[b].status = ST_CHOL_FAILED;
-    return;
-  }
-  if (fw) {
-    // L_kk -> A (lower, zero above), from its LDS copy (lane = row)
-    double lmax = 0.0;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int c = 16 * w + q;
-      const double v = sh.L[c * (NB + 2) + l];
-      Ab[(size_t)c * ld + l] = v;
-      lmax = fmax(lmax, fabs(v));
-    }
-    lmax = wave_max(lmax);
-    if (l == 0) smax[0][w] = lmax;
-    if (w == 0) {
-      const double ld_part = wave_sum(log(sh.diag[l]));
-      if (l == 0) S.red[RED_LOGDET + k] = ld_part;
-    }
-  } else {
-    // L_kk^-1 -> W: rows staged as sh.X[row][col]; columns written coalesced
-    // (lane = row)
-    const int wi = w - 4;
-    double xmax = 0.0;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int c = 16 * wi + q;
-      const double v = sh.X[l * (NB + 1) + c];
-      Wb[(size_t)c * ld + l] = v;
-      xmax = fmax(xmax, fabs(v));
-    }
-    xmax = wave_max(xmax);
-    if (l == 0) smax[1][wi] = xmax;
-  }
-  __syncthreads();
-  // condition estimate of L_kk for the panel kernel's refinement decision
-  if (tid == 0) {
-    const double lm = fmax(fmax(smax[0][0], smax[0][1]), fmax(smax[0][2], smax[0][3]));
-    const double xm = fmax(fmax(smax[1][0], smax[1][1]), fmax(smax[1][2], smax[1][3]));
-    S.red[red_cond_off(S.nblk) + k] = (double)NB * lm * xm;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// (2b) panel: L(r, k) = A(r, k) * L_kk^-T for row blocks r > k, as a product
-// with the explicit inverse from the diagonal-block kernel.  When the
-// diagonal block is ill-conditioned (its estimate above PANEL_REFINE_COND)
-// the product is refined once, X += (A - X L_kk^T) L_kk^-T: the product
-// alone is accurate to cond(L_kk) eps relative to |L_kk^-1|, the refined one
-// to the level of a substitution (dtrsm, as LAPACK's dpotrf uses).  The
-// unrefined X waits in W's strict upper triangle (row block k, column block
-// r: unused until the inverse is formed) while the residual is formed.
-// grid (nblk_max - k - 1, nslots), 256 threads, three waves per SIMD (a
-// few registers spilled; 64 x n = 1024 Cholesky 1.019 -> 1.007 ms against
-// two, n = 8192 7.35 -> 7.25 ms)
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(TPB, 3) void k_potrf_panel(const Slot* __restrict__ slots,
-                                                     const SlotParams* __restrict__ params,
-                                                     SlotOut* __restrict__ out, int k) {
-  const TileSlot ts = tile_slot();
-  const int b = ts.slot;
-  const Slot S = slots[b];
-  const int r = k + 1 + ts.tile;
-  if (!slot_live(params[b], out[b]) || r >= S.nblk || params[b].mode == MODE_FACTOR) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wr = w >> 1, wc = w & 1;
-  const int i0 = r * NB, k0 = k * NB, ld = S.npad;
-  __shared__ double sbuf[4 * KC * LDSS];
-  d4 acc[2][2];
-  acc_zero(acc);
-  // A(i0 + ii, k) times Dinv(c, k) at W[k * ld + k0 + c]
-  tile_mainloop<false, false, false>(S.A, ld, i0, S.W, ld, k0, k0, k0 + NB, sbuf, acc, tid, lane, wr, wc);
-  double* A21 = S.A + (size_t)k0 * ld + i0;
-  if (S.red[red_cond_off(S.nblk) + k] > PANEL_REFINE_COND) {
-    // X^T into W(k0 + c, i0 + r); the residual A21 - X L_kk^T into A21
-    acc_store_t(acc, S.W + (size_t)i0 * ld + k0, ld, lane, wr, wc);
-    d4 res[2][2];
-    acc_load(res, A21, ld, lane, wr, wc);
-    __syncthreads();
-    tile_mainloop<true, false, true>(S.W, ld, i0, S.A, ld, k0, k0, k0 + NB, sbuf, res, tid, lane, wr, wc);
-    acc_store(res, A21, ld, lane, wr, wc);
-    __syncthreads();
-    // X += residual Dinv^T
-    tile_mainloop<false, false, false>(S.A, ld, i0, S.W, ld, k0, k0, k0 + NB, sbuf, acc, tid, lane, wr, wc);
-  }
-  acc_store(acc, A21, ld, lane, wr, wc);
-  // this block's column sums of |L| for ||L||_1: rows bi in the lane, the 16
-  // lanes of a column group by shuffles, the two row waves through LDS
-  __shared__ double scol[NB];
-  double cs[2][4];
-#pragma unroll
-  for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      double v = fabs(acc[0][bj][e]) + fabs(acc[1][bj][e]);
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off, 64);
-      cs[bj][e] = v;
-    }
-  if (wr == 1 && (lane & 15) == 0) {
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) scol[acc_col(lane, wc, bj, e)] = cs[bj][e];
-  }
-  __syncthreads();
-  if (wr == 0 && (lane & 15) == 0) {
-    double* part = S.red + red_lcol_off(S.nblk) + (size_t)r * ld + k0;
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int c = acc_col(lane, wc, bj, e);
-        part[c] = cs[bj][e] + scol[c];
-      }
   }
 }
 
@@ -849,10 +424,9 @@ __global__ __launch_bounds__(MV_TPB) void k_solve_x(const Slot* __restrict__ slo
   double* x = S.V + (size_t)(S.p + 3) * ld;
   double mW = 0.0, mL = 0.0;
   // ||L||_1: L's columns are read only inside the diagonal block; below it
-  // the panel kernel's per-block column sums stand in for them (a factor
+  // the sums of 16 rows each that the Cholesky left stand in for them (a factor
   // given as input had no panel step: then all of L is read)
   const int lend = (params[b].mode == MODE_FACTOR) ? ld : (ts.tile + 1) * NB;
-  const double* lpart = S.red + red_lcol_off(S.nblk);
   // wave w takes the block's columns c0 .. c0 + CW - 1 together: one pass
   // down the rows with one load of E* and CW coalesced column loads in
   // flight per row group (the reductions run once per column at the end)
@@ -883,7 +457,9 @@ __global__ __launch_bounds__(MV_TPB) void k_solve_x(const Slot* __restrict__ slo
     double al = 0.0;
     for (int i = c + lane; i < lend; i += 64) al += fabs(gload(Ac + i));
     if (lend < ld)
-      for (int r = ts.tile + 1 + lane; r < S.nblk; r += 64) al += lpart[(size_t)r * ld + c];
+      // four partial sums per row block (lcol_part in lk_potrf.hip)
+      for (int r = 4 * (ts.tile + 1) + lane; r < 4 * S.nblk; r += 64)
+        al += S.A[(size_t)((r >> 2) * NB + (r & 3)) * ld + c];
     const double sx = wave_sum(s[q]);
     const double awx = wave_sum(aw[q]);
     al = wave_sum(al);
@@ -899,6 +475,12 @@ __global__ __launch_bounds__(MV_TPB) void k_solve_x(const Slot* __restrict__ slo
     sm[1][w] = mL;
   }
   __syncthreads();
+  // the block's share of the log-determinant, sum log L_cc
+  if (w == MV_W - 1) {
+    const int c = ts.tile * NB + lane;
+    const double t = wave_sum(log(gload(S.A + (size_t)c * ld + c)));
+    if (lane == 0) S.red[RED_LOGDET + ts.tile] = t;
+  }
   if (tid == 0) {
     double a = sm[0][0], l = sm[1][0];
     for (int q = 1; q < MV_W; ++q) {
@@ -1995,16 +1577,6 @@ hipError_t launch_build(const Batch& B) {
     hipLaunchKernelGGL(k_build<16>, grid, dim3(TPB), 0, B.stream, B.slots, B.params, B.out);
   else
     hipLaunchKernelGGL(k_build<32>, grid, dim3(TPB), 0, B.stream, B.slots, B.params, B.out);
-  return hipGetLastError();
-}
-hipError_t launch_potrf_diag(const Batch& B, int k) {
-  hipLaunchKernelGGL(k_potrf_diag, dim3(B.nslots), dim3(DIAG_TPB), 0, B.stream, B.slots, B.params, B.out, k);
-  return hipGetLastError();
-}
-hipError_t launch_potrf_panel(const Batch& B, int k) {
-  const int T = B.nblk_max - k - 1;
-  if (T <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_potrf_panel, dim3(T, B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params, B.out, k);
   return hipGetLastError();
 }
 hipError_t launch_potrf_update(const Batch& B, int kb, int ke, int c0, int c1) {

@@ -574,10 +574,24 @@ std::vector<Runtime::Step> Runtime::pipeline_steps(const Batch& B, bool want_gra
   std::vector<Step> v;
   v.push_back({1u << 0, "build", [B] { return launch_build(B); }});
   // blocked right-looking Cholesky, two levels: panels of P block columns;
-  // inside a panel each step updates only the panel's remaining columns,
+  // inside a panel each pair of columns updates only the panel's remaining columns,
   // then one trailing update with K = 64 P per panel
   const int P = panel_blocks;
   bool first_update = true;
+  // one panel: two block columns at a time, each pair's update reaching only
+  // the panel's remaining columns
+  auto panel = [&](int K0, int K1) {
+    for (int k = K0; k < K1; k += 2) {
+      const int nb = std::min(2, K1 - k);
+      v.push_back({1u << 1, "potrf_chain", [B, k, nb] { return launch_potrf_chain(B, k, nb); }});
+      v.push_back({1u << 1, "potrf_rows", [B, k, nb] { return launch_potrf_rows(B, k, nb); }});
+      if (k + nb < K1) {
+        v.push_back({(1u << 1) | (first_update ? 1u << 2 : 0u), "potrf_update (panel)",
+                     [B, k, nb, K1] { return launch_potrf_update(B, k, k + nb, k + nb, K1 - 1); }});
+        first_update = false;
+      }
+    }
+  };
   if (lookahead && B.nslots == 1 && B.nblk_max >= kLookaheadMinBlocks) {
     // look-ahead: after panel p, its update of panel p + 1's columns runs on
     // the main stream, then panel p + 1's chain (diagonal blocks, panels,
@@ -593,12 +607,7 @@ std::vector<Runtime::Step> Runtime::pipeline_steps(const Batch& B, bool want_gra
     bool pending = false;
     for (int K0 = 0; K0 < B.nblk_max; K0 += P) {
       const int K1 = std::min(K0 + P, B.nblk_max);
-      for (int k = K0; k < K1; ++k) {
-        v.push_back({1u << 1, "potrf_diag", [B, k] { return launch_potrf_diag(B, k); }});
-        v.push_back({1u << 1, "potrf_panel", [B, k] { return launch_potrf_panel(B, k); }});
-        if (k + 1 < K1)
-          v.push_back({1u << 1, "potrf_update (panel)", [B, k, K1] { return launch_potrf_update(B, k, k + 1, k + 1, K1 - 1); }});
-      }
+      panel(K0, K1);
       if (K1 >= B.nblk_max) break;
       const int K2 = std::min(K1 + P, B.nblk_max);
       if (pending) v.push_back({1u << 1, "wait bulk update", [sa, evB] { return hipStreamWaitEvent(sa, evB, 0); }});
@@ -622,15 +631,7 @@ std::vector<Runtime::Step> Runtime::pipeline_steps(const Batch& B, bool want_gra
   } else
   for (int K0 = 0; K0 < B.nblk_max; K0 += P) {
     const int K1 = std::min(K0 + P, B.nblk_max);
-    for (int k = K0; k < K1; ++k) {
-      v.push_back({1u << 1, "potrf_diag", [B, k] { return launch_potrf_diag(B, k); }});
-      v.push_back({1u << 1, "potrf_panel", [B, k] { return launch_potrf_panel(B, k); }});
-      if (k + 1 < K1) {
-        v.push_back({(1u << 1) | (first_update ? 1u << 2 : 0u), "potrf_update (panel)",
-                     [B, k, K1] { return launch_potrf_update(B, k, k + 1, k + 1, K1 - 1); }});
-        first_update = false;
-      }
-    }
+    panel(K0, K1);
     if (K1 < B.nblk_max) {
       v.push_back({(1u << 1) | (first_update ? 1u << 2 : 0u), "potrf_update (trailing)",
                    [B, K0, K1, wide] {
@@ -640,7 +641,8 @@ std::vector<Runtime::Step> Runtime::pipeline_steps(const Batch& B, bool want_gra
     }
   }
   const int lv = trtri_levels(B.nblk_max);
-  for (int l = 0; l < lv; ++l) {
+  if (lv > 0) v.push_back({1u << 3, "trtri base", [B] { return launch_trtri_base(B); }});
+  for (int l = 2; l < lv; ++l) {
     v.push_back({1u << 3, "trtri step 0", [B, l] { return launch_trtri_level(B, 1 << l, 0); }});
     v.push_back({1u << 3, "trtri step 1", [B, l] { return launch_trtri_level(B, 1 << l, 1); }});
   }
