@@ -109,6 +109,15 @@ __device__ inline double wave_max(double v) {
   return fmax(a, b);
 }
 
+// Orders one wave's LDS writes before its later reads by other lanes (a
+// wave's LDS operations complete in order; this keeps the compiler from
+// moving them)
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // lower-triangular tile index t -> (i, j), i >= j, row-major over i
 __device__ inline void tri_decode(int t, int& i, int& j) {
   int r = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);

@@ -96,6 +96,13 @@ __host__ __device__ inline int v_loo_t(int p) { return 2 * p + 11; }
 __host__ __device__ inline int v_loo_bw(int p) { return 2 * p + 12; }
 __host__ __device__ inline int v_cols(int p) { return 2 * p + 13; }
 
+// the row blocks' sums of [F* | y*]'[F* | y*] between k_solve_fy and k_gls:
+// gram_entries(p) each, in the columns the leave-one-out objective fills
+// later (p + 6 of them: 64 (p + 6) doubles per row block)
+__host__ __device__ inline int v_gram(int p) { return p + 7; }
+__host__ __device__ inline int gram_entries(int p) { return p * (p + 3) / 2; }
+static_assert(PMAX * (PMAX + 3) / 2 <= NB * (PMAX + 6), "the Gram sums fit their columns");
+
 // objective of a batched evaluation
 enum Objective { OBJ_LL = 0, OBJ_LOO = 1, OBJ_LMP = 2, OBJ_COUNT = 3 };
 
@@ -153,7 +160,6 @@ hipError_t launch_finalize_ll(const Batch& b);
 hipError_t launch_lauum_adjoint(const Batch& b);
 
 hipError_t launch_finalize_grad(const Batch& b);
-hipError_t launch_rcond_estimate(const Batch& b);
 
 int trtri_levels(int nblk);
 

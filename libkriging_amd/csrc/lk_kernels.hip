@@ -16,7 +16,7 @@
 //   trtri           L^-1 by recursive doubling, FP64 MFMA
 //   solve_fy, gls, solve_e, solve_x   F* = L^-1 F, y* = L^-1 y, GLS beta,
 //                   E* = L^-1 (y - F beta), x = L^-T E*, |L|_1, |L^-1|_1
-//   finalize_ll     log-det, SSE, LL, rcond check
+//   finalize_ll     log-det, SSE, LL, rcond check (and its 1-norm estimate)
 //   lauum_adjoint   R^-1 = L^-T L^-1 tile by tile on MFMA; each tile is
 //                   contracted at once with dR/dtheta_k recomputed from X
 //                   (all k, plus the nugget direction), never stored
@@ -318,84 +318,106 @@ __global__ __launch_bounds__(MV_TPB) void k_solve_fy(const Slot* __restrict__ sl
   const int rb = ts.tile;
   // [F | y] -> V columns 0 .. p in one pass over this row block of Linv
   lower_matvec_block(S, rb, S.F, S.n, S.n, S.p + 1, S.V, S.npad, nullptr, S.y);
+  // this row block's part of F*'F* and F*'y* (upper triangle and last column
+  // of [F* | y*]'[F* | y*], a-major), for k_gls: its columns were just
+  // written by this workgroup
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, p = S.p;
+  const double* v = S.V + rb * NB + lane;
+  double* part = S.V + (size_t)v_gram(p) * S.npad + (size_t)rb * gram_entries(p);
+  int e = 0;
+  for (int a = 0; a < p; ++a)
+    for (int c = a; c <= p; ++c, ++e)
+      if (e % MV_W == w) {
+        const double t = wave_sum(v[(size_t)a * S.npad] * v[(size_t)c * S.npad]);
+        if (lane == 0) part[e] = t;
+      }
 }
 
 // GLS: R* = chol_upper(F*'F*), beta = R*^-1 R*^-T F*'y*, r = y - F beta
-// (KrigingImpl.cpp:105-121).  One workgroup per slot.
+// (KrigingImpl.cpp:105-121).  Every workgroup adds the row blocks' Gram sums
+// and factors the p x p system for itself (one wave, lane = column), then
+// takes 256 rows of r: one pass over F instead of one per entry of F*'F* by a
+// single workgroup (n = 4096, p = 9: 194 us; n = 8192, p = 1: 40 us).
+// grid (ceil(nblk_max / 4), nslots), 256 threads
 __global__ __launch_bounds__(TPB) void k_gls(const Slot* __restrict__ slots, const SlotParams* __restrict__ params,
                                              SlotOut* __restrict__ out) {
-  const int b = blockIdx.x;
+  const int b = blockIdx.y;
   const Slot S = slots[b];
-  if (!slot_live(params[b], out[b])) return;
+  if (!slot_live(params[b], out[b]) || (int)blockIdx.x * TPB >= S.npad) return;
   const int tid = threadIdx.x, p = S.p, n = S.n, ld = S.npad;
-  __shared__ double G[PMAX * (PMAX + 1)];  // p x (p + 1): [F*'F* | F*'y*]
+  __shared__ double G[PMAX * (PMAX + 1)];  // p x (p + 1): [F*'F* | F*'y*], then [R* | R*^-T F*'y*]
   __shared__ double part[TPB];
   __shared__ double beta[PMAX];
-  for (int a = 0; a < p; ++a)
-    for (int c = a; c <= p; ++c) {  // column c == p is F*'y*
-      double s = 0.0;
-      for (int i = tid; i < n; i += TPB) s = fma(S.V[(size_t)a * ld + i], S.V[(size_t)c * ld + i], s);
-      part[tid] = s;
-      __syncthreads();
-      for (int h = TPB / 2; h > 0; h >>= 1) {
-        if (tid < h) part[tid] += part[tid + h];
-        __syncthreads();
-      }
-      if (tid == 0) G[a + c * PMAX] = part[0];
-      __syncthreads();
+  const int ne = gram_entries(p);
+  const double* gram = S.V + (size_t)v_gram(p) * ld;
+  // entry e of the sums at G(a, c); consecutive threads take consecutive
+  // entries, and with fewer entries than threads the row blocks are dealt to
+  // np groups of threads whose sums are added in order
+  const int np = (ne >= TPB || ne == 0) ? 1 : TPB / ne;
+  for (int e0 = 0; e0 < ne; e0 += TPB) {
+    const int e = e0 + tid % (np > 1 ? ne : TPB), g = np > 1 ? tid / ne : 0;
+    double s = 0.0;
+    if (e < ne && g < np)
+      for (int q = g; q < S.nblk; q += np) s += gload(gram + (size_t)q * ne + e);
+    part[tid] = s;
+    __syncthreads();
+    if (e < ne && g == 0) {
+      for (int q = 1; q < np; ++q) s += part[tid + q * ne];
+      int a = 0, r = e;
+      while (r > p - a) r -= p - a + 1, ++a;
+      G[a + (a + r) * PMAX] = s;
     }
-  if (tid == 0) {
-    // upper Cholesky U'U = G (stored in place in the upper triangle)
+    __syncthreads();
+  }
+  if (tid < 64) {
+    // upper Cholesky in place, row by row: lane c has column c; column p
+    // becomes R*^-T F*'y* on the way
     bool ok = true;
+    const int c = tid;
     for (int j = 0; j < p; ++j) {
-      double s = G[j + j * PMAX];
-      for (int q = 0; q < j; ++q) s -= G[q + j * PMAX] * G[q + j * PMAX];
-      ok = ok && (s > 0.0);
-      const double ujj = sqrt(s);
-      G[j + j * PMAX] = ujj;
-      for (int c = j + 1; c < p; ++c) {
-        double t = G[j + c * PMAX];
-        for (int q = 0; q < j; ++q) t -= G[q + j * PMAX] * G[q + c * PMAX];
-        G[j + c * PMAX] = t / ujj;
+      const double d = G[j + j * PMAX];
+      ok = ok && (d > 0.0);
+      const double ujj = sqrt(d);
+      double u = 0.0;
+      if (c >= j && c <= p) u = (c == j) ? ujj : G[j + c * PMAX] / ujj;
+      wave_lds_fence();
+      if (c >= j && c <= p) G[j + c * PMAX] = u;
+      wave_lds_fence();
+      if (c > j && c <= p)
+        for (int i = j + 1; i < p && i <= c; ++i) G[i + c * PMAX] = fma(-G[j + i * PMAX], u, G[i + c * PMAX]);
+      wave_lds_fence();
+    }
+    // R* beta = z, lane c holds z_c
+    double z = (c < p) ? G[c + p * PMAX] : 0.0;
+    for (int a = p - 1; a >= 0; --a) {
+      const double ba = __shfl(z, a, 64) / G[a + a * PMAX];
+      if (c == a) z = ba;
+      if (c < a) z = fma(-G[c + a * PMAX], ba, z);
+    }
+    if (c < p) beta[c] = z;
+    if (blockIdx.x == 0) {
+      if (c < p) out[b].beta[c] = z;
+      double* rs = S.red + red_rstar_off(S.nblk);
+      for (int q = 0; q < p; ++q)
+        if (c < p) rs[c + q * p] = (c <= q) ? G[c + q * PMAX] : 0.0;
+      const double ldr = wave_sum(c < p ? log(G[c + c * PMAX]) : 0.0);
+      if (c == 0) {
+        out[b].logdet_rstar = ldr;
+        if (!ok) out[b].status = ST_CHOL_FAILED;
       }
     }
-    // beta: U' z = h, U beta = z
-    double z[PMAX];
-    for (int a = 0; a < p; ++a) {
-      double t = G[a + p * PMAX];
-      for (int q = 0; q < a; ++q) t -= G[q + a * PMAX] * z[q];
-      z[a] = t / G[a + a * PMAX];
-    }
-    for (int a = p - 1; a >= 0; --a) {
-      double t = z[a];
-      for (int q = a + 1; q < p; ++q) t -= G[a + q * PMAX] * z[q];
-      z[a] = t / G[a + a * PMAX];
-    }
-    for (int a = 0; a < p; ++a) {
-      beta[a] = z[a];
-      out[b].beta[a] = z[a];
-    }
-    double* rs = S.red + red_rstar_off(S.nblk);
-    double ldr = 0.0;
-    for (int c = 0; c < p; ++c) {
-      ldr += log(G[c + c * PMAX]);
-      for (int a = 0; a < p; ++a) rs[a + c * p] = (a <= c) ? G[a + c * PMAX] : 0.0;
-    }
-    out[b].logdet_rstar = ldr;
-    if (!ok) out[b].status = ST_CHOL_FAILED;
   }
   __syncthreads();
   // residual r = y - F beta into V column p + 1 (zero in padded rows)
-  double* r = S.V + (size_t)(p + 1) * ld;
-  for (int i = tid; i < ld; i += TPB) {
-    double v = 0.0;
-    if (i < n) {
-      double s = 0.0;
-      for (int a = 0; a < p; ++a) s = fma(S.F[(size_t)a * n + i], beta[a], s);
-      v = S.y[i] - s;
-    }
-    r[i] = v;
+  const int i = blockIdx.x * TPB + tid;
+  if (i >= ld) return;
+  double v = 0.0;
+  if (i < n) {
+    double s = 0.0;
+    for (int a = 0; a < p; ++a) s = fma(S.F[(size_t)a * n + i], beta[a], s);
+    v = S.y[i] - s;
   }
+  S.V[(size_t)(p + 1) * ld + i] = v;
 }
 
 // E* = Linv r, SSE partials
@@ -490,82 +512,6 @@ __global__ __launch_bounds__(MV_TPB) void k_solve_x(const Slot* __restrict__ slo
     S.red[red_colW_off(S.nblk) + ts.tile] = a;
     S.red[red_colL_off(S.nblk) + ts.tile] = l;
   }
-}
-
-// ---------------------------------------------------------------------------
-// (5) LL value and condition check (Kriging.cpp:247-289,
-// LinearAlgebra.cpp:68-115).  One thread per slot.
-// ---------------------------------------------------------------------------
-__global__ void k_finalize_ll(const Slot* __restrict__ slots, const SlotParams* __restrict__ params,
-                              SlotOut* __restrict__ out, int nslots) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nslots) return;
-  const Slot S = slots[b];
-  const SlotParams& P = params[b];
-  SlotOut& O = out[b];
-  if (!slot_live(P, O)) return;
-  const int nb = S.nblk;
-  double logdet = 0.0, sse = 0.0, nL = 0.0, nW = 0.0;
-  for (int q = 0; q < nb; ++q) {
-    logdet += S.red[RED_LOGDET + q];
-    sse += S.red[red_sse_off(nb) + q];
-    nL = fmax(nL, S.red[red_colL_off(nb) + q]);
-    nW = fmax(nW, S.red[red_colW_off(nb) + q]);
-  }
-  const double n = (double)S.n;
-  const double two_pi = 2.0 * 3.14159265358979323846;
-  O.logdet = logdet;
-  O.sse = sse;
-  O.norm1_L = nL;
-  O.norm1_Linv = nW;
-  const double rc = (1.0 / nL) / nW;
-  O.rcond2 = rc * rc;
-  if (P.rcond_check && !(O.rcond2 >= P.min_rcond) && O.status == ST_OK)
-    O.status = ST_RCOND_SUSPECT;
-  // a given factor: rcond from the 1-norm estimator, as arma::rcond
-  if (P.mode == MODE_FACTOR && O.status == ST_OK) O.status = ST_RCOND_SUSPECT;
-  double ll, s2g;
-  if (P.objective == OBJ_LMP) {
-    // log marginal likelihood of Kriging::_logMargPost (Kriging.cpp:560-583),
-    // S_2 = y'R^-1 y - y'P y = SSE; the prior term is added by the host
-    const double nmp = n - S.p;
-    if (S.noise == NOISE_NUGGET) {
-      if (P.est_sigma2 && P.est_nugget) s2g = sse / nmp;
-      else if (P.est_sigma2 || P.est_nugget) s2g = P.sigma2 / P.alpha;
-      else s2g = P.sigma2 + P.nugget;
-    } else {
-      s2g = P.est_sigma2 ? sse / nmp : P.sigma2;
-    }
-    O.ll = -logdet - O.logdet_rstar - 0.5 * nmp * log(s2g * nmp);
-    O.sigma2 = s2g;
-    return;
-  }
-  if (S.noise == NOISE_NUGGET) {
-    const double a = P.alpha;
-    double s2 = P.sigma2, nug = P.nugget;
-    if (P.est_sigma2) {
-      if (P.est_nugget) {
-        const double var = sse / n;
-        s2 = a * var;
-        nug = (1.0 - a) * var;
-      } else {
-        s2 = P.nugget * a / (1.0 - a);
-      }
-    } else if (P.est_nugget) {
-      nug = P.sigma2 * (1.0 - a) / a;
-    }
-    const double tv = s2 + nug;
-    ll = -0.5 * (n * log(two_pi * tv) + 2.0 * logdet + sse / tv);
-    s2g = tv;
-  } else if (P.est_sigma2) {
-    s2g = sse / n;
-    ll = -0.5 * (n * log(two_pi * s2g) + 2.0 * logdet + n);
-  } else {
-    s2g = P.sigma2;
-    ll = -0.5 * (n * log(two_pi * s2g) + 2.0 * logdet + sse / s2g);
-  }
-  O.ll = ll;
-  O.sigma2 = s2g;
 }
 
 // ---------------------------------------------------------------------------
@@ -975,7 +921,7 @@ __global__ __launch_bounds__(FG_TPB) void k_finalize_grad(const Slot* __restrict
 }
 
 // ---------------------------------------------------------------------------
-// (8) 1-norm estimate of Linv (Higham, ACM TOMS 14 (1988) 381-396, Alg. 4.1
+// (8) LL value, and the 1-norm estimate of Linv (Higham, ACM TOMS 14 (1988) 381-396, Alg. 4.1
 // with the alternating-sign extra estimate), run only for slots whose exact
 // rcond fell below the threshold.  The estimate never exceeds the exact norm,
 // so an exact rcond above the threshold implies the estimate-based one is
@@ -1001,15 +947,115 @@ __device__ void est_upper_mv(const Slot& S, const double* __restrict__ in, doubl
   }
 }
 
-__global__ __launch_bounds__(TPB) void k_rcond_estimate(const Slot* __restrict__ slots,
+// ---------------------------------------------------------------------------
+// (5) LL value and condition check (Kriging.cpp:247-289,
+// LinearAlgebra.cpp:68-115), by one thread, from the row blocks' sums and
+// maxima.
+// ---------------------------------------------------------------------------
+__device__ inline void finalize_ll(const Slot& S, const SlotParams& P, SlotOut& O, double logdet, double sse,
+                                   double nL, double nW) {
+  const double n = (double)S.n;
+  const double two_pi = 2.0 * 3.14159265358979323846;
+  O.logdet = logdet;
+  O.sse = sse;
+  O.norm1_L = nL;
+  O.norm1_Linv = nW;
+  const double rc = (1.0 / nL) / nW;
+  O.rcond2 = rc * rc;
+  if (P.rcond_check && !(O.rcond2 >= P.min_rcond) && O.status == ST_OK)
+    O.status = ST_RCOND_SUSPECT;
+  // a given factor: rcond from the 1-norm estimator, as arma::rcond
+  if (P.mode == MODE_FACTOR && O.status == ST_OK) O.status = ST_RCOND_SUSPECT;
+  double ll, s2g;
+  if (P.objective == OBJ_LMP) {
+    // log marginal likelihood of Kriging::_logMargPost (Kriging.cpp:560-583),
+    // S_2 = y'R^-1 y - y'P y = SSE; the prior term is added by the host
+    const double nmp = n - S.p;
+    if (S.noise == NOISE_NUGGET) {
+      if (P.est_sigma2 && P.est_nugget) s2g = sse / nmp;
+      else if (P.est_sigma2 || P.est_nugget) s2g = P.sigma2 / P.alpha;
+      else s2g = P.sigma2 + P.nugget;
+    } else {
+      s2g = P.est_sigma2 ? sse / nmp : P.sigma2;
+    }
+    O.ll = -logdet - O.logdet_rstar - 0.5 * nmp * log(s2g * nmp);
+    O.sigma2 = s2g;
+    return;
+  }
+  if (S.noise == NOISE_NUGGET) {
+    const double a = P.alpha;
+    double s2 = P.sigma2, nug = P.nugget;
+    if (P.est_sigma2) {
+      if (P.est_nugget) {
+        const double var = sse / n;
+        s2 = a * var;
+        nug = (1.0 - a) * var;
+      } else {
+        s2 = P.nugget * a / (1.0 - a);
+      }
+    } else if (P.est_nugget) {
+      nug = P.sigma2 * (1.0 - a) / a;
+    }
+    const double tv = s2 + nug;
+    ll = -0.5 * (n * log(two_pi * tv) + 2.0 * logdet + sse / tv);
+    s2g = tv;
+  } else if (P.est_sigma2) {
+    s2g = sse / n;
+    ll = -0.5 * (n * log(two_pi * s2g) + 2.0 * logdet + n);
+  } else {
+    s2g = P.sigma2;
+    ll = -0.5 * (n * log(two_pi * s2g) + 2.0 * logdet + sse / s2g);
+  }
+  O.ll = ll;
+  O.sigma2 = s2g;
+}
+
+// One workgroup per slot: the sums above, finalize_ll, and the estimate where
+// it is needed.
+__global__ __launch_bounds__(TPB) void k_finalize_ll(const Slot* __restrict__ slots,
                                                         const SlotParams* __restrict__ params,
                                                         SlotOut* __restrict__ out) {
   const int b = blockIdx.x;
   const Slot S = slots[b];
   const SlotParams& P = params[b];
   SlotOut& O = out[b];
-  if (!P.active || O.status != ST_RCOND_SUSPECT) return;
+  if (!slot_live(P, O)) return;
   const int n = S.n, ld = S.npad, tid = threadIdx.x;
+  __shared__ double sred[4][TPB / 64];
+  __shared__ int suspect;
+  {
+    const int nb = S.nblk, lane = tid & 63, w = tid >> 6;
+    double logdet = 0.0, sse = 0.0, nL = 0.0, nW = 0.0;
+    for (int q = tid; q < nb; q += TPB) {
+      logdet += S.red[RED_LOGDET + q];
+      sse += S.red[red_sse_off(nb) + q];
+      nL = fmax(nL, S.red[red_colL_off(nb) + q]);
+      nW = fmax(nW, S.red[red_colW_off(nb) + q]);
+    }
+    logdet = wave_sum(logdet);
+    sse = wave_sum(sse);
+    nL = wave_max(nL);
+    nW = wave_max(nW);
+    if (lane == 0) {
+      sred[0][w] = logdet;
+      sred[1][w] = sse;
+      sred[2][w] = nL;
+      sred[3][w] = nW;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      for (int q = 1; q < TPB / 64; ++q) {
+        logdet += sred[0][q];
+        sse += sred[1][q];
+        nL = fmax(nL, sred[2][q]);
+        nW = fmax(nW, sred[3][q]);
+      }
+      finalize_ll(S, P, O, logdet, sse, nL, nW);
+      suspect = O.status == ST_RCOND_SUSPECT;
+    }
+    __syncthreads();
+  }
+  if (!suspect) return;
   double* x = S.V + (size_t)(S.p + 4) * ld;
   double* xi = S.V + (size_t)(S.p + 5) * ld;
   double* y = S.V + (size_t)(S.p + 6) * ld;
@@ -1635,7 +1681,7 @@ hipError_t launch_solve_fy(const Batch& B) {
   return hipGetLastError();
 }
 hipError_t launch_gls(const Batch& B) {
-  hipLaunchKernelGGL(k_gls, dim3(B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params, B.out);
+  hipLaunchKernelGGL(k_gls, dim3((B.nblk_max + 3) / 4, B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params, B.out);
   return hipGetLastError();
 }
 hipError_t launch_solve_e(const Batch& B) {
@@ -1647,8 +1693,7 @@ hipError_t launch_solve_x(const Batch& B) {
   return hipGetLastError();
 }
 hipError_t launch_finalize_ll(const Batch& B) {
-  hipLaunchKernelGGL(k_finalize_ll, dim3((B.nslots + 63) / 64), dim3(64), 0, B.stream, B.slots, B.params, B.out,
-                     B.nslots);
+  hipLaunchKernelGGL(k_finalize_ll, dim3(B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params, B.out);
   return hipGetLastError();
 }
 template <bool LMP>
@@ -1681,9 +1726,4 @@ hipError_t launch_finalize_grad(const Batch& B) {
   hipLaunchKernelGGL(k_finalize_grad, dim3(B.nslots), dim3(FG_TPB), 0, B.stream, B.slots, B.params, B.out, B.nslots);
   return hipGetLastError();
 }
-hipError_t launch_rcond_estimate(const Batch& B) {
-  hipLaunchKernelGGL(k_rcond_estimate, dim3(B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params, B.out);
-  return hipGetLastError();
-}
-
 }  // namespace lk

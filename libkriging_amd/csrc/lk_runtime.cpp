@@ -651,7 +651,6 @@ std::vector<Runtime::Step> Runtime::pipeline_steps(const Batch& B, bool want_gra
   v.push_back({1u << 4, "solve_e", [B] { return launch_solve_e(B); }});
   v.push_back({1u << 4, "solve_x", [B] { return launch_solve_x(B); }});
   v.push_back({1u << 4, "finalize_ll", [B] { return launch_finalize_ll(B); }});
-  v.push_back({1u << 4, "rcond_estimate", [B] { return launch_rcond_estimate(B); }});
   if (objective == OBJ_LOO) {
     // leave-one-out value (diag B from the columns of L^-1), then its
     // gradient: B w, Bs = B diag(sqrt a) into A, Bs Bs' contracted with dR
