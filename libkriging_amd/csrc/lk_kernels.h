@@ -132,9 +132,16 @@ struct Batch {
   int nslots;
   int nblk_max;             // grid extent (max nblk over slots)
   int dmax;                 // max d over slots (selects the unrolled kernel variant)
+  // pinned host tables of the same slots: the parameters are read and the
+  // results written by kernels of the pipeline; null: the caller copies
+  const SlotParams* host_params = nullptr;
+  SlotOut* host_out = nullptr;
   hipStream_t stream;
 };
 
+// parameters from and results to the pinned host tables (no-ops without)
+hipError_t launch_params_in(const Batch& b);
+hipError_t launch_results_out(const Batch& b);
 // Launchers (each returns the hipGetLastError of the launch).
 hipError_t launch_build(const Batch& b);
 // the diagonal blocks k .. k + nb - 1 (nb 1 or 2) and the tile between them

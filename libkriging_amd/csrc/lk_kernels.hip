@@ -33,6 +33,39 @@
 namespace lk {
 
 // ---------------------------------------------------------------------------
+// (0) Parameters in, results out: one wave per slot reads its parameters from
+// (writes its results to) pinned host memory.  As launches of the captured
+// pipeline these replace a copy before it and one after it, each its own
+// submission with 8 - 12 us between it and the kernels (n = 200: 20 us of a
+// 225 us evaluation).  grid (nslots), 64 threads
+// ---------------------------------------------------------------------------
+static_assert(sizeof(SlotParams) % 4 == 0 && sizeof(SlotOut) % 8 == 0, "copied by words");
+__global__ __launch_bounds__(64) void k_params_in(const SlotParams* __restrict__ host, SlotParams* __restrict__ params) {
+  const int* src = reinterpret_cast<const int*>(host + blockIdx.x);
+  int* dst = reinterpret_cast<int*>(params + blockIdx.x);
+  for (int i = threadIdx.x; i < (int)(sizeof(SlotParams) / 4); i += 64) dst[i] = src[i];
+}
+__device__ inline void result_out(const SlotOut* out, SlotOut* host, int tid, int nthreads) {
+  const double* src = reinterpret_cast<const double*>(out);
+  double* dst = reinterpret_cast<double*>(host);
+  for (int i = tid; i < (int)(sizeof(SlotOut) / 8); i += nthreads) dst[i] = src[i];
+}
+__global__ __launch_bounds__(64) void k_results_out(const SlotOut* __restrict__ out, SlotOut* __restrict__ host) {
+  result_out(out + blockIdx.x, host + blockIdx.x, threadIdx.x, 64);
+}
+hipError_t launch_params_in(const Batch& B) {
+  if (B.host_params == nullptr) return hipSuccess;
+  hipLaunchKernelGGL(k_params_in, dim3(B.nslots), dim3(64), 0, B.stream, B.host_params,
+                     const_cast<SlotParams*>(B.params));
+  return hipGetLastError();
+}
+hipError_t launch_results_out(const Batch& B) {
+  if (B.host_out == nullptr) return hipSuccess;
+  hipLaunchKernelGGL(k_results_out, dim3(B.nslots), dim3(64), 0, B.stream, B.out, B.host_out);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // (1) covariance build: lower 64 x 64 tiles (diagonal tiles in full)
 // grid (ntiles(nblk_max), nslots), 256 threads
 // ---------------------------------------------------------------------------
@@ -836,15 +869,7 @@ __global__ __launch_bounds__(FG1_TPB) void k_grad_groups(const Slot* __restrict_
   }
 }
 
-__global__ __launch_bounds__(FG_TPB) void k_finalize_grad(const Slot* __restrict__ slots,
-                                                          const SlotParams* __restrict__ params,
-                                                          SlotOut* __restrict__ out, int nslots) {
-  const int b = blockIdx.x;
-  if (b >= nslots) return;
-  const Slot S = slots[b];
-  const SlotParams& P = params[b];
-  SlotOut& O = out[b];
-  if (!slot_live(P, O) || !P.want_grad) return;
+__device__ inline void finalize_grad(const Slot& S, const SlotParams& P, SlotOut& O) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int ntiles = S.nblk * (S.nblk + 1) / 2;
   constexpr int NW = FG_TPB / 64;
@@ -918,6 +943,21 @@ __global__ __launch_bounds__(FG_TPB) void k_finalize_grad(const Slot* __restrict
     }
     O.grad[d] = ga;
   }
+}
+
+// with `host`, also the last launch of the pipeline: every slot's results
+// (failed and inactive ones' status too) to the pinned table
+__global__ __launch_bounds__(FG_TPB) void k_finalize_grad(const Slot* __restrict__ slots,
+                                                          const SlotParams* __restrict__ params,
+                                                          SlotOut* __restrict__ out, SlotOut* __restrict__ host) {
+  const int b = blockIdx.x;
+  if (slot_live(params[b], out[b]) && params[b].want_grad) {
+    const Slot S = slots[b];
+    finalize_grad(S, params[b], out[b]);
+  }
+  if (host == nullptr) return;
+  __syncthreads();
+  result_out(out + b, host + b, threadIdx.x, FG_TPB);
 }
 
 // ---------------------------------------------------------------------------
@@ -1723,7 +1763,7 @@ hipError_t launch_finalize_grad(const Batch& B) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k_finalize_grad, dim3(B.nslots), dim3(FG_TPB), 0, B.stream, B.slots, B.params, B.out, B.nslots);
+  hipLaunchKernelGGL(k_finalize_grad, dim3(B.nslots), dim3(FG_TPB), 0, B.stream, B.slots, B.params, B.out, B.host_out);
   return hipGetLastError();
 }
 }  // namespace lk

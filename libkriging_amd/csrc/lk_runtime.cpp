@@ -150,12 +150,16 @@ void Runtime::set_streams(int S) {
   streams_ = S;
 }
 
+void Runtime::drop_graphs() {
+  for (auto& g : graphs_) hipGraphExecDestroy(g.exec);
+  graphs_.clear();
+}
+
 Runtime::~Runtime() {
   hipSetDevice(device_);
   for (auto& e : tev_)
     if (e) hipEventDestroy(e);
-  for (auto& g : graphs_)
-    if (g.exec) hipGraphExecDestroy(g.exec);
+  drop_graphs();
   for (auto& kv : problems_) {
     hipFree(kv.second.X);
     hipFree(kv.second.y);
@@ -168,6 +172,7 @@ Runtime::~Runtime() {
   if (d_out_) hipFree(d_out_);
   if (h_params_) hipHostFree(h_params_);
   if (h_out_) hipHostFree(h_out_);
+  if (h_slots_pin_) hipHostFree(h_slots_pin_);
   if (fork_) hipEventDestroy(fork_);
   for (auto& e : la_ev_)
     if (e) hipEventDestroy(e);
@@ -519,6 +524,8 @@ void Runtime::ensure_slots(const std::vector<EvalRequest>& reqs) {
     S.noise = P.noise;
   }
   if (!noalloc_ && (size_t)ns > slot_cap_) {
+    drop_graphs();  // they read these tables
+    if (h_slots_pin_) hipHostFree(h_slots_pin_);
     if (d_slots_) hipFree(d_slots_);
     if (d_params_) hipFree(d_params_);
     if (d_out_) hipFree(d_out_);
@@ -528,11 +535,20 @@ void Runtime::ensure_slots(const std::vector<EvalRequest>& reqs) {
     hip_check(hipMalloc(&d_slots_, sizeof(Slot) * cap), "hipMalloc slots");
     hip_check(hipMalloc(&d_params_, sizeof(SlotParams) * cap), "hipMalloc params");
     hip_check(hipMalloc(&d_out_, sizeof(SlotOut) * cap), "hipMalloc out");
-    hip_check(hipHostMalloc(&h_params_, sizeof(SlotParams) * cap, hipHostMallocDefault), "hipHostMalloc params");
-    hip_check(hipHostMalloc(&h_out_, sizeof(SlotOut) * cap), "hipHostMalloc out");
+    hip_check(hipHostMalloc(&h_params_, sizeof(SlotParams) * cap, hipHostMallocCoherent),
+              "hipHostMalloc params");
+    hip_check(hipHostMalloc(&h_out_, sizeof(SlotOut) * cap, hipHostMallocCoherent), "hipHostMalloc out");
+    hip_check(hipHostMalloc(&h_slots_pin_, sizeof(Slot) * cap), "hipHostMalloc slots");
     slot_cap_ = cap;
   }
-  hip_check(hipMemcpy(d_slots_, h_slots_.data(), sizeof(Slot) * ns, hipMemcpyHostToDevice), "upload slots");
+  if (noalloc_) {
+    hip_check(hipMemcpy(d_slots_, h_slots_.data(), sizeof(Slot) * ns, hipMemcpyHostToDevice), "upload slots");
+  } else {
+    // (the stream was idle above, and every evaluation ends synchronised)
+    std::memcpy(h_slots_pin_, h_slots_.data(), sizeof(Slot) * ns);
+    hip_check(hipMemcpyAsync(d_slots_, h_slots_pin_, sizeof(Slot) * ns, hipMemcpyHostToDevice, stream_),
+              "upload slots");
+  }
   // contiguous slot range of each bucket present; more than kMaxStreams
   // buckets: the smallest adjacent ones merged
   std::vector<Part> parts;
@@ -557,7 +573,6 @@ void Runtime::ensure_slots(const std::vector<EvalRequest>& reqs) {
   nslots_ = ns;
   nblk_max_ = nblk_max;
   dmax_ = dmax;
-  ++layout_version_;
 }
 
 // The pipeline as an ordered list of launches, each tagged with the stages
@@ -572,6 +587,7 @@ void Runtime::apply_tuning(Part& q) const {
 std::vector<Runtime::Step> Runtime::pipeline_steps(const Batch& B, bool want_grad, int objective,
                                                    int panel_blocks, int wide, bool lookahead) const {
   std::vector<Step> v;
+  if (B.host_params != nullptr) v.push_back({0u, "params in", [B] { return launch_params_in(B); }});
   v.push_back({1u << 0, "build", [B] { return launch_build(B); }});
   // blocked right-looking Cholesky, two levels: panels of P block columns;
   // inside a panel each pair of columns updates only the panel's remaining columns,
@@ -663,6 +679,7 @@ std::vector<Runtime::Step> Runtime::pipeline_steps(const Batch& B, bool want_gra
       v.push_back({1u << 5, "loo_adjoint", [B] { return launch_loo_adjoint(B); }});
       v.push_back({0u, "loo_finalize_grad", [B] { return launch_loo_finalize_grad(B); }});
     }
+    if (B.host_out != nullptr) v.push_back({0u, "results out", [B] { return launch_results_out(B); }});
     return v;
   }
   if (objective == OBJ_LMP) {
@@ -672,12 +689,16 @@ std::vector<Runtime::Step> Runtime::pipeline_steps(const Batch& B, bool want_gra
       v.push_back({1u << 5, "loo_g", [B] { return launch_loo_g(B); }});
       v.push_back({1u << 5, "lmp_adjoint", [B] { return launch_lmp_adjoint(B); }});
       v.push_back({0u, "finalize_grad", [B] { return launch_finalize_grad(B); }});
+    } else if (B.host_out != nullptr) {
+      v.push_back({0u, "results out", [B] { return launch_results_out(B); }});
     }
     return v;
   }
   if (want_grad) {
     v.push_back({1u << 5, "lauum_adjoint", [B] { return launch_lauum_adjoint(B); }});
     v.push_back({0u, "finalize_grad", [B] { return launch_finalize_grad(B); }});
+  } else if (B.host_out != nullptr) {
+    v.push_back({0u, "results out", [B] { return launch_results_out(B); }});
   }
   return v;
 }
@@ -771,6 +792,8 @@ Batch Runtime::part_batch(const Part& q, hipStream_t s) const {
   B.nslots = q.count;
   B.nblk_max = q.nblk_max;
   B.dmax = q.dmax;
+  B.host_params = noalloc_ ? nullptr : h_params_ + q.first;
+  B.host_out = noalloc_ ? nullptr : h_out_ + q.first;
   B.stream = s;
   return B;
 }
@@ -793,8 +816,9 @@ void Runtime::issue_split(const std::vector<Step>* parts, int S) {
 }
 
 void Runtime::run_pipeline(bool want_grad, BenchMap* bench, int objective) {
-  hip_check(hipMemcpyAsync(d_params_, h_params_, sizeof(SlotParams) * nslots_, hipMemcpyHostToDevice, stream_),
-            "upload params");
+  if (noalloc_)  // host arrays that are not pinned; else a kernel of the pipeline reads them
+    hip_check(hipMemcpyAsync(d_params_, h_params_, sizeof(SlotParams) * nslots_, hipMemcpyHostToDevice, stream_),
+              "upload params");
   Part all{0, nslots_, nblk_max_, dmax_};
   apply_tuning(all);
   const bool la = lookahead_active();
@@ -828,11 +852,28 @@ void Runtime::run_pipeline(bool want_grad, BenchMap* bench, int objective) {
     hipEventDestroy(e1);
   } else if (use_graph && !noalloc_ && !la) {
     if (objective < 0 || objective >= OBJ_COUNT) throw std::invalid_argument("unknown objective");
-    GraphEntry& G = graphs_[2 * objective + (want_grad ? 1 : 0)];
-    if (G.version != layout_version_ || G.exec == nullptr || G.timed_stage != timed_stage_ || G.split != S) {
-      if (G.exec) hip_check(hipGraphExecDestroy(G.exec), "graph exec destroy");
-      G.exec = nullptr;
+    // A graph holds its launches' grids and the addresses of the tables they
+    // read; which design a slot evaluates and where it works are in the
+    // tables.  So one graph serves every batch that is cut into the same
+    // parts: a program that goes from one design to another of its size
+    // captures nothing again (n = 200: 90 us, 64 x n = 1024: 150 us).
+    GraphKey key;
+    key.tables[0] = d_slots_;
+    key.tables[1] = d_params_;
+    key.tables[2] = d_out_;
+    key.tables[3] = h_params_;
+    key.tables[4] = h_out_;
+    key.objective = objective;
+    key.want_grad = want_grad;
+    key.timed_stage = timed ? timed_stage_ : -1;
+    for (const Part& q : plan)
+      for (int v : {q.first, q.count, q.nblk_max, q.dmax, q.panel_blocks, q.wide}) key.parts.push_back(v);
+    auto it = std::find_if(graphs_.begin(), graphs_.end(), [&](const GraphEntry& g) { return g.key == key; });
+    if (it != graphs_.end()) {
+      std::rotate(graphs_.begin(), it, it + 1);  // most recently used first
+    } else {
       hipGraph_t graph = nullptr;
+      hipGraphExec_t exec = nullptr;
       if (split) {
         hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "begin capture");
         try {
@@ -870,13 +911,16 @@ void Runtime::run_pipeline(bool want_grad, BenchMap* bench, int objective) {
         add_event(tev_[1]);
         add_child(rng.second, steps.size());
       }
-      hip_check(hipGraphInstantiate(&G.exec, graph, nullptr, nullptr, 0), "graph instantiate");
-      hip_check(hipGraphDestroy(graph), "graph destroy");
-      G.version = layout_version_;
-      G.timed_stage = timed_stage_;
-      G.split = S;
+      const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+      hipGraphDestroy(graph);
+      hip_check(ie, "graph instantiate");
+      while (graphs_.size() >= kMaxGraphs) {
+        hipGraphExecDestroy(graphs_.back().exec);
+        graphs_.pop_back();
+      }
+      graphs_.insert(graphs_.begin(), GraphEntry{key, exec});
     }
-    hip_check(hipGraphLaunch(G.exec, stream_), "graph launch");
+    hip_check(hipGraphLaunch(graphs_.front().exec, stream_), "graph launch");
   } else if (split) {
     issue_split(part, S);
   } else {
@@ -886,8 +930,9 @@ void Runtime::run_pipeline(bool want_grad, BenchMap* bench, int objective) {
     if (timed) hip_check(hipEventRecord(tev_[1], stream_), "timing event");
     run_steps(steps, rng.second, steps.size());
   }
-  hip_check(hipMemcpyAsync(h_out_, d_out_, sizeof(SlotOut) * nslots_, hipMemcpyDeviceToHost, stream_),
-            "download results");
+  if (noalloc_)
+    hip_check(hipMemcpyAsync(h_out_, d_out_, sizeof(SlotOut) * nslots_, hipMemcpyDeviceToHost, stream_),
+              "download results");
   hip_check(hipStreamSynchronize(stream_), "stream sync");
   if (timed && bench == nullptr) {
     float ms = 0.f;

@@ -5,6 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <functional>
 #include <map>
@@ -192,7 +193,7 @@ class Runtime {
   // look-ahead Cholesky for one-slot batches of at least kLookaheadMinBlocks
   // blocks (on by default; LKGPU_LOOKAHEAD=0 or this call turns it off):
   // results are the same either way
-  void set_lookahead(bool on) { lookahead_ = on; ++layout_version_; }
+  void set_lookahead(bool on) { lookahead_ = on; }
   bool lookahead_active() const { return lookahead_ && nslots_ == 1 && nblk_max_ >= kLookaheadMinBlocks; }
   // parts of the last run (slot ranges in bucket order) and their bucket
   int last_parts() const { return last_parts_; }
@@ -264,6 +265,7 @@ class Runtime {
   SlotOut np_out_[NOALLOC_MAX_ITEMS] = {};
   std::vector<size_t> slot_bytes_;
   std::vector<Slot> h_slots_;
+  Slot* h_slots_pin_ = nullptr;     // pinned staging of the slot table
   Slot* d_slots_ = nullptr;
   SlotParams* h_params_ = nullptr;  // pinned
   SlotParams* d_params_ = nullptr;
@@ -273,16 +275,24 @@ class Runtime {
   double* pool_ = nullptr;
   size_t pool_bytes_ = 0;
   int nslots_ = 0, nblk_max_ = 0, dmax_ = 0;
-  uint64_t layout_version_ = 0;
 
-  // graph cache: (layout_version, objective, want_grad) -> exec
+  // captured pipelines, most recently used first (at most kMaxGraphs)
+  struct GraphKey {
+    const void* tables[5] = {};  // slot, parameter and result tables, device and pinned
+    std::vector<int> parts;      // the parts' slot ranges, extents and launch parameters
+    int objective = 0, want_grad = 0, timed_stage = -1;
+    bool operator==(const GraphKey& o) const {
+      return std::equal(tables, tables + 5, o.tables) && parts == o.parts && objective == o.objective &&
+             want_grad == o.want_grad && timed_stage == o.timed_stage;
+    }
+  };
   struct GraphEntry {
-    uint64_t version = ~0ull;
-    int timed_stage = -1;
-    int split = 1;
+    GraphKey key;
     hipGraphExec_t exec = nullptr;
   };
-  GraphEntry graphs_[2 * OBJ_COUNT];
+  static constexpr size_t kMaxGraphs = 16;
+  std::vector<GraphEntry> graphs_;
+  void drop_graphs();
   int last_objective_ = OBJ_LL;
   int timed_stage_ = -1;
   // the batch split into S equal parts on S streams: the latency-bound
