@@ -281,8 +281,8 @@ struct NkArgs {
   const int* tile_group;   // Npad / 64: group of each 64-row tile
   const int2* pairs;       // npairs (i < j) group pairs
   const double* Xc;        // qc x d points of this chunk, ld = qc
-  double* C;               // Npad x qpad: k(x_a, x_t), then R_g^-1 k_g
-  double* U;               // Npad x qpad: L_g^-1 k_g
+  double* C;               // Npad rows of qpad points: k(x_a, x_t), then R_g^-1 k_g
+  double* U;               // Npad rows of qpad points: L_g^-1 k_g; then nslice * npairs rows: the pairs' sums
   double* M;               // qc x p: submodel means
   double* Kd;              // qc x p: k_g' R_g^-1 k_g
   double* KM;              // qc x p x p: cov(M_i, M_j) / sigma2 (column-major per point)
@@ -293,11 +293,17 @@ struct NkArgs {
   double itheta[DMAX];     // 1 / theta (1 beyond d): wave-uniform kernel arguments
   double beta0, sigma2, jitter;
   int Npad, d, p, qc, qpad, kernel, npairs;
+  int nslice;              // nk_pair_slices
 };
 hipError_t launch_nk_prepare(const NkArgs& a, hipStream_t stream);  // C, U, M, Kd, R_g^-1 k_g
-// points per workgroup of the pair kernel: the chunk's points are padded to
-// a multiple of it (qpad)
-constexpr int NK_QT = 128;
+constexpr int NK_QT = 512;         // points per workgroup of the pair kernel at its widest
+// up to here its form for few points: a whole prediction at 30 points takes
+// 0.80 .. 1.0 times the wide form's time (n = 900 .. 20000), at 60 points 1.03
+// .. 1.15 times
+constexpr int NK_FEW = 32;
+constexpr int NK_WGS = 2048;       // workgroups to aim at, many points
+constexpr int NK_WGS_FEW = 3072;   // and few
+int nk_pair_slices(int npairs, int qc, int max_tiles);
 hipError_t launch_nk_pairs(const NkArgs& a, hipStream_t stream);    // off-diagonal KM
 hipError_t launch_nk_solve(const NkArgs& a, hipStream_t stream);    // per-point aggregation
 hipError_t launch_nk_alpha(const NkArgs& a, const double* r, hipStream_t stream);  // alpha = Linv' r

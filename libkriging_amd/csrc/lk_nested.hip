@@ -13,13 +13,14 @@
 // where R_g = k(X_g, X_g) + jitter I (NestedKriging.cpp:337-346).
 //
 // The dominant term is sum_{i<j} n_i n_j per point (N^2 q / 2 multiply-adds
-// for q points): k_pair forms R_ij on the fly from X in LDS (never stored)
-// and contracts it on the FP64 MFMA tiles against W_j = R_j^-1 k_j, then
-// against W_i in the epilogue.  One workgroup owns one group pair and 64
-// points and loops over all the pair's row tiles, so the per-pair sums are
-// reduced in registers in a fixed order (deterministic, no atomics).
+// for q points): k_nk_pair forms R_ij on the fly from X (never stored) and
+// contracts it on the FP64 MFMA against W_j = R_j^-1 k_j, then against W_i.
+// A workgroup owns one group pair, a slice of its row tiles and a range of
+// points; its sums stay in registers and the slices are added in order
+// (deterministic, no atomics).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include <math.h>
@@ -29,6 +30,8 @@
 
 namespace lk {
 
+// The chunk's arrays C, U, W keep the points contiguous (row a of a group at
+// a * qpad): every later reader takes 16 consecutive points per row.
 // ---------------------------------------------------------------------------
 // (1) C(a, t) = k(x_a - x_t; theta) for the group-ordered design rows a and
 // the chunk's points t; zero on pad rows / pad points.  grid (qpad/64, Npad/64)
@@ -37,46 +40,46 @@ template <int DT>
 __global__ __launch_bounds__(TPB) void k_nk_cross(NkArgs a) {
   const int t0 = blockIdx.x * NB, i0 = blockIdx.y * NB, tid = threadIdx.x;
   const NkGroup G = a.groups[a.tile_group[blockIdx.y]];
-  const int d = a.d, qc = a.qc, ld = a.Npad;
+  const int d = a.d, qc = a.qc;
   const int nvalid = G.off + G.n;  // rows >= nvalid are the group's padding
   __shared__ double sXo[DT * NB];
   __shared__ double sXn[DT * NB];
   for (int q = tid; q < d * NB; q += TPB) {
     const int k = q / NB, r = q % NB;
-    sXo[q] = a.Xg[(size_t)k * ld + i0 + r];
+    sXo[q] = a.Xg[(size_t)k * a.Npad + i0 + r];
     sXn[q] = (t0 + r < qc) ? a.Xc[(size_t)k * qc + t0 + r] : 0.0;
   }
   double it[DT];
 #pragma unroll
   for (int k = 0; k < DT; ++k) it[k] = (k < d) ? 1.0 / a.theta[k] : 1.0;
   __syncthreads();
-  const int ii = tid & 63, gi = i0 + ii;
+  const int jj = tid & 63, gt = t0 + jj;
   double dx[DT];
   for (int r = 0; r < NB / 4; ++r) {
-    const int jj = (tid >> 6) + 4 * r, gt = t0 + jj;
+    const int ii = (tid >> 6) + 4 * r, gi = i0 + ii;
     double v = 0.0;
     if (gi < nvalid && gt < qc) {
 #pragma unroll
       for (int k = 0; k < DT; ++k) dx[k] = (k < d) ? sXo[k * NB + ii] - sXn[k * NB + jj] : 0.0;
       v = kern_rho<DT>(a.kernel, dx, it);
     }
-    a.C[(size_t)gt * ld + gi] = v;
+    a.C[(size_t)gi * a.qpad + gt] = v;
   }
 }
 
-// (2) U_g = L_g^-1 C_g: tile (row tile of group g, 64 points), K over the
+// (2) U_g = L_g^-1 C_g: tile (64 points, row tile of group g), K over the
 // group's blocks up to the diagonal.  grid (qpad/64, Npad/64)
 __global__ __launch_bounds__(TPB) void k_nk_trmm(NkArgs a) {
   const int t0 = blockIdx.x * NB, i0 = blockIdx.y * NB;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wr = w >> 1, wc = w & 1;
   const NkGroup G = a.groups[a.tile_group[blockIdx.y]];
-  const int il = i0 - G.off, ld = a.Npad;
+  const int il = i0 - G.off, ld = a.qpad;
   __shared__ double sbuf[4 * KC * LDSS];
   d4 acc[2][2];
   acc_zero(acc);
-  tile_mainloop<false, true, false>(a.Linv + G.loff, G.npad, il, a.C + G.off, ld, t0, 0, il + NB, sbuf, acc, tid,
-                                    lane, wr, wc);
-  acc_store(acc, a.U + (size_t)t0 * ld + i0, ld, lane, wr, wc);
+  tile_mainloop<false, false, false>(a.C + (size_t)G.off * ld, ld, t0, a.Linv + G.loff, G.npad, il, 0, il + NB, sbuf,
+                                     acc, tid, lane, wr, wc);
+  acc_store(acc, a.U + (size_t)i0 * ld + t0, ld, lane, wr, wc);
 }
 
 // (3) W_g = L_g^-T U_g = R_g^-1 k_g, written over C (after k_nk_stats has
@@ -85,35 +88,52 @@ __global__ __launch_bounds__(TPB) void k_nk_trmm_t(NkArgs a) {
   const int t0 = blockIdx.x * NB, i0 = blockIdx.y * NB;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wr = w >> 1, wc = w & 1;
   const NkGroup G = a.groups[a.tile_group[blockIdx.y]];
-  const int il = i0 - G.off, ld = a.Npad;
+  const int il = i0 - G.off, ld = a.qpad;
   __shared__ double sbuf[4 * KC * LDSS];
   d4 acc[2][2];
   acc_zero(acc);
-  tile_mainloop<true, true, false>(a.Linv + G.loff, G.npad, il, a.U + G.off, ld, t0, il, G.npad, sbuf, acc, tid,
-                                   lane, wr, wc);
-  acc_store(acc, a.C + (size_t)t0 * ld + i0, ld, lane, wr, wc);
+  tile_mainloop<false, true, false>(a.U + (size_t)G.off * ld, ld, t0, a.Linv + G.loff, G.npad, il, il, G.npad, sbuf,
+                                    acc, tid, lane, wr, wc);
+  acc_store(acc, a.C + (size_t)i0 * ld + t0, ld, lane, wr, wc);
 }
 
-// (4) per (point, group): M = beta0 + C_g' alpha_g, Kd = |U_g|^2.
-// One wave per point; grid (ceil(qc / 4), p)
-__global__ __launch_bounds__(TPB) void k_nk_stats(NkArgs a) {
+// (4) per (point, group): M = beta0 + C_g' alpha_g, Kd = |U_g|^2.  Lane =
+// point, the rows over the 16 waves (batches of 4), their sums added in wave
+// order.  grid (qpad / 64, p)
+constexpr int NK_ST_W = 16;
+__global__ __launch_bounds__(64 * NK_ST_W) void k_nk_stats(NkArgs a) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int t = blockIdx.x * 4 + w, g = blockIdx.y;
-  if (t >= a.qc) return;
+  const int t = blockIdx.x * NB + lane, g = blockIdx.y;
   const NkGroup G = a.groups[g];
-  const double* c = a.C + (size_t)t * a.Npad + G.off;
-  const double* u = a.U + (size_t)t * a.Npad + G.off;
+  const double* c = a.C + (size_t)G.off * a.qpad + t;
+  const double* u = a.U + (size_t)G.off * a.qpad + t;
   const double* al = a.alpha + G.off;
+  __shared__ double red[2][NK_ST_W][NB];
   double m = 0.0, s = 0.0;
-  for (int i = lane; i < G.n; i += 64) {
-    m = fma(c[i], al[i], m);
-    s = fma(u[i], u[i], s);
+  for (int i = 4 * w; i < G.n; i += 4 * NK_ST_W) {
+    double cv[4], uv[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {  // rows beyond n are the group's padding: zero, as alpha is there
+      cv[q] = gload(c + (size_t)(i + q) * a.qpad);
+      uv[q] = gload(u + (size_t)(i + q) * a.qpad);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      m = fma(cv[q], al[i + q], m);
+      s = fma(uv[q], uv[q], s);
+    }
   }
-  m = wave_sum(m);
-  s = wave_sum(s);
-  if (lane == 0) {
-    a.M[(size_t)t * a.p + g] = a.beta0 + m;
-    a.Kd[(size_t)t * a.p + g] = s;
+  red[0][w][lane] = m;
+  red[1][w][lane] = s;
+  __syncthreads();
+  if (w < 2 && t < a.qc) {
+    double v = red[w][0][lane];
+#pragma unroll
+    for (int q = 1; q < NK_ST_W; ++q) v += red[w][q][lane];
+    if (w == 0)
+      a.M[(size_t)t * a.p + g] = a.beta0 + v;
+    else
+      a.Kd[(size_t)t * a.p + g] = v;
   }
 }
 
@@ -136,148 +156,359 @@ __global__ __launch_bounds__(TPB) void k_nk_alpha(NkArgs a, const double* __rest
 }
 
 // ---------------------------------------------------------------------------
-// (6) KM_ij(t) = sum_a W_i(a, t) sum_b R(x_a, x_b) W_j(b, t) for i < j.
-// grid (npairs, qpad / NK_QT), 256 threads; wave w owns the NK_QW points
-// t0 + NK_QW w .. of the workgroup's NK_QT.  Per 64-row tile of group i and
-// chunk of NK_PKC rows of group j:
-//   R(a, b) generated once into LDS (4 kernel values per thread), then
-//   reused by all NK_QT points on the MFMA
-//   acc(a, t) += sum_b R(a, b) W_j(b, t)   (64 x NK_QW per wave)
-// and per row tile  part(t) += sum_a W_i(a, t) acc(a, t)  in registers.
-// Every sum over rows stays inside one wave (fixed order, no atomics).
-// Three waves per SIMD (168 registers, a few spilled outside the MFMA loop):
-// one workgroup's kernel-value generation runs beside the others' MFMAs
-// (0.37 -> 0.41 of the FP64 peak against two waves per SIMD).
+// (6) part(t) = sum_a W_i(a, t) sum_b R(x_a, x_b) W_j(b, t) for i < j over a
+// slice of group i's 64-row tiles, written over U (done with by then) at
+// row slice * npairs + pair; k_nk_solve adds the slices in order.  R is
+// generated from X and never stored; acc(a, t) += R(a, b) W_j(b, t) on the
+// MFMA, 64 rows a by 16 NBJ points per wave, then part(t) += W_i(a, t)
+// acc(a, t).  W_j is read straight into the MFMA's operand registers: a wave
+// owns its points, so nothing of it is shared, and 16 points of a row are
+// one 128-byte line.
 // ---------------------------------------------------------------------------
-constexpr int NK_PKC = 16;      // rows of group j per chunk
-constexpr int NK_QW = NK_QT / 4;  // points per wave
-constexpr int NK_QB = NK_QW / 16;  // 16-point MFMA blocks per wave
-constexpr int NK_SB = NK_QT + 1;  // W_j chunk row stride (odd: transposed stores conflict-free)
+constexpr int NK_DR = 8;    // dimensions kept in registers; beyond, X_i's tile is in LDS
+constexpr int NK_PKC = 16;  // rows of group j per chunk
 
-template <int DT, int KT>
-__global__ __launch_bounds__(TPB, 3) void k_nk_pair(NkArgs a) {
-  const int2 pr = a.pairs[blockIdx.x];
-  const int t0 = blockIdx.y * NK_QT;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int r16 = lane & 15, kq = lane >> 4;
-  const NkGroup Gi = a.groups[pr.x], Gj = a.groups[pr.y];
-  const int d = a.d, ld = a.Npad;
-  constexpr int WV2 = NK_PKC * NK_QT / (2 * TPB);  // W_j 16-byte pairs per thread per chunk
-  constexpr int XR = (DT * NK_PKC + TPB - 1) / TPB;  // X_j values per thread per chunk
-  __shared__ double sA[NK_PKC * LDSS];   // R chunk: sA[kk * LDSS + ii] = R(a_ii, b_kk)
-  __shared__ double sB[NK_PKC * NK_SB];  // W_j chunk: sB[kk * NK_SB + jj] = W_j(b_kk, t0 + jj)
-  __shared__ double sXa[DT * NB];        // rows of the current a tile
-  __shared__ double sXb[DT * NK_PKC];    // rows of the current b chunk
-  const double* it = a.itheta;  // kernel arguments: scalar registers
-  double part[NK_QB][4];
+// V covariances at once, of V points (coordinates xa(k, v)) with one (xb(k));
+// c[k] is the kernel's scale over theta_k (uniform)
+template <int DT, int KT, int V, class XA, class XB>
+__device__ inline void nk_values(int d, const double* c, XA xa, XB xb, double (&out)[V]) {
+  double s[V], pr[V];
 #pragma unroll
-  for (int bj = 0; bj < NK_QB; ++bj)
+  for (int v = 0; v < V; ++v) {
+    s[v] = 0.0;
+    pr[v] = 1.0;
+  }
+  auto dim = [&](int k) __attribute__((always_inline)) {
+    const double xbk = xb(k), ck = c[k];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) part[bj][e] = 0.0;
-
-  const double* Wi = a.C + (size_t)t0 * ld + Gi.off;
-  const double* Wj = a.C + (size_t)t0 * ld + Gj.off;
-  const int ii = tid & 63;
-  // register stage of the next chunk (W_j pairs, X_j coordinates), loaded
-  // while the current chunk is generated and contracted
-  d2 rw[WV2];
-  double rx[XR];
-  auto load_chunk = [&](int b0) {
-#pragma unroll
-    for (int r = 0; r < WV2; ++r) {
-      const int q = tid + r * TPB;
-      const int bp = q % (NK_PKC / 2), t = q / (NK_PKC / 2);
-      rw[r] = gload(reinterpret_cast<const d2*>(Wj + (size_t)t * ld + b0 + 2 * bp));
-    }
-#pragma unroll
-    for (int r = 0; r < XR; ++r) {
-      const int q = tid + r * TPB;
-      rx[r] = (q < d * NK_PKC) ? a.Xg[(size_t)(q / NK_PKC) * ld + Gj.off + b0 + (q % NK_PKC)] : 0.0;
+    for (int v = 0; v < V; ++v) {
+      const double u = (xa(k, v) - xbk) * ck;
+      if constexpr (KT == K_GAUSS) {
+        s[v] = fma(u, u, s[v]);
+      } else {
+        s[v] += fabs(u);
+        if constexpr (KT == K_MATERN32) pr[v] = fma(pr[v], fabs(u), pr[v]);
+        if constexpr (KT == K_MATERN52) pr[v] = fma(pr[v], fabs(u) * fma(fabs(u), 1.0 / 3.0, 1.0), pr[v]);
+      }
     }
   };
-  for (int a0 = 0; a0 < Gi.npad; a0 += NB) {
-    for (int q = tid; q < d * NB; q += TPB) {
-      const int k = q / NB, r = q % NB;
-      sXa[q] = a.Xg[(size_t)k * ld + Gi.off + a0 + r];
+  if constexpr (DT <= NK_DR) {
+#pragma unroll
+    for (int k = 0; k < DT; ++k) {
+      if (k > 0 && k >= d) break;
+      dim(k);
     }
-    d4 acc[4][NK_QB];
+  } else {
+#pragma unroll 4
+    for (int k = 0; k < d; ++k) dim(k);
+  }
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    const double e = exp(KT == K_GAUSS ? -0.5 * s[v] : -s[v]);
+    out[v] = (KT == K_MATERN32 || KT == K_MATERN52) ? e * pr[v] : e;
+  }
+}
+
+// a uniform value the compiler takes as new: addresses made from it are not
+// computed ahead of the loop and kept in registers
+__device__ inline int nk_fresh(int v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
+// here the value has arrived (the wait stands at this point and not, for
+// every load behind it too, at each use after the branches join)
+__device__ inline void nk_arrived(double v) { asm volatile("" : : "v"(v)); }
+
+// uniform base and a lane's offset in bytes (one register, not a pointer)
+__device__ inline double nk_load(const double* base, unsigned bytes) {
+  return gload(reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + bytes));
+}
+
+// part of one wave -> its points' sums: add the four lanes (kq) of a point
+__device__ inline double nk_fold(double v) {
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+
+// (6a) many points: 128 NBJ points per 512-thread workgroup, 16 NBJ per wave;
+// a chunk of R (64 x 16) is generated by all eight waves into LDS and used by
+// all points.  Bound by the FP64 pipes, which the products (64 x 16 x 128 NBJ
+// multiply-adds a chunk) share with the generation: at 512 points a value's
+// ~45 vector instructions are 12 % of a chunk's time, at 128 points 36 %.
+// What else the loop does: each operand is loaded a chunk ahead (W_j into the
+// ring as its last use retires it, the chunk's coordinates into one register
+// per lane, read back by v_readlane), two LDS buffers and one barrier per
+// chunk, and the second wave of each SIMD runs half a chunk behind the first,
+// so that one generates while the other multiplies.  64 rows x 64 points per
+// wave: 128 accumulator registers, two waves per SIMD.  n = 20000 in 32
+// groups, d = 5, 500 points: 3.77 ms, 53 TFLOP/s (a 64 x 128 tile of four
+// waves with W_j staged through LDS and three barriers a chunk: 5.89 ms; the
+// waves in step: 3.83 ms).  grid (npairs, slices, tiles), points tbase + 128
+// NBJ blockIdx.z ..
+template <int DT, int KT, int NBJ>
+__global__ __launch_bounds__(512, 2) void k_nk_pair(NkArgs a, int tbase) {
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, kq = lane >> 4;
+  const int2 pr = a.pairs[blockIdx.x];
+  const NkGroup Gi = a.groups[pr.x], Gj = a.groups[pr.y];
+  const int d = a.d, ld = a.qpad;
+  const int nti = Gi.npad / NB, nch = (Gj.n + NK_PKC - 1) / NK_PKC;
+  const int tile0 = nti * (int)blockIdx.y / a.nslice, tile1 = nti * ((int)blockIdx.y + 1) / a.nslice;
+  __shared__ double sA[2][NK_PKC * LDSS];
+  __shared__ double sX[DT > NK_DR ? DT * NB : 1];
+  // a wave whose points lie beyond the chunk only helps to generate; block
+  // starts beyond it are read at its last 16 points and dropped at the store
+  const int tw = tbase + 128 * NBJ * (int)blockIdx.z + 16 * NBJ * w;
+  const bool on = tw < a.qc;
+  unsigned lo[NBJ];  // row kq, this lane's point
+#pragma unroll
+  for (int bj = 0; bj < NBJ; ++bj) lo[bj] = 8u * (kq * ld + min(tw + 16 * bj, ld - 16) + r16);
+  double part[NBJ];
+  d4 acc[4][NBJ];
+#pragma unroll
+  for (int bj = 0; bj < NBJ; ++bj) {
+    part[bj] = 0.0;
+#pragma unroll
+    for (int bi = 0; bi < 4; ++bi) acc[bi][bj] = d4{0.0, 0.0, 0.0, 0.0};
+  }
+  const double* Wj = a.C + (size_t)Gj.off * ld;
+  double ring[NK_PKC / 4][NBJ];  // the chunk's W_j operands, refilled as they are used
+  auto load_ring = [&](int s, int b0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int bj = 0; bj < NBJ; ++bj) ring[s][bj] = nk_load(Wj + (size_t)(b0 + 4 * s) * ld, lo[bj]);
+  };
+  double xa[DT > NK_DR ? 1 : DT];
+  auto load_tile = [&](int tile) __attribute__((always_inline)) {
+    const double* X = a.Xg + Gi.off + tile * NB;
+    if constexpr (DT > NK_DR) {
+      __syncthreads();
+      for (int q = tid; q < d * NB; q += 512) sX[q] = X[(size_t)(q / NB) * a.Npad + q % NB];
+      __syncthreads();
+    } else {
+#pragma unroll
+      for (int k = 0; k < DT; ++k) xa[k] = nk_load(X + (size_t)min(k, d - 1) * a.Npad, 8u * lane);
+#pragma unroll
+      for (int k = 0; k < DT; ++k) nk_arrived(xa[k]);
+    }
+  };
+  // rows b0 + w and b0 + w + 8 of the chunk by this wave, lane = row a; lane
+  // 2 k + q holds coordinate k of row q of the pair, loaded a chunk ahead
+  const unsigned xo = 8u * (min(lane >> 1, d - 1) * a.Npad + w + 8 * (lane & 1));
+  double xb;
+  auto load_b = [&](int b0) __attribute__((always_inline)) { xb = nk_load(a.Xg + Gj.off + b0, xo); };
+  auto generate = [&](double* dst) __attribute__((always_inline)) {
+    double v[2];
+    nk_values<DT, KT, 2>(
+        d, a.itheta, [&](int k, int q) { return readlane_d(xb, 2 * k + q); },
+        [&](int k) {
+          if constexpr (DT > NK_DR)
+            return sX[k * NB + lane];
+          else
+            return xa[k];
+        },
+        v);
+    dst[w * LDSS + lane] = v[0];
+    dst[(w + 8) * LDSS + lane] = v[1];
+  };
+  // waves 4 .. 7 run half a chunk behind
+  const bool late = DT <= NK_DR && w >= 4;
+  // two instances of the loop, so that a wave without points carries no
+  // branch around the others' loads
+  auto run = [&](auto on_tag) __attribute__((always_inline)) {
+    constexpr bool ON = decltype(on_tag)::value;
+    load_tile(tile0);
+    load_b(0);
+    int gtile = tile0, gc = 0, gbuf = 0;  // what generate_next makes
+    auto generate_next = [&]() __attribute__((always_inline)) {
+      generate(sA[gbuf]);
+      gbuf ^= 1;
+      if (++gc == nch) {
+        gc = 0;
+        ++gtile;
+        if (gtile < tile1) load_tile(gtile);
+      }
+      load_b(gc * NK_PKC);
+    };
+    if (!late) {
+      generate_next();
+      __syncthreads();
+    }
+    // (in the loop's order: a wait there then leaves the later ones in flight)
+    if constexpr (ON) {
+#pragma unroll
+      for (int s = 0; s < NK_PKC / 4; ++s) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_ring(s, 0);
+      }
+    }
+    int buf = 0;
+    for (int tile = tile0; tile < tile1; ++tile)
+      for (int c = 0; c < nch; ++c, buf ^= 1) {
+        const bool last = c + 1 == nch;
+        const int bn = last ? 0 : (c + 1) * NK_PKC;
+        if (gtile < tile1) generate_next();
+        if (late) __syncthreads();
+        if constexpr (ON) {
+          double an[4];
+          const double* pa = sA[buf] + kq * LDSS + r16;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) an[q] = pa[16 * q];
+#pragma unroll
+          for (int s = 0; s < NK_PKC / 4; ++s) {
+            double av[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              av[q] = an[q];
+              if (s + 1 < NK_PKC / 4) an[q] = pa[4 * (s + 1) * LDSS + 16 * q];
+            }
+            __builtin_amdgcn_sched_barrier(0);  // the next step's operands are on their way
+#pragma unroll
+            for (int bj = 0; bj < NBJ; ++bj)
+#pragma unroll
+              for (int bi = 0; bi < 4; ++bi)
+                acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[bi], ring[s][bj], acc[bi][bj], 0, 0, 0);
+            load_ring(s, bn);
+          }
+          if (last) {
+            // lane (r16, kq), register e of block (bi, bj): row 16 bi + kq +
+            // 4 e, point r16 of the block
+            const double* Wi = a.C + ((size_t)Gi.off + nk_fresh(tile) * NB) * ld;
+#pragma unroll
+            for (int bj = 0; bj < NBJ; ++bj) {
+              double wv[16];
+#pragma unroll
+              for (int q = 0; q < 16; ++q) wv[q] = nk_load(Wi + (size_t)(4 * q) * ld, lo[bj]);
+#pragma unroll
+              for (int bi = 0; bi < 4; ++bi) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) part[bj] = fma(acc[bi][bj][e], wv[4 * bi + e], part[bj]);
+                acc[bi][bj] = d4{0.0, 0.0, 0.0, 0.0};
+              }
+              __builtin_amdgcn_sched_barrier(0);  // sixteen loads at a time: registers
+            }
+          }
+        }
+        if (!late) __syncthreads();
+      }
+    if (late) __syncthreads();
+  };
+  if (tile0 < tile1) {
+    if (on)
+      run(std::true_type{});
+    else
+      run(std::false_type{});
+  }
+  double* P = a.U + ((size_t)blockIdx.y * a.npairs + blockIdx.x) * ld;
+#pragma unroll
+  for (int bj = 0; bj < NBJ; ++bj) {
+    const double v = nk_fold(part[bj]);
+    const int t = tw + 16 * bj + r16;
+    if (kq == 0 && t < a.qc) P[t] = v;
+  }
+}
+
+// (6b) few points (<= 32): a value of R serves so few points that the time is
+// its generation, so each wave generates its own operands in the MFMA's
+// register layout (lane = row r16, column kq), four independent values at a
+// time, with no LDS and no barrier; the four waves take the rows b in
+// turn and their parts are added at the end.  A whole prediction, n = 20000
+// in 32 groups: 0.80 ms at 16 points against 1.03 through (6a) and 2.06 when
+// every call was padded to 128 points.  grid (npairs, slices)
+template <int DT, int KT, int NBJ>
+__global__ __launch_bounds__(TPB, 2) void k_nk_pair_few(NkArgs a, int tbase) {
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, kq = lane >> 4;
+  const int2 pr = a.pairs[blockIdx.x];
+  const NkGroup Gi = a.groups[pr.x], Gj = a.groups[pr.y];
+  const int d = a.d, ld = a.qpad;
+  const int nti = Gi.npad / NB;
+  const int tile0 = nti * (int)blockIdx.y / a.nslice, tile1 = nti * ((int)blockIdx.y + 1) / a.nslice;
+  // K-steps of 4 rows b: wave w's are s0 .. s1 - 1 (rows beyond n: W_j = 0)
+  const int nst = (Gj.n + 3) / 4, s0 = nst * w / 4, s1 = nst * (w + 1) / 4;
+  __shared__ double sX[DT > NK_DR ? DT * NB : 1];
+  __shared__ double red[4][16 * NBJ];
+  double part[NBJ];
+#pragma unroll
+  for (int bj = 0; bj < NBJ; ++bj) part[bj] = 0.0;
+  const unsigned lo = 8u * (kq * ld + r16);  // row kq, point r16
+  const double* Wj = a.C + (size_t)Gj.off * ld + tbase;
+  const double* Xb = a.Xg + Gj.off;
+  for (int tile = tile0; tile < tile1; ++tile) {
+    const double* X = a.Xg + Gi.off + tile * NB;
+    if constexpr (DT > NK_DR) {
+      __syncthreads();
+      for (int q = tid; q < d * NB; q += TPB) sX[q] = X[(size_t)(q / NB) * a.Npad + q % NB];
+      __syncthreads();
+    }
+    double xa[DT > NK_DR ? 1 : DT][4];
+    if constexpr (DT <= NK_DR) {
+#pragma unroll
+      for (int k = 0; k < DT; ++k)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          xa[k][q] = nk_load(X + (size_t)min(k, d - 1) * a.Npad + 16 * q, 8u * r16);
+    }
+    d4 acc[4][NBJ];
 #pragma unroll
     for (int bi = 0; bi < 4; ++bi)
 #pragma unroll
-      for (int bj = 0; bj < NK_QB; ++bj) acc[bi][bj] = d4{0.0, 0.0, 0.0, 0.0};
-    load_chunk(0);
-    for (int b0 = 0; b0 < Gj.npad; b0 += NK_PKC) {
+      for (int bj = 0; bj < NBJ; ++bj) acc[bi][bj] = d4{0.0, 0.0, 0.0, 0.0};
+    double xb[DT > NK_DR ? 1 : DT], bv[NBJ];
+    auto load_step = [&](int s) __attribute__((always_inline)) {
+      if constexpr (DT <= NK_DR) {
 #pragma unroll
-      for (int r = 0; r < WV2; ++r) {
-        const int q = tid + r * TPB;
-        const int bp = q % (NK_PKC / 2), t = q / (NK_PKC / 2);
-        sB[(2 * bp) * NK_SB + t] = rw[r].x;
-        sB[(2 * bp + 1) * NK_SB + t] = rw[r].y;
+        for (int k = 0; k < DT; ++k) xb[k] = nk_load(Xb + (size_t)min(k, d - 1) * a.Npad + 4 * s, 8u * kq);
       }
 #pragma unroll
-      for (int r = 0; r < XR; ++r) {
-        const int q = tid + r * TPB;
-        if (q < d * NK_PKC) sXb[q] = rx[r];
-      }
-      __syncthreads();
-      if (b0 + NK_PKC < Gj.npad) load_chunk(b0 + NK_PKC);
-      double dx[DT];
+      for (int bj = 0; bj < NBJ; ++bj) bv[bj] = nk_load(Wj + (size_t)(4 * s) * ld + 16 * bj, lo);
+    };
+    if (s0 < s1) load_step(s0);
 #pragma unroll 1
-      for (int r = 0; r < (NK_PKC * NB) / TPB; ++r) {
-        const int kk = (tid >> 6) + 4 * r;
+    for (int s = s0; s < s1; ++s) {
+      double av[4], b[NBJ], x[DT > NK_DR ? 1 : DT];
+      if constexpr (DT <= NK_DR) {
 #pragma unroll
-        for (int k = 0; k < DT; ++k) dx[k] = (k < d) ? sXa[k * NB + ii] - sXb[k * NK_PKC + kk] : 0.0;
-        // the padded coordinates (d .. DT - 1) are skipped
-        sA[kk * LDSS + ii] = kern_rho<DT>(KT, dx, it, d);
+        for (int k = 0; k < DT; ++k) x[k] = xb[k];
       }
-      __syncthreads();
 #pragma unroll
-      for (int k0 = 0; k0 < NK_PKC; k0 += 4) {
-        const double* pa = sA + (k0 + kq) * LDSS + r16;
-        const double* pb = sB + (k0 + kq) * NK_SB + NK_QW * w + r16;
-        double av[4], bv[NK_QB];
+      for (int bj = 0; bj < NBJ; ++bj) b[bj] = bv[bj];
+      load_step(min(s + 1, s1 - 1));
+      __builtin_amdgcn_sched_barrier(0);  // the next step's loads fly during this one
+      if constexpr (DT > NK_DR)
+        nk_values<DT, KT, 4>(
+            d, a.itheta, [&](int k, int q) { return sX[k * NB + 16 * q + r16]; },
+            [&](int k) { return nk_load(Xb + (size_t)k * a.Npad + 4 * s, 8u * kq); }, av);
+      else
+        nk_values<DT, KT, 4>(
+            d, a.itheta, [&](int k, int q) { return xa[k][q]; }, [&](int k) { return x[k]; }, av);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) av[q] = pa[16 * q];
+      for (int bi = 0; bi < 4; ++bi)
 #pragma unroll
-        for (int q = 0; q < NK_QB; ++q) bv[q] = pb[16 * q];
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-          for (int bj = 0; bj < NK_QB; ++bj)
-            acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[bj], av[bi], acc[bi][bj], 0, 0, 0);
-      }
-      __syncthreads();
+        for (int bj = 0; bj < NBJ; ++bj)
+          acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[bi], b[bj], acc[bi][bj], 0, 0, 0);
     }
-    // weight by W_i(a, t) and sum this tile's rows into part: lane (r16, kq),
-    // register e of block (bi, bj) holds row 16 bi + r16, point
-    // NK_QW w + 16 bj + kq + 4 e
+    const double* Wi = a.C + ((size_t)Gi.off + nk_fresh(tile) * NB) * ld + tbase;
 #pragma unroll
-    for (int bj = 0; bj < NK_QB; ++bj)
+    for (int bj = 0; bj < NBJ; ++bj) {
+      double wv[16];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const double* wcol = Wi + (size_t)(NK_QW * w + 16 * bj + kq + 4 * e) * ld + a0 + r16;
-        double s = part[bj][e];
+      for (int q = 0; q < 16; ++q) wv[q] = nk_load(Wi + (size_t)(4 * q) * ld + 16 * bj, lo);
 #pragma unroll
-        for (int bi = 0; bi < 4; ++bi) s = fma(acc[bi][bj][e], gload(wcol + 16 * bi), s);
-        part[bj][e] = s;
-      }
+      for (int bi = 0; bi < 4; ++bi)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part[bj] = fma(acc[bi][bj][e], wv[4 * bi + e], part[bj]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
-  // reduce over the 16 lanes holding different rows of the same points
-  const size_t pp = (size_t)a.p * a.p;
 #pragma unroll
-  for (int bj = 0; bj < NK_QB; ++bj)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      double v = part[bj][e];
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off, 64);
-      const int t = t0 + NK_QW * w + 16 * bj + kq + 4 * e;
-      if (r16 == 0 && t < a.qc) {
-        double* K = a.KM + (size_t)t * pp;
-        K[(size_t)pr.y * a.p + pr.x] = v;
-        K[(size_t)pr.x * a.p + pr.y] = v;
-      }
-    }
+  for (int bj = 0; bj < NBJ; ++bj) {
+    const double v = nk_fold(part[bj]);
+    if (kq == 0) red[w][16 * bj + r16] = v;
+  }
+  __syncthreads();
+  const int t = tbase + tid;
+  if (tid < 16 * NBJ && t < a.qc)
+    a.U[((size_t)blockIdx.y * a.npairs + blockIdx.x) * ld + t] = (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
 }
 
 // ---------------------------------------------------------------------------
@@ -304,6 +535,13 @@ __global__ __launch_bounds__(TPB) void k_nk_solve(NkArgs a) {
     const double v = a.Kd[(size_t)t * p + i] + a.jitter;
     K[(size_t)i * p + i] = v;
     kM[i] = v;
+  }
+  for (int q = tid; q < a.npairs; q += TPB) {
+    const int2 pr = a.pairs[q];
+    double v = a.U[(size_t)q * a.qpad + t];
+    for (int z = 1; z < a.nslice; ++z) v += a.U[((size_t)z * a.npairs + q) * a.qpad + t];
+    K[(size_t)pr.y * p + pr.x] = v;
+    K[(size_t)pr.x * p + pr.y] = v;
   }
   __syncthreads();
   for (size_t q = tid; q < pp; q += TPB) F[q] = K[q];
@@ -474,36 +712,73 @@ hipError_t launch_nk_prepare(const NkArgs& a, hipStream_t stream) {
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_nk_trmm, grid, dim3(TPB), 0, stream, a);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_nk_stats, dim3((a.qc + 3) / 4, a.p), dim3(TPB), 0, stream, a);
+  hipLaunchKernelGGL(k_nk_stats, dim3(a.qpad / NB, a.p), dim3(64 * NK_ST_W), 0, stream, a);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL(k_nk_trmm_t, grid, dim3(TPB), 0, stream, a);
   return hipGetLastError();
 }
 
-hipError_t launch_nk_pairs(const NkArgs& a, hipStream_t stream) {
-  if (a.npairs <= 0) return hipSuccess;
-  if (a.qpad % NK_QT != 0) return hipErrorInvalidValue;
-  const dim3 grid(a.npairs, a.qpad / NK_QT);
-  // one instance per (dimension bound, covariance kernel): the kernel-value
-  // generation runs one kernel's code, not a branch per value
-  auto go = [&](auto dtag) {
+// Slices of group i's row tiles, so that few pairs still cover the chip and
+// the last workgroups are a small part of the time.  Aims, measured at 496
+// pairs and 500 points: 2048 workgroups of 512 threads, one per CU at a time
+// (pair kernel 3.77 ms; 3.82 for 1024, 4.02 for 4096, where the start of
+// each shows); 3072 of the short 256-thread ones
+int nk_pair_slices(int npairs, int qc, int max_tiles) {
+  if (npairs <= 0) return 1;
+  const int have = qc <= NK_FEW ? npairs : npairs * ((qc + NK_QT - 1) / NK_QT);
+  const int want = qc <= NK_FEW ? NK_WGS_FEW : NK_WGS;
+  return std::max(1, std::min(max_tiles, (want + have - 1) / have));
+}
+
+hipError_t launch_nk_pairs(const NkArgs& args, hipStream_t stream) {
+  if (args.npairs <= 0) return hipSuccess;
+  if (args.qpad % NB != 0 || args.qc > args.qpad || args.nslice < 1) return hipErrorInvalidValue;
+  NkArgs a = args;
+  // the kernels' scale of |x - x'| / theta
+  const double scale = a.kernel == K_MATERN32 ? SQRT3 : a.kernel == K_MATERN52 ? SQRT5 : 1.0;
+  for (int k = 0; k < DMAX; ++k) a.itheta[k] *= scale;
+  // one instance per (dimension bound, covariance kernel, points per wave):
+  // the generation runs one kernel's code, not a branch per value
+  auto run = [&](auto dtag, auto ktag, int tbase, int tiles, int nbj) {
     constexpr int DT = decltype(dtag)::value;
+    constexpr int KT = decltype(ktag)::value;
+    const dim3 grid(a.npairs, a.nslice, tiles);
+    switch (nbj) {
+      case 1: hipLaunchKernelGGL((k_nk_pair<DT, KT, 1>), grid, dim3(512), 0, stream, a, tbase); break;
+      case 2: hipLaunchKernelGGL((k_nk_pair<DT, KT, 2>), grid, dim3(512), 0, stream, a, tbase); break;
+      case 3: hipLaunchKernelGGL((k_nk_pair<DT, KT, 3>), grid, dim3(512), 0, stream, a, tbase); break;
+      default: hipLaunchKernelGGL((k_nk_pair<DT, KT, 4>), grid, dim3(512), 0, stream, a, tbase); break;
+    }
+    return hipGetLastError();
+  };
+  auto run_few = [&](auto dtag, auto ktag, int tbase, int points) {
+    constexpr int DT = decltype(dtag)::value;
+    constexpr int KT = decltype(ktag)::value;
+    const dim3 grid(a.npairs, a.nslice);
+    if (points <= 16)
+      hipLaunchKernelGGL((k_nk_pair_few<DT, KT, 1>), grid, dim3(TPB), 0, stream, a, tbase);
+    else
+      hipLaunchKernelGGL((k_nk_pair_few<DT, KT, 2>), grid, dim3(TPB), 0, stream, a, tbase);
+    return hipGetLastError();
+  };
+  auto go = [&](auto dtag, auto ktag) {
+    // whole tiles of 512 points, the rest in one launch of its own width
+    const int tiles = a.qc / NK_QT, rest = a.qc % NK_QT;
+    hipError_t e = hipSuccess;
+    if (tiles > 0) e = run(dtag, ktag, 0, tiles, 4);
+    if (e == hipSuccess && rest > NK_FEW) e = run(dtag, ktag, tiles * NK_QT, 1, (rest + 127) / 128);
+    if (e == hipSuccess && rest > 0 && rest <= NK_FEW) e = run_few(dtag, ktag, tiles * NK_QT, rest);
+    return e;
+  };
+  auto kern = [&](auto dtag) {
     switch (a.kernel) {
-      case K_GAUSS: hipLaunchKernelGGL((k_nk_pair<DT, K_GAUSS>), grid, dim3(TPB), 0, stream, a); break;
-      case K_EXP: hipLaunchKernelGGL((k_nk_pair<DT, K_EXP>), grid, dim3(TPB), 0, stream, a); break;
-      case K_MATERN32: hipLaunchKernelGGL((k_nk_pair<DT, K_MATERN32>), grid, dim3(TPB), 0, stream, a); break;
-      default: hipLaunchKernelGGL((k_nk_pair<DT, K_MATERN52>), grid, dim3(TPB), 0, stream, a); break;
+      case K_GAUSS: return go(dtag, std::integral_constant<int, K_GAUSS>{});
+      case K_EXP: return go(dtag, std::integral_constant<int, K_EXP>{});
+      case K_MATERN32: return go(dtag, std::integral_constant<int, K_MATERN32>{});
+      default: return go(dtag, std::integral_constant<int, K_MATERN52>{});
     }
   };
-  if (a.d <= 4)
-    go(std::integral_constant<int, 4>{});
-  else if (a.d <= 8)
-    go(std::integral_constant<int, 8>{});
-  else if (a.d <= 16)
-    go(std::integral_constant<int, 16>{});
-  else
-    go(std::integral_constant<int, 32>{});
-  return hipGetLastError();
+  return a.d <= NK_DR ? kern(std::integral_constant<int, NK_DR>{}) : kern(std::integral_constant<int, DMAX>{});
 }
 
 hipError_t launch_nk_solve(const NkArgs& a, hipStream_t stream) {

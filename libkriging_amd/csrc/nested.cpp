@@ -543,15 +543,20 @@ void NestedKriging::predict_poe(const double* Xn, int m, bool want_stdev, double
 void NestedKriging::predict_nk(const double* Xn, int m, bool want_stdev, double* mean, double* stdev) {
   const int p = (int)groups_.size(), d = d_;
   hip_check(hipSetDevice(device_), "hipSetDevice");
+  // U's rows also hold the pairs' sums, nslice per pair (at most as many as
+  // the smallest chunk is cut into)
+  int max_tiles = 1;
+  for (int np : gpad_) max_tiles = std::max(max_tiles, np / NB);
+  const size_t u_rows = std::max((size_t)Npad_, (size_t)nk_pair_slices(npairs_, 1, max_tiles) * npairs_);
   // chunk: explicit, else as many points as fit in ~8 GiB of workspace
   int qc = chunk_;
   if (qc <= 0) {
-    const double per_point = 8.0 * (2.0 * Npad_ + 2.0 * (double)p * p + 2.0 * p + 4.0 + d);
+    const double per_point = 8.0 * ((double)Npad_ + (double)u_rows + 2.0 * (double)p * p + 2.0 * p + 4.0 + d);
     qc = (int)std::min<double>(8192.0, std::max(64.0, (8.0 * (1ull << 30)) / per_point));
     qc = std::max(64, qc / 64 * 64);
   }
   qc = std::min(qc, m);
-  const int qpad_max = (qc + NK_QT - 1) / NK_QT * NK_QT;
+  const int qpad_max = (qc + NB - 1) / NB * NB;
   double *dXc = nullptr, *dC = nullptr, *dU = nullptr, *dM = nullptr, *dKd = nullptr, *dKM = nullptr, *dKF = nullptr,
          *dout = nullptr;
   int* dinfo = nullptr;
@@ -571,7 +576,7 @@ void NestedKriging::predict_nk(const double* Xn, int m, bool want_stdev, double*
     const size_t pp = (size_t)p * p;
     hip_check(hipMalloc(&dXc, sizeof(double) * (size_t)qc * d), "hipMalloc");
     hip_check(hipMalloc(&dC, sizeof(double) * (size_t)Npad_ * qpad_max), "hipMalloc");
-    hip_check(hipMalloc(&dU, sizeof(double) * (size_t)Npad_ * qpad_max), "hipMalloc");
+    hip_check(hipMalloc(&dU, sizeof(double) * u_rows * qpad_max), "hipMalloc");
     hip_check(hipMalloc(&dM, sizeof(double) * (size_t)qc * p), "hipMalloc");
     hip_check(hipMalloc(&dKd, sizeof(double) * (size_t)qc * p), "hipMalloc");
     hip_check(hipMalloc(&dKM, sizeof(double) * (size_t)qc * pp), "hipMalloc");
@@ -611,7 +616,8 @@ void NestedKriging::predict_nk(const double* Xn, int m, bool want_stdev, double*
       a.d = d;
       a.p = p;
       a.qc = mc;
-      a.qpad = (mc + NK_QT - 1) / NK_QT * NK_QT;
+      a.qpad = (mc + NB - 1) / NB * NB;
+      a.nslice = nk_pair_slices(npairs_, mc, max_tiles);
       a.kernel = kernel_id(kernel_);
       a.npairs = npairs_;
       hip_check(launch_nk_prepare(a, st), "nk prepare");
