@@ -894,8 +894,8 @@ void Kriging::update(const double* y_u, const double* X_u, int m, bool refit) {
   if (m > 0 && d_L_ != nullptr && d_Linv_ != nullptr) {
     hip_check(hipSetDevice(device_), "hipSetDevice");
     const size_t bn = sizeof(double) * (size_t)N * N;
-    hip_check(hipMalloc(&dR, bn), "hipMalloc");
-    hip_check(hipMalloc(&dLn, bn), "hipMalloc");
+    hip_check(rt_->alloc(&dR, bn), "hipMalloc");
+    hip_check(rt_->alloc(&dLn, bn), "hipMalloc");
     const DeviceProblem& P = rt_->problem(problem_);
     CovMatArgs c{};
     c.X1 = P.X;
@@ -953,50 +953,57 @@ void Kriging::predict(const double* Xn, int m, bool want_stdev, double* mean, do
     if (!want_cov) chunk = std::min(chunk, cmax);
   }
   const int mpad_max = (chunk + NB - 1) / NB * NB;
-  double *dXn = nullptr, *dRon = nullptr, *dC = nullptr, *dout = nullptr, *dcoef = nullptr, *dEc = nullptr,
-         *dCov = nullptr, *dDR = nullptr, *dDW = nullptr, *dDm = nullptr, *dDv = nullptr;
-  auto cleanup = [&] {
-    for (double* q : {dXn, dRon, dC, dout, dcoef, dEc, dCov, dDR, dDW, dDm, dDv})
-      if (q) hipFree(q);
-  };
-  try {
-    hip_check(hipMalloc(&dXn, sizeof(double) * (size_t)chunk * d), "hipMalloc");
-    hip_check(hipMalloc(&dRon, sizeof(double) * (size_t)npad_ * mpad_max), "hipMalloc");
-    hip_check(hipMalloc(&dC, sizeof(double) * (size_t)npad_ * mpad_max), "hipMalloc");
-    hip_check(hipMalloc(&dout, sizeof(double) * 2 * (size_t)chunk), "hipMalloc");
-    hip_check(hipMalloc(&dcoef, sizeof(double) * (size_t)(p + p * p + 1)), "hipMalloc");
-    if ((want_cov || want_deriv) && p > 0)
-      hip_check(hipMalloc(&dEc, sizeof(double) * (size_t)chunk * p), "hipMalloc");
-    if (want_cov) hip_check(hipMalloc(&dCov, sizeof(double) * (size_t)m * m), "hipMalloc");
+  // one block of device memory, and pinned staging for what goes up ([coef |
+  // points]) and comes down ([out | derivatives]), one copy each per chunk; a
+  // large covariance goes to the caller's memory directly
+  const size_t ncoef = (size_t)p + (size_t)p * p, nder = want_deriv ? (size_t)chunk * d : 0;
+  const size_t nup = ncoef + (size_t)chunk * d, ndown = 2 * (size_t)chunk + 2 * nder;
+  const size_t ncov = want_cov ? (size_t)m * m : 0;
+  const bool stage_cov = want_cov && cov != nullptr && ncov * sizeof(double) <= (size_t(16) << 20);
+  double *dup = nullptr, *dout = nullptr, *dRon = nullptr, *dC = nullptr, *dEc = nullptr, *dCov = nullptr,
+         *dDR = nullptr, *dDW = nullptr;
+  auto layout = [&](Carve& c) {
+    dup = c.take<double>(nup);
+    dout = c.take<double>(ndown);
+    dRon = c.take<double>((size_t)npad_ * mpad_max);
+    dC = c.take<double>((size_t)npad_ * mpad_max);
+    if ((want_cov || want_deriv) && p > 0) dEc = c.take<double>((size_t)chunk * p);
+    if (want_cov) dCov = c.take<double>(ncov);
     if (want_deriv) {
-      hip_check(hipMalloc(&dDR, sizeof(double) * (size_t)npad_ * mpad_max * d), "hipMalloc");
-      hip_check(hipMalloc(&dDW, sizeof(double) * (size_t)npad_ * mpad_max * d), "hipMalloc");
-      hip_check(hipMalloc(&dDm, sizeof(double) * (size_t)chunk * d), "hipMalloc");
-      hip_check(hipMalloc(&dDv, sizeof(double) * (size_t)chunk * d), "hipMalloc");
+      dDR = c.take<double>((size_t)npad_ * mpad_max * d);
+      dDW = c.take<double>((size_t)npad_ * mpad_max * d);
     }
-    std::vector<double> coef(p + p * p);
-    for (int a = 0; a < p; ++a) coef[a] = beta_[a];
-    for (int q = 0; q < p * p; ++q) coef[p + q] = Rstar_[q];
-    if (p > 0) hip_check(hipMemcpy(dcoef, coef.data(), sizeof(double) * coef.size(), hipMemcpyHostToDevice), "upload");
+  };
+  Carve sizes;
+  layout(sizes);
+  ScratchLease lease(*rt_, sizes.bytes(), sizeof(double) * (nup + ndown + (stage_cov ? ncov : 0)));
+  Carve parts(lease.dev());
+  layout(parts);
+  double* const up = reinterpret_cast<double*>(lease.pin());
+  double* const host_out = up + nup;
+  double* const hcov = host_out + ndown;
+  double* const xn = up + ncoef;
+  for (int a = 0; a < p; ++a) up[a] = beta_[a];
+  for (int q = 0; q < p * p; ++q) up[p + q] = Rstar_[q];
+  {
     const bool nug = noise_ == NoiseModel::Nugget;
     const double var_scale = nug ? sigma2_ / alpha_ : sigma2_;
     const double vs = var_scale * scaleY_ * scaleY_;
-    std::vector<double> xn((size_t)chunk * d), host_out(2 * (size_t)chunk), hdm, hdv;
-    if (want_deriv) {
-      hdm.resize((size_t)chunk * d);
-      hdv.resize((size_t)chunk * d);
-    }
+    const double* const hdm = host_out + 2 * (size_t)chunk;
+    const double* const hdv = hdm + nder;
     for (int s0 = 0; s0 < m; s0 += chunk) {
       const int mc = std::min(chunk, m - s0);
       for (int k = 0; k < d; ++k)
         for (int j = 0; j < mc; ++j) xn[j + (size_t)k * mc] = (Xn[s0 + j + (size_t)k * m] - centerX_[k]) / scaleX_[k];
-      hip_check(hipMemcpy(dXn, xn.data(), sizeof(double) * (size_t)mc * d, hipMemcpyHostToDevice), "upload Xn");
+      hip_check(hipMemcpyAsync(dup, up, sizeof(double) * (ncoef + (size_t)mc * d), hipMemcpyHostToDevice,
+                               rt_->stream()),
+                "upload Xn");
       PredictArgs a{};
       a.X = rt_->problem(problem_).X;
       a.Linv = d_Linv_;
       a.MZ = d_vec_;
-      a.coef = dcoef;
-      a.Xn = dXn;
+      a.coef = dup;
+      a.Xn = dup + ncoef;
       a.Ron = dRon;
       a.C = dC;
       a.out = dout;
@@ -1005,8 +1012,8 @@ void Kriging::predict(const double* Xn, int m, bool want_stdev, double* mean, do
       a.nn_factor = nug ? alpha_ : 1.0;
       a.DR = dDR;
       a.DW = dDW;
-      a.dmean = dDm;
-      a.dvar = dDv;
+      a.dmean = dout + 2 * (size_t)chunk;
+      a.dvar = a.dmean + nder;
       for (int k = 0; k < d; ++k) a.theta[k] = theta_[k];
       a.factor = nug ? alpha_ : 1.0;
       a.n = n_;
@@ -1021,19 +1028,12 @@ void Kriging::predict(const double* Xn, int m, bool want_stdev, double* mean, do
       hip_check(launch_predict(a, rt_->stream()), "predict");
       if (want_cov) hip_check(launch_predict_cov(a, rt_->stream()), "predict cov");
       if (want_deriv) hip_check(launch_predict_deriv(a, rt_->stream()), "predict deriv");
-      hip_check(hipMemcpyAsync(host_out.data(), dout, sizeof(double) * 2 * mc, hipMemcpyDeviceToHost, rt_->stream()),
-                "download");
-      if (want_deriv) {
-        hip_check(hipMemcpyAsync(hdm.data(), dDm, sizeof(double) * (size_t)mc * d, hipMemcpyDeviceToHost,
-                                 rt_->stream()),
-                  "download");
-        if (want_stdev)
-          hip_check(hipMemcpyAsync(hdv.data(), dDv, sizeof(double) * (size_t)mc * d, hipMemcpyDeviceToHost,
-                                   rt_->stream()),
-                    "download");
-      }
+      // the variances' derivatives, last, only when they were asked for
+      const size_t nd = !want_deriv ? 2 * (size_t)mc : ndown - (want_stdev ? 0 : nder);
+      hip_check(hipMemcpyAsync(host_out, dout, sizeof(double) * nd, hipMemcpyDeviceToHost, rt_->stream()), "download");
       if (want_cov && cov != nullptr)
-        hip_check(hipMemcpyAsync(cov, dCov, sizeof(double) * (size_t)m * m, hipMemcpyDeviceToHost, rt_->stream()),
+        hip_check(hipMemcpyAsync(stage_cov ? hcov : cov, dCov, sizeof(double) * ncov, hipMemcpyDeviceToHost,
+                                 rt_->stream()),
                   "download");
       hip_check(hipStreamSynchronize(rt_->stream()), "sync");
       for (int j = 0; j < mc; ++j) {
@@ -1054,13 +1054,12 @@ void Kriging::predict(const double* Xn, int m, bool want_stdev, double* mean, do
           }
       }
     }
-    if (want_cov && cov != nullptr)
-      for (size_t q = 0; q < (size_t)m * m; ++q) cov[q] *= vs;
-  } catch (...) {
-    cleanup();
-    throw;
+    if (want_cov && cov != nullptr) {
+      const double* c = stage_cov ? hcov : cov;
+      for (size_t q = 0; q < ncov; ++q) cov[q] = c[q] * vs;
+    }
   }
-  cleanup();
+  lease.finished();
 }
 
 // Evaluate the model at (theta, alpha), keep L^-1, z, M, R* on the device
@@ -1086,12 +1085,12 @@ void Kriging::commit(const std::vector<double>& theta, double alpha) {
 }
 
 // a model buffer of `bytes`, reallocated only when its size changes
-static void ensure_model_buffer(double*& ptr, size_t& cap, size_t bytes) {
+static void ensure_model_buffer(Runtime& rt, double*& ptr, size_t& cap, size_t bytes) {
   if (ptr != nullptr && cap == bytes) return;
   if (ptr != nullptr) hipFree(ptr);
   ptr = nullptr;
   cap = 0;
-  hip_check(hipMalloc(&ptr, bytes), "hipMalloc model");
+  hip_check(rt.alloc(&ptr, bytes), "hipMalloc model");
   cap = bytes;
 }
 
@@ -1109,9 +1108,9 @@ void Kriging::commit_copy(int slot, const EvalResult& r) {
   const Runtime::SlotView v = rt_->slot_view(slot);
   npad_ = v.npad;
   hip_check(hipSetDevice(device_), "hipSetDevice");
-  ensure_model_buffer(d_L_, cap_L_, sizeof(double) * (size_t)n_ * n_);
-  ensure_model_buffer(d_Linv_, cap_Linv_, sizeof(double) * (size_t)npad_ * npad_);
-  ensure_model_buffer(d_vec_, cap_vec_, sizeof(double) * (size_t)npad_ * (p + 1));
+  ensure_model_buffer(*rt_, d_L_, cap_L_, sizeof(double) * (size_t)n_ * n_);
+  ensure_model_buffer(*rt_, d_Linv_, cap_Linv_, sizeof(double) * (size_t)npad_ * npad_);
+  ensure_model_buffer(*rt_, d_vec_, cap_vec_, sizeof(double) * (size_t)npad_ * (p + 1));
   hip_check(hipMemcpy2DAsync(d_L_, sizeof(double) * n_, v.A, sizeof(double) * npad_, sizeof(double) * n_, n_,
                              hipMemcpyDeviceToDevice, rt_->stream()),
             "copy model");
@@ -1242,9 +1241,9 @@ void Kriging::cov_mat(const double* X1, int n1, const double* X2, int n2, double
     if (dO) hipFree(dO);
   };
   try {
-    hip_check(hipMalloc(&dA, sizeof(double) * a.size()), "hipMalloc");
-    hip_check(hipMalloc(&dB, sizeof(double) * b.size()), "hipMalloc");
-    hip_check(hipMalloc(&dO, sizeof(double) * (size_t)n1 * n2), "hipMalloc");
+    hip_check(rt_->alloc(&dA, sizeof(double) * a.size()), "hipMalloc");
+    hip_check(rt_->alloc(&dB, sizeof(double) * b.size()), "hipMalloc");
+    hip_check(rt_->alloc(&dO, sizeof(double) * (size_t)n1 * n2), "hipMalloc");
     hip_check(hipMemcpy(dA, a.data(), sizeof(double) * a.size(), hipMemcpyHostToDevice), "upload");
     hip_check(hipMemcpy(dB, b.data(), sizeof(double) * b.size(), hipMemcpyHostToDevice), "upload");
     CovMatArgs c{};

@@ -181,7 +181,94 @@ Runtime::~Runtime() {
     if (join_[q]) hipEventDestroy(join_[q]);
     if (xstream_[q]) hipStreamDestroy(xstream_[q]);
   }
+  scratch_trim();
   if (stream_) hipStreamDestroy(stream_);
+}
+
+hipError_t Runtime::alloc(void** ptr, size_t bytes) {
+  hipError_t e = hipMalloc(ptr, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  scratch_trim();
+  return hipMalloc(ptr, bytes);
+}
+
+void Runtime::scratch_free(ScratchBlock& b) {
+  if (b.dev) hipFree(b.dev);
+  if (b.pin) hipHostFree(b.pin);
+  b = ScratchBlock{};
+}
+
+void Runtime::scratch_trim() {
+  std::vector<ScratchBlock> idle;
+  {
+    std::lock_guard<std::mutex> lock(scratch_mutex_);
+    idle.swap(scratch_idle_);
+  }
+  for (auto& b : idle) scratch_free(b);
+}
+
+// the smallest idle block that is large enough, or else the last one used,
+// grown
+Runtime::ScratchBlock Runtime::scratch_take(size_t dev_bytes, size_t pin_bytes) {
+  ScratchBlock b;
+  {
+    std::lock_guard<std::mutex> lock(scratch_mutex_);
+    size_t best = scratch_idle_.size();
+    for (size_t q = 0; q < scratch_idle_.size(); ++q) {
+      const ScratchBlock& c = scratch_idle_[q];
+      if (c.dev_bytes < dev_bytes || c.pin_bytes < pin_bytes) continue;
+      if (best == scratch_idle_.size() || c.dev_bytes < scratch_idle_[best].dev_bytes) best = q;
+    }
+    if (best == scratch_idle_.size() && best > 0) best -= 1;
+    if (best < scratch_idle_.size()) {
+      b = scratch_idle_[best];
+      scratch_idle_.erase(scratch_idle_.begin() + (long)best);
+    }
+  }
+  try {
+    constexpr size_t unit = size_t(2) << 20;
+    if (b.dev_bytes < dev_bytes) {
+      if (b.dev) hip_check(hipFree(b.dev), "hipFree scratch");
+      b.dev = nullptr;
+      b.dev_bytes = 0;
+      const size_t want = (dev_bytes + unit - 1) / unit * unit;
+      hip_check(alloc(&b.dev, want), "hipMalloc");
+      b.dev_bytes = want;
+    }
+    if (b.pin_bytes < pin_bytes) {
+      if (b.pin) hip_check(hipHostFree(b.pin), "hipHostFree scratch");
+      b.pin = nullptr;
+      b.pin_bytes = 0;
+      hip_check(hipHostMalloc((void**)&b.pin, pin_bytes), "hipHostMalloc");
+      b.pin_bytes = pin_bytes;
+    }
+  } catch (...) {
+    scratch_free(b);
+    throw;
+  }
+  return b;
+}
+
+void Runtime::scratch_give(ScratchBlock b) {
+  {
+    std::lock_guard<std::mutex> lock(scratch_mutex_);
+    size_t dev = b.dev_bytes, pin = b.pin_bytes;
+    for (const auto& c : scratch_idle_) {
+      dev += c.dev_bytes;
+      pin += c.pin_bytes;
+    }
+    if (dev <= kScratchKeep && pin <= kScratchKeepPinned && scratch_idle_.size() < kScratchBlocks) {
+      scratch_idle_.push_back(b);
+      return;
+    }
+  }
+  scratch_free(b);
+}
+
+ScratchLease::~ScratchLease() {
+  if (!finished_) hipStreamSynchronize(rt_.stream());
+  rt_.scratch_give(b_);
 }
 
 int Runtime::add_problem(const double* X, int n, int d, const double* y, const double* F, int p, int kernel,
@@ -207,9 +294,9 @@ int Runtime::add_problem(const double* X, int n, int d, const double* y, const d
     P.range[k] = mx - mn;
   }
   P.noise = noise;
-  hip_check(hipMalloc(&P.X, sizeof(double) * (size_t)n * d), "hipMalloc X");
-  hip_check(hipMalloc(&P.y, sizeof(double) * (size_t)n), "hipMalloc y");
-  hip_check(hipMalloc(&P.F, sizeof(double) * (size_t)n * std::max(p, 1)), "hipMalloc F");
+  hip_check(alloc(&P.X, sizeof(double) * (size_t)n * d), "hipMalloc X");
+  hip_check(alloc(&P.y, sizeof(double) * (size_t)n), "hipMalloc y");
+  hip_check(alloc(&P.F, sizeof(double) * (size_t)n * std::max(p, 1)), "hipMalloc F");
   hip_check(hipMemcpy(P.X, X, sizeof(double) * (size_t)n * d, hipMemcpyHostToDevice), "upload X");
   hip_check(hipMemcpy(P.y, y, sizeof(double) * (size_t)n, hipMemcpyHostToDevice), "upload y");
   if (p > 0) hip_check(hipMemcpy(P.F, F, sizeof(double) * (size_t)n * p, hipMemcpyHostToDevice), "upload F");
@@ -228,10 +315,10 @@ int Runtime::add_matrix_problem(const double* M, int n, bool device_memory) {
   P.range.assign(1, 0.0);
   // the likelihood stages that run after the factorisation read X, y: zeros
   std::vector<double> zeros(n, 0.0);
-  hip_check(hipMalloc(&P.X, sizeof(double) * (size_t)n), "hipMalloc X");
-  hip_check(hipMalloc(&P.y, sizeof(double) * (size_t)n), "hipMalloc y");
-  hip_check(hipMalloc(&P.F, sizeof(double)), "hipMalloc F");
-  hip_check(hipMalloc(&P.M, sizeof(double) * (size_t)n * n), "hipMalloc M");
+  hip_check(alloc(&P.X, sizeof(double) * (size_t)n), "hipMalloc X");
+  hip_check(alloc(&P.y, sizeof(double) * (size_t)n), "hipMalloc y");
+  hip_check(alloc(&P.F, sizeof(double)), "hipMalloc F");
+  hip_check(alloc(&P.M, sizeof(double) * (size_t)n * n), "hipMalloc M");
   P.owns_M = true;
   hip_check(hipMemcpy(P.X, zeros.data(), sizeof(double) * n, hipMemcpyHostToDevice), "upload X");
   hip_check(hipMemcpy(P.y, zeros.data(), sizeof(double) * n, hipMemcpyHostToDevice), "upload y");
@@ -314,8 +401,8 @@ void Runtime::chol_block(const double* C, int n, const double* Loo, int no, doub
     }
   } fr{{&dC, &dL}};
   const size_t bn = sizeof(double) * (size_t)n * n;
-  hip_check(hipMalloc(&dC, bn), "hipMalloc");
-  hip_check(hipMalloc(&dL, bn), "hipMalloc");
+  hip_check(alloc(&dC, bn), "hipMalloc");
+  hip_check(alloc(&dL, bn), "hipMalloc");
   hip_check(hipMemcpy(dC, C, bn, hipMemcpyHostToDevice), "upload C");
   chol_block_device(dC, n, problem(pid).M, no, v.W, v.npad, no, dL);
   hip_check(hipMemcpy(L, dL, bn, hipMemcpyDeviceToHost), "read L");
@@ -350,10 +437,10 @@ bool Runtime::chol_block_device(const double* dC, int n, const double* dLoo, int
     }
   } fr{{&dB, &dU, &dCuu, &dS}};
   const size_t bu = sizeof(double) * (size_t)ldi * mpad, bs = sizeof(double) * (size_t)nu * nu;
-  hip_check(hipMalloc(&dB, bu), "hipMalloc");
-  hip_check(hipMalloc(&dU, bu), "hipMalloc");
-  hip_check(hipMalloc(&dCuu, bs), "hipMalloc");
-  hip_check(hipMalloc(&dS, bs), "hipMalloc");
+  hip_check(alloc(&dB, bu), "hipMalloc");
+  hip_check(alloc(&dU, bu), "hipMalloc");
+  hip_check(alloc(&dCuu, bs), "hipMalloc");
+  hip_check(alloc(&dS, bs), "hipMalloc");
   // C_ou (no x nu) into a zero-padded ldi x mpad block, C_uu (nu x nu)
   hip_check(hipMemsetAsync(dB, 0, bu, stream_), "clear");
   hip_check(hipMemcpy2DAsync(dB, sizeof(double) * ldi, dC + (size_t)no * n, sizeof(double) * n, sizeof(double) * no,
@@ -430,6 +517,7 @@ void Runtime::remove_problem(int id) {
   hipFree(it->second.F);
   if (it->second.owns_M && it->second.M) hipFree(it->second.M);
   problems_.erase(it);
+  if (problems_.empty()) scratch_trim();
   // slots that pointed at it must be rebuilt
   slot_problem_.clear();
 }
@@ -494,7 +582,7 @@ void Runtime::ensure_slots(const std::vector<EvalRequest>& reqs) {
   } else if (total > pool_bytes_) {
     if (pool_) hip_check(hipFree(pool_), "hipFree pool");
     pool_ = nullptr;
-    hip_check(hipMalloc(&pool_, total), "hipMalloc slot pool");
+    hip_check(alloc(&pool_, total), "hipMalloc slot pool");
     pool_bytes_ = total;
   }
   if (!noalloc_) base = reinterpret_cast<char*>(pool_);
@@ -532,9 +620,9 @@ void Runtime::ensure_slots(const std::vector<EvalRequest>& reqs) {
     if (h_params_) hipHostFree(h_params_);
     if (h_out_) hipHostFree(h_out_);
     const size_t cap = std::max<size_t>(ns, 8);
-    hip_check(hipMalloc(&d_slots_, sizeof(Slot) * cap), "hipMalloc slots");
-    hip_check(hipMalloc(&d_params_, sizeof(SlotParams) * cap), "hipMalloc params");
-    hip_check(hipMalloc(&d_out_, sizeof(SlotOut) * cap), "hipMalloc out");
+    hip_check(alloc(&d_slots_, sizeof(Slot) * cap), "hipMalloc slots");
+    hip_check(alloc(&d_params_, sizeof(SlotParams) * cap), "hipMalloc params");
+    hip_check(alloc(&d_out_, sizeof(SlotOut) * cap), "hipMalloc out");
     hip_check(hipHostMalloc(&h_params_, sizeof(SlotParams) * cap, hipHostMallocCoherent),
               "hipHostMalloc params");
     hip_check(hipHostMalloc(&h_out_, sizeof(SlotOut) * cap, hipHostMallocCoherent), "hipHostMalloc out");

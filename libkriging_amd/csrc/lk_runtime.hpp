@@ -9,6 +9,7 @@
 #include <cstdint>
 #include <functional>
 #include <map>
+#include <mutex>
 #include <memory>
 #include <stdexcept>
 #include <string>
@@ -206,7 +207,34 @@ class Runtime {
   hipStream_t stream() const { return stream_; }
   int device() const { return device_; }
 
+  // hipMalloc that first gives the idle scratch blocks back when memory is out
+  hipError_t alloc(void** ptr, size_t bytes);
+  template <class T>
+  hipError_t alloc(T** ptr, size_t bytes) {
+    return alloc(reinterpret_cast<void**>(ptr), bytes);
+  }
+
  private:
+  // Scratch of the calls that need it for their own duration (ScratchLease):
+  // a device block and a pinned host block, which the next call takes up
+  // again.  At most kScratchBlocks idle ones and kScratchKeep bytes (a larger
+  // block is freed when its call ends); all are freed when the last problem
+  // is removed, when an allocation fails and with the runtime.
+  friend class ScratchLease;
+  struct ScratchBlock {
+    char* dev = nullptr;
+    size_t dev_bytes = 0;
+    char* pin = nullptr;
+    size_t pin_bytes = 0;
+  };
+  static constexpr size_t kScratchKeep = size_t(2) << 30, kScratchKeepPinned = size_t(64) << 20;
+  static constexpr size_t kScratchBlocks = 4;
+  std::mutex scratch_mutex_;
+  std::vector<ScratchBlock> scratch_idle_;
+  ScratchBlock scratch_take(size_t dev_bytes, size_t pin_bytes);
+  void scratch_give(ScratchBlock b);
+  static void scratch_free(ScratchBlock& b);
+  void scratch_trim();
   void ensure_slots(const std::vector<EvalRequest>& reqs);
   int slot_of(int req) const;  // slot of request `req` of the last evaluate()
   void add_lmp_prior(const std::vector<EvalRequest>& reqs, std::vector<EvalResult>& res, bool want_grad) const;
@@ -307,6 +335,44 @@ class Runtime {
   hipEvent_t tev_[2] = {nullptr, nullptr};
   double timed_sum_ms_ = 0.0;
   int timed_count_ = 0;
+};
+
+// Device and pinned host memory for one call.  The caller's work on it is
+// enqueued on the runtime's stream; finished() says that the stream has been
+// waited for, otherwise (an exception) the end of the lease waits.
+class ScratchLease {
+ public:
+  ScratchLease(Runtime& rt, size_t dev_bytes, size_t pin_bytes)
+      : rt_(rt), b_(rt.scratch_take(dev_bytes, pin_bytes)) {}
+  ~ScratchLease();
+  ScratchLease(const ScratchLease&) = delete;
+  ScratchLease& operator=(const ScratchLease&) = delete;
+  char* dev() const { return b_.dev; }
+  char* pin() const { return b_.pin; }
+  void finished() { finished_ = true; }
+
+ private:
+  Runtime& rt_;
+  Runtime::ScratchBlock b_;
+  bool finished_ = false;
+};
+
+// consecutive 256-byte aligned parts of one block: sizes first (base null),
+// then the pointers
+class Carve {
+ public:
+  explicit Carve(char* base = nullptr) : base_(base) {}
+  template <class T>
+  T* take(size_t count) {
+    T* q = base_ == nullptr ? nullptr : reinterpret_cast<T*>(base_ + at_);
+    at_ += (sizeof(T) * count + 255) / 256 * 256;
+    return q;
+  }
+  size_t bytes() const { return at_; }
+
+ private:
+  char* base_;
+  size_t at_ = 0;
 };
 
 }  // namespace lk

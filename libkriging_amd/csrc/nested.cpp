@@ -417,12 +417,12 @@ void NestedKriging::precompute_nk() {
   });
   npairs_ = (int)pairs.size();
 
-  hip_check(hipMalloc(&d_Xg_, sizeof(double) * Xg.size()), "hipMalloc");
-  hip_check(hipMalloc(&d_Linv_, sizeof(double) * lsize), "hipMalloc");
-  hip_check(hipMalloc(&d_alpha_, sizeof(double) * Npad_), "hipMalloc");
-  hip_check(hipMalloc(&d_groups_, sizeof(NkGroup) * p), "hipMalloc");
-  hip_check(hipMalloc(&d_tile_group_, sizeof(int) * tg.size()), "hipMalloc");
-  if (npairs_ > 0) hip_check(hipMalloc(&d_pairs_, sizeof(int2) * pairs.size()), "hipMalloc");
+  hip_check(rt_->alloc(&d_Xg_, sizeof(double) * Xg.size()), "hipMalloc");
+  hip_check(rt_->alloc(&d_Linv_, sizeof(double) * lsize), "hipMalloc");
+  hip_check(rt_->alloc(&d_alpha_, sizeof(double) * Npad_), "hipMalloc");
+  hip_check(rt_->alloc(&d_groups_, sizeof(NkGroup) * p), "hipMalloc");
+  hip_check(rt_->alloc(&d_tile_group_, sizeof(int) * tg.size()), "hipMalloc");
+  if (npairs_ > 0) hip_check(rt_->alloc(&d_pairs_, sizeof(int2) * pairs.size()), "hipMalloc");
   hip_check(hipMemcpy(d_Xg_, Xg.data(), sizeof(double) * Xg.size(), hipMemcpyHostToDevice), "upload");
   hip_check(hipMemcpy(d_groups_, G.data(), sizeof(NkGroup) * p, hipMemcpyHostToDevice), "upload");
   hip_check(hipMemcpy(d_tile_group_, tg.data(), sizeof(int) * tg.size(), hipMemcpyHostToDevice), "upload");
@@ -458,7 +458,7 @@ void NestedKriging::precompute_nk() {
     for (int a = 0; a < ng; ++a) r[goff_[g] + a] = ys[a] - beta0_ * Fs[a];
   }
   double* d_r = nullptr;
-  hip_check(hipMalloc(&d_r, sizeof(double) * Npad_), "hipMalloc");
+  hip_check(rt_->alloc(&d_r, sizeof(double) * Npad_), "hipMalloc");
   try {
     hip_check(hipMemcpyAsync(d_r, r.data(), sizeof(double) * Npad_, hipMemcpyHostToDevice, rt_->stream()), "upload");
     NkArgs a{};
@@ -557,40 +557,38 @@ void NestedKriging::predict_nk(const double* Xn, int m, bool want_stdev, double*
   }
   qc = std::min(qc, m);
   const int qpad_max = (qc + NB - 1) / NB * NB;
+  fallbacks_ = 0;
+  const size_t pp = (size_t)p * p;
   double *dXc = nullptr, *dC = nullptr, *dU = nullptr, *dM = nullptr, *dKd = nullptr, *dKM = nullptr, *dKF = nullptr,
          *dout = nullptr;
-  int* dinfo = nullptr;
-  auto cleanup = [&] {
-    dfree(dXc);
-    dfree(dC);
-    dfree(dU);
-    dfree(dM);
-    dfree(dKd);
-    dfree(dKM);
-    dfree(dKF);
-    dfree(dout);
-    dfree(dinfo);
+  // out (2 qc) and info (qc ints) come down in one copy
+  const size_t down_bytes = sizeof(double) * 2 * qc + sizeof(int) * qc;
+  auto layout = [&](Carve& c) {
+    dXc = c.take<double>((size_t)qc * d);
+    dC = c.take<double>((size_t)Npad_ * qpad_max);
+    dU = c.take<double>(u_rows * qpad_max);
+    dM = c.take<double>((size_t)qc * p);
+    dKd = c.take<double>((size_t)qc * p);
+    dKM = c.take<double>((size_t)qc * pp);
+    dKF = c.take<double>((size_t)qc * pp);
+    dout = reinterpret_cast<double*>(c.take<char>(down_bytes));
   };
-  fallbacks_ = 0;
-  try {
-    const size_t pp = (size_t)p * p;
-    hip_check(hipMalloc(&dXc, sizeof(double) * (size_t)qc * d), "hipMalloc");
-    hip_check(hipMalloc(&dC, sizeof(double) * (size_t)Npad_ * qpad_max), "hipMalloc");
-    hip_check(hipMalloc(&dU, sizeof(double) * u_rows * qpad_max), "hipMalloc");
-    hip_check(hipMalloc(&dM, sizeof(double) * (size_t)qc * p), "hipMalloc");
-    hip_check(hipMalloc(&dKd, sizeof(double) * (size_t)qc * p), "hipMalloc");
-    hip_check(hipMalloc(&dKM, sizeof(double) * (size_t)qc * pp), "hipMalloc");
-    hip_check(hipMalloc(&dKF, sizeof(double) * (size_t)qc * pp), "hipMalloc");
-    hip_check(hipMalloc(&dout, sizeof(double) * 2 * (size_t)qc), "hipMalloc");
-    hip_check(hipMalloc(&dinfo, sizeof(int) * (size_t)qc), "hipMalloc");
-    std::vector<double> xc((size_t)qc * d), hout(2 * (size_t)qc);
-    std::vector<int> hinfo(qc);
+  Carve sizes;
+  layout(sizes);
+  ScratchLease lease(*rt_, sizes.bytes(), sizeof(double) * (size_t)qc * d + down_bytes);
+  Carve parts(lease.dev());
+  layout(parts);
+  int* const dinfo = reinterpret_cast<int*>(dout + 2 * (size_t)qc);
+  double* const xc = reinterpret_cast<double*>(lease.pin());
+  double* const hout = xc + (size_t)qc * d;
+  const int* const hinfo = reinterpret_cast<const int*>(hout + 2 * (size_t)qc);
+  {
     hipStream_t st = rt_->stream();
     for (int s0 = 0; s0 < m; s0 += qc) {
       const int mc = std::min(qc, m - s0);
       for (int k = 0; k < d; ++k)
         for (int t = 0; t < mc; ++t) xc[t + (size_t)k * mc] = Xn[s0 + t + (size_t)k * m];
-      hip_check(hipMemcpyAsync(dXc, xc.data(), sizeof(double) * (size_t)mc * d, hipMemcpyHostToDevice, st), "upload");
+      hip_check(hipMemcpyAsync(dXc, xc, sizeof(double) * (size_t)mc * d, hipMemcpyHostToDevice, st), "upload");
       NkArgs a{};
       a.Xg = d_Xg_;
       a.Linv = d_Linv_;
@@ -625,8 +623,7 @@ void NestedKriging::predict_nk(const double* Xn, int m, bool want_stdev, double*
       hip_check(launch_nk_pairs(a, st), "nk pairs");
       if (time_pairs_) hip_check(hipEventRecord(pev_[1], st), "event record");
       hip_check(launch_nk_solve(a, st), "nk solve");
-      hip_check(hipMemcpyAsync(hout.data(), dout, sizeof(double) * 2 * mc, hipMemcpyDeviceToHost, st), "download");
-      hip_check(hipMemcpyAsync(hinfo.data(), dinfo, sizeof(int) * mc, hipMemcpyDeviceToHost, st), "download");
+      hip_check(hipMemcpyAsync(hout, dout, down_bytes, hipMemcpyDeviceToHost, st), "download");
       hip_check(hipStreamSynchronize(st), "sync");
       if (time_pairs_) {
         float ms = 0.f;
@@ -660,11 +657,8 @@ void NestedKriging::predict_nk(const double* Xn, int m, bool want_stdev, double*
         if (want_stdev && stdev != nullptr) stdev[s0 + t] = std::sqrt(var);
       }
     }
-  } catch (...) {
-    cleanup();
-    throw;
   }
-  cleanup();
+  lease.finished();
 }
 
 std::string NestedKriging::summary() const {
