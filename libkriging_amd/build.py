@@ -19,6 +19,7 @@ LIB = os.path.join(HERE, "liblkgpu.so")
 SOURCES = [
     "lk_kernels.hip",
     "lk_potrf.hip",
+    "lk_predict.hip",
     "lk_nested.hip",
     "lk_loo.hip",
     "lk_noalloc.hip",

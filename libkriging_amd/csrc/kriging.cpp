@@ -960,19 +960,15 @@ void Kriging::predict(const double* Xn, int m, bool want_stdev, double* mean, do
   const size_t nup = ncoef + (size_t)chunk * d, ndown = 2 * (size_t)chunk + 2 * nder;
   const size_t ncov = want_cov ? (size_t)m * m : 0;
   const bool stage_cov = want_cov && cov != nullptr && ncov * sizeof(double) <= (size_t(16) << 20);
-  double *dup = nullptr, *dout = nullptr, *dRon = nullptr, *dC = nullptr, *dEc = nullptr, *dCov = nullptr,
-         *dDR = nullptr, *dDW = nullptr;
+  const int groups = want_deriv ? 1 + d : 1;
+  double *dup = nullptr, *dout = nullptr, *dRon = nullptr, *dC = nullptr, *dEc = nullptr, *dCov = nullptr;
   auto layout = [&](Carve& c) {
     dup = c.take<double>(nup);
     dout = c.take<double>(ndown);
-    dRon = c.take<double>((size_t)npad_ * mpad_max);
-    dC = c.take<double>((size_t)npad_ * mpad_max);
+    dRon = c.take<double>((size_t)npad_ * mpad_max * groups);
+    dC = c.take<double>((size_t)npad_ * mpad_max * groups);
     if ((want_cov || want_deriv) && p > 0) dEc = c.take<double>((size_t)chunk * p);
     if (want_cov) dCov = c.take<double>(ncov);
-    if (want_deriv) {
-      dDR = c.take<double>((size_t)npad_ * mpad_max * d);
-      dDW = c.take<double>((size_t)npad_ * mpad_max * d);
-    }
   };
   Carve sizes;
   layout(sizes);
@@ -1010,11 +1006,9 @@ void Kriging::predict(const double* Xn, int m, bool want_stdev, double* mean, do
       a.ecirc = dEc;
       a.cov = dCov;
       a.nn_factor = nug ? alpha_ : 1.0;
-      a.DR = dDR;
-      a.DW = dDW;
       a.dmean = dout + 2 * (size_t)chunk;
       a.dvar = a.dmean + nder;
-      for (int k = 0; k < d; ++k) a.theta[k] = theta_[k];
+      for (int k = 0; k < DMAX; ++k) a.itheta[k] = (k < d) ? 1.0 / theta_[k] : 1.0;
       a.factor = nug ? alpha_ : 1.0;
       a.n = n_;
       a.d = d;
@@ -1022,12 +1016,13 @@ void Kriging::predict(const double* Xn, int m, bool want_stdev, double* mean, do
       a.p = p;
       a.m = mc;
       a.mpad = (mc + NB - 1) / NB * NB;
+      a.groups = groups;
       a.kernel = kernel_id(kernel_);
       a.linear_trend = regmodel_ == RegModel::Linear;
       a.want_var = want_stdev ? 1 : 0;
       hip_check(launch_predict(a, rt_->stream()), "predict");
-      if (want_cov) hip_check(launch_predict_cov(a, rt_->stream()), "predict cov");
       if (want_deriv) hip_check(launch_predict_deriv(a, rt_->stream()), "predict deriv");
+      if (want_cov) hip_check(launch_predict_cov(a, rt_->stream()), "predict cov");
       // the variances' derivatives, last, only when they were asked for
       const size_t nd = !want_deriv ? 2 * (size_t)mc : ndown - (want_stdev ? 0 : nder);
       hip_check(hipMemcpyAsync(host_out, dout, sizeof(double) * nd, hipMemcpyDeviceToHost, rt_->stream()), "download");

@@ -186,23 +186,23 @@ struct PredictArgs {
   const double* MZ;    // npad x (p + 1): [M = F* | z]
   const double* coef;  // beta (p) then R* (p x p, column-major upper)
   const double* Xn;    // m x d new points (normalised), ld = m
-  double* Ron;         // npad x mpad workspace: R(x_obs, x_new)
-  double* C;           // npad x mpad workspace: L^-1 R_on
+  // npad rows of groups * mpad columns, point j of group g at g mpad + j: R_on
+  // = R(x_obs, x_new) in group 0, dR_on / dx_new,k in group 1 + k (derivatives
+  // wanted: groups = 1 + d, else 1); C = L^-1 of it
+  double* Ron;
+  double* C;
   double* out;         // 2 m: mean (normalised), variance factor
   double* ecirc;       // m x p (ld = m): E circ rows, when cov or derivatives are wanted (else null)
   // covariance (KrigingImpl.cpp:245-253): m x m, ld = m, before var_scale
   double* cov;
   double nn_factor;    // R_nn_factor (alpha for the nugget model); diagonal 1
-  // derivatives (KrigingImpl.cpp:255-291): dR_on / dx_new and L^-1 of it,
-  // npad x (d mpad) with column k mpad + j for point j and coordinate k;
-  // dmean, dvar: m x d (ld = m), normalised units
-  double* DR;
-  double* DW;
+  // derivatives (KrigingImpl.cpp:255-291): dmean, dvar: m x d (ld = m),
+  // normalised units
   double* dmean;
   double* dvar;
-  double theta[DMAX];
+  double itheta[DMAX];  // 1 / theta
   double factor;       // R_on_factor (alpha for the nugget model)
-  int n, d, npad, p, m, mpad;
+  int n, d, npad, p, m, mpad, groups;
   int kernel, linear_trend;
   int want_var;        // derivatives of the variance too
 };
@@ -219,9 +219,9 @@ struct CovMatArgs {
   int pad_;
 };
 hipError_t launch_cov_mat(const CovMatArgs& a, hipStream_t stream);
-// C = Linv R_on alone (PredictArgs' Linv, Ron, C, npad, mpad; both padded
-// to whole 64-row blocks, Linv's diagonal blocks zero above the diagonal)
-hipError_t launch_trmm_lower(const PredictArgs& a, hipStream_t stream);
+// C = Linv B, Linv npad x npad (lower, its diagonal blocks zero above the
+// diagonal), B and C npad x cpad (ld = npad), all in whole 64-row blocks
+hipError_t launch_trmm_lower(const double* Linv, const double* B, double* C, int npad, int cpad, hipStream_t stream);
 // Schur complement of a block Cholesky update: S = Cuu - U' U, with U
 // kdim x mpad (ld = kdim, both padded to whole 64-row blocks, zero padding),
 // Cuu and S m x m (ld = m); S is written in full (both triangles)

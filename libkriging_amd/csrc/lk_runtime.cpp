@@ -450,13 +450,7 @@ bool Runtime::chol_block_device(const double* dC, int n, const double* dLoo, int
                              sizeof(double) * nu, nu, hipMemcpyDeviceToDevice, stream_),
             "copy C_uu");
   // U = Loo^-1 C_ou = L_ou' (LinearAlgebra.cpp:271), S = C_uu - U' U
-  PredictArgs t{};
-  t.Linv = dLooInv;
-  t.Ron = dB;
-  t.C = dU;
-  t.npad = ldi;
-  t.mpad = mpad;
-  hip_check(launch_trmm_lower(t, stream_), "trmm");
+  hip_check(launch_trmm_lower(dLooInv, dB, dU, ldi, mpad, stream_), "trmm");
   SchurArgs sa{};
   sa.U = dU;
   sa.Cuu = dCuu;
