@@ -327,6 +327,94 @@ __device__ inline void tile_mainloop(const double* __restrict__ A, int lda, int 
 }
 
 // ---------------------------------------------------------------------------
+// One 16 x 16 block per wave, operands straight from memory into the MFMA's
+// registers, sixteen steps of 4 ahead: for launches with so few tiles that
+// the chain of a tile's chunks (stage, barrier, multiply) is their time, and
+// a quarter of the workgroup's quarter is enough work per wave.  The same
+// products in the same order as tile_mainloop: bit for bit its block.
+// acc: element e of lane l is row (l & 15), column (l >> 4) + 4 e.
+// kend - kbeg a multiple of 64.
+// ---------------------------------------------------------------------------
+template <bool NEG>
+__device__ inline void block16_direct(const double* __restrict__ A, int lda, int ai0, const double* __restrict__ B,
+                                      int ldb, int bj0, int kbeg, int kend, d4& acc, int lane) {
+  constexpr int D = 16;
+  const int r16 = lane & 15, kq = lane >> 4, nst = (kend - kbeg) / 4;
+  const double* Ap = A + (size_t)(kbeg + kq) * lda + ai0 + r16;
+  const double* Bp = B + (size_t)(kbeg + kq) * ldb + bj0 + r16;
+  double a[D], b[D];
+  auto load = [&](int u, int s) __attribute__((always_inline)) {
+    a[u] = gload(Ap + (size_t)(4 * s) * lda);
+    b[u] = gload(Bp + (size_t)(4 * s) * ldb);
+  };
+  if (nst <= 0) return;
+#pragma unroll
+  for (int u = 0; u < D; ++u) {
+    __builtin_amdgcn_sched_barrier(0);
+    load(u, u);
+  }
+  for (int s = D; s < nst; s += D) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      __builtin_amdgcn_sched_barrier(0);
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(b[u], NEG ? -a[u] : a[u], acc, 0, 0, 0);
+      load(u, s + u);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < D; ++u) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(b[u], NEG ? -a[u] : a[u], acc, 0, 0, 0);
+}
+
+// The same with B transposed (k contiguous: B[j * ldb + k]): 16 lanes of an
+// operand load would touch 16 lines, so the 32 columns of the workgroup's
+// four waves go through LDS, 64 k at a time, a chunk ahead.  bw: this wave's
+// first column of the 32.  sB: 2 * B16_BUF doubles.
+constexpr int B16_S = 33;  // odd: the transposed stores and the reads are conflict-free
+constexpr int B16_BUF = 64 * B16_S;
+__device__ inline void block16_bt(const double* __restrict__ A, int lda, int ai0, const double* __restrict__ B,
+                                  int ldb, int bj0, int bw, int kbeg, int kend, double* __restrict__ sB, d4& acc,
+                                  int tid) {
+  constexpr int D = 16;
+  const int lane = tid & 63, r16 = lane & 15, kq = lane >> 4, nch = (kend - kbeg) / 64;
+  const double* Ap = A + (size_t)(kbeg + kq) * lda + ai0 + r16;
+  const int sj = tid >> 3, sk = 2 * (tid & 7);  // staged: column sj, k = sk + 16 q and the next
+  const double* Bp = B + (size_t)(bj0 + sj) * ldb + kbeg + sk;
+  double a[D];
+  d2 rb[4];
+  auto load_b = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) rb[q] = gload(reinterpret_cast<const d2*>(Bp + 64 * c + 16 * q));
+  };
+  if (nch <= 0) return;
+  load_b(0);
+#pragma unroll
+  for (int u = 0; u < D; ++u) {
+    __builtin_amdgcn_sched_barrier(0);
+    a[u] = gload(Ap + (size_t)(4 * u) * lda);
+  }
+  for (int c = 0; c < nch; ++c) {
+    double* buf = sB + (c & 1) * B16_BUF;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      buf[(sk + 16 * q) * B16_S + sj] = rb[q].x;
+      buf[(sk + 16 * q + 1) * B16_S + sj] = rb[q].y;
+    }
+    __syncthreads();
+    const int cn = min(c + 1, nch - 1);  // (the last chunk again: dropped)
+    load_b(cn);
+    double b[D];
+#pragma unroll
+    for (int u = 0; u < D; ++u) b[u] = buf[(4 * u + kq) * B16_S + bw + r16];
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      __builtin_amdgcn_sched_barrier(0);
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(b[u], a[u], acc, 0, 0, 0);
+      a[u] = gload(Ap + (size_t)(64 * cn + 4 * u) * lda);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Wide tiles: 128 rows (two 64-row blocks of A) x 64 columns per 256-thread
 // workgroup, both operands plain (i contiguous in memory); wave (wr, wc) owns
 // rows 64 wr .. 64 wr + 63 and columns 32 wc .. 32 wc + 31 as 4 x 2 MFMA

@@ -235,6 +235,31 @@ __global__ __launch_bounds__(TPB, 4) void k_potrf_update(const Slot* __restrict_
   update_tile(S, r, c, kb, ke, sbuf);
 }
 
+// The same, a quarter of a tile (32 x 32) per workgroup and 16 x 16 of it per
+// wave: bound by one load, K / 4 MFMAs and one store in a row.  grid (4
+// tiles, nslots)
+__global__ __launch_bounds__(TPB) void k_potrf_update_s(const Slot* __restrict__ slots,
+                                                        const SlotParams* __restrict__ params,
+                                                        SlotOut* __restrict__ out, int kb, int ke, int c0, int c1) {
+  const TileSlot ts = tile_slot();
+  const int b = ts.slot;
+  const Slot S = slots[b];
+  if (!slot_live(params[b], out[b]) || params[b].mode == MODE_FACTOR) return;
+  const int nb = S.nblk;
+  if (c0 >= nb || ke > nb) return;
+  int r, c;
+  if (!update_tile_rc(ts.tile >> 2, nb, c0, c1, r, c)) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, ld = S.npad;
+  const int i0 = r * NB + 32 * (ts.tile & 1) + 16 * (w & 1), j0 = c * NB + 16 * (ts.tile & 2) + 16 * (w >> 1);
+  double* C = S.A + (size_t)(j0 + (lane >> 4)) * ld + i0 + (lane & 15);
+  d4 acc;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc[e] = gload(C + (size_t)(4 * e) * ld);
+  block16_direct<true>(S.A, ld, i0, S.A, ld, j0, kb * NB, ke * NB, acc, lane);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) C[(size_t)(4 * e) * ld] = acc[e];
+}
+
 // The trailing update (every column from c0 on) on 128 x 64 tiles: column c's
 // row blocks c, c+1, ... taken in pairs (the last one alone when their count
 // is odd).  Tile t -> (c, first row block).  grid (tiles, nslots)
@@ -338,6 +363,40 @@ __global__ __launch_bounds__(TPB, 4) void k_trtri(const Slot* __restrict__ slots
     tile_mainloop<false, false, true>(S.W, ld, i0, S.W, ld, j0, bot * NB, (it + 1) * NB, sbuf, acc, tid, lane, wr,
                                       wc);
     acc_store(acc, S.W + (size_t)j0 * ld + i0, ld, lane, wr, wc);
+  }
+}
+
+// The same, a quarter of a tile (32 x 32) per workgroup and 16 x 16 of it per
+// wave.  Step 0's Linv is transposed and goes through LDS (read straight from
+// memory a level of n = 1500 took 41 us, so 18).  grid (4 npairs_max * s * s,
+// nslots)
+__global__ __launch_bounds__(TPB) void k_trtri_s(const Slot* __restrict__ slots, const SlotParams* __restrict__ params,
+                                                 SlotOut* __restrict__ out, int s, int step) {
+  const TileSlot ts = tile_slot();
+  const int b = ts.slot;
+  const Slot S = slots[b];
+  if (!slot_live(params[b], out[b])) return;
+  const int per_pair = s * s, tile = ts.tile >> 2;
+  const int pr = tile / per_pair, rem = tile % per_pair;
+  const int ti = (step == 0) ? rem % s : s - 1 - rem / s;
+  const int tj = (step == 0) ? rem / s : rem % s;
+  const int top = 2 * pr * s, bot = top + s;
+  const int it = bot + ti, jt = top + tj;
+  if (bot >= S.nblk || it >= S.nblk) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, ld = S.npad;
+  const int i0 = it * NB + 32 * (ts.tile & 1) + 16 * (w & 1), j0 = jt * NB + 16 * (ts.tile & 2) + 16 * (w >> 1);
+  const int i = i0 + (lane & 15), j = j0 + (lane >> 4);
+  d4 acc = d4{0.0, 0.0, 0.0, 0.0};
+  if (step == 0) {
+    __shared__ double sB[2 * B16_BUF];
+    block16_bt(S.A, ld, i0, S.W, ld, jt * NB + 16 * (ts.tile & 2), 16 * (w >> 1), jt * NB, (top + s) * NB, sB, acc,
+               (int)threadIdx.x);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) S.W[(size_t)i * ld + j + 4 * e] = acc[e];
+  } else {
+    block16_direct<true>(S.W, ld, i0, S.W, ld, j0, bot * NB, (it + 1) * NB, acc, lane);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) S.W[(size_t)(j + 4 * e) * ld + i] = acc[e];
   }
 }
 
@@ -1349,6 +1408,14 @@ hipError_t launch_build(const Batch& B) {
     hipLaunchKernelGGL(k_build<32>, grid, dim3(TPB), 0, B.stream, B.slots, B.params, B.out);
   return hipGetLastError();
 }
+// Up to here (64 x 64 tiles in the launch) the quarter-tile kernels: below,
+// the launch is one tile's chain, above it is the MFMA and LDS staging reads
+// the operands once for four waves.  Updates of one n = 4096 Cholesky: 697 us
+// without the line, 621 at 256 tiles, 631 at 512, 681 at 1024; its L^-1
+// levels: 581, 584 at 256, 563 at 512.  n = 1000: an update 11.9 -> 6.3 us, a
+// level 20.3 -> 8.8; n = 1500: 12.5 -> 8.1 and 26 -> 13.4.
+constexpr int kUpdateSmall = 256;
+constexpr int kTrtriSmall = 512;
 hipError_t launch_potrf_update(const Batch& B, int kb, int ke, int c0, int c1) {
   const int nb = B.nblk_max;
   if (c0 >= nb) return hipSuccess;
@@ -1359,6 +1426,11 @@ hipError_t launch_potrf_update(const Batch& B, int kb, int ke, int c0, int c1) {
     for (int c = c0; c <= c1 && c < nb; ++c) tiles += nb - c;
   }
   if (tiles <= 0) return hipSuccess;
+  if (tiles * B.nslots <= kUpdateSmall) {
+    hipLaunchKernelGGL(k_potrf_update_s, dim3(4 * tiles, B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params, B.out, kb,
+                       ke, c0, c1);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_potrf_update, dim3(tiles, B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params, B.out, kb, ke,
                      c0, c1);
   return hipGetLastError();
@@ -1396,6 +1468,11 @@ int trtri_levels(int nblk) {
 hipError_t launch_trtri_level(const Batch& B, int s, int step) {
   const int npairs = (B.nblk_max + 2 * s - 1) / (2 * s);
   if (npairs <= 0) return hipSuccess;
+  if (npairs * s * s * B.nslots <= kTrtriSmall) {
+    hipLaunchKernelGGL(k_trtri_s, dim3(4 * npairs * s * s, B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params, B.out,
+                       s, step);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_trtri, dim3(npairs * s * s, B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params, B.out, s,
                      step);
   return hipGetLastError();
