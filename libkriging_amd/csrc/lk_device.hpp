@@ -654,26 +654,91 @@ __device__ inline double kern_rho_g(int kern, const double* dx, const double* it
 }
 
 // The matrix-vector kernels stream the L^-1 (and L) triangles once; they
-// run 16 waves per workgroup and issue MV_U independent loads per lane
-// before the first dependent FMA, so a workgroup keeps ~64 KB in flight
-// instead of one 512-byte line per wave (one workgroup per 64-row block:
-// for one large matrix the last row block's workgroup reads its whole
-// row alone, at what its loads in flight allow).
+// run 16 waves per workgroup with a batch of independent loads per lane in
+// flight before the first dependent FMA and the next batch behind them (one
+// workgroup per 64-row block: for one large matrix the last row block's
+// workgroup reads its whole row alone, at what its loads in flight allow).
 constexpr int MV_TPB = 1024;
 constexpr int MV_W = MV_TPB / 64;
 constexpr int MV_U = 8;
 static_assert(4 * MV_U <= 64, "one lane per (input column, batch column)");
 
+// a uniform read of memory that no launch in flight writes (scalar unit)
+__device__ inline double sload(const double* p) { return *(const __attribute__((address_space(4))) double*)p; }
+
+// acc += sum over this wave's columns k < kend of W(row, k) col(k), one input
+// column: read by the scalar unit, an operand of the FMA.  Batches of 16, the
+// next one's loads in flight (n = 8192: 106 -> 81 us, n = 4096: 45 -> 31; with
+// four columns always computed from broadcast lanes the loop was bound by
+// its instructions).
+__device__ inline double lower_matvec_one(const double* __restrict__ Wr, int ld, int kend, int w,
+                                          const double* __restrict__ col) {
+  constexpr int U = 16, STEP = MV_W * U;
+  double acc = 0.0;
+  auto load = [&](double (&lv)[U], int kb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) lv[u] = gload(Wr + (size_t)min(kb + u, kend - 1) * ld);
+  };
+  auto add = [&](const double (&lv)[U], int kb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (kb + u < kend) acc = fma(lv[u], sload(col + kb + u), acc);
+  };
+  auto add_whole = [&](const double (&lv)[U], int kb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc = fma(lv[u], sload(col + kb + u), acc);
+  };
+  double la[U], lb[U];
+  int kb = w * U;
+  if (kb >= kend) return acc;
+  load(la, kb);
+  while (true) {
+    if (kb + STEP < kend) load(lb, kb + STEP);
+    kb + U <= kend ? add_whole(la, kb) : add(la, kb);
+    kb += STEP;
+    if (kb >= kend) break;
+    if (kb + STEP < kend) load(la, kb + STEP);
+    kb + U <= kend ? add_whole(lb, kb) : add(lb, kb);
+    kb += STEP;
+    if (kb >= kend) break;
+  }
+  return acc;
+}
+
+// The same for NC input columns, batches of MV_U.  Lane c MV_U + u fetches
+// column c at k = kb + u: one coalesced load per batch instead of NC MV_U
+// same-address loads, each of which would move 64 lanes' worth of data;
+// v_readlane broadcasts.  (By the scalar unit a batch of 32 n = 1024 slots
+// took 57 us, so 43 or less: its cache serves two CUs' waves.)
+template <int NC>
+__device__ inline void lower_matvec_cols(const double* __restrict__ Wr, int ld, int kend, int w,
+                                         const double* __restrict__ my_col, double (&acc)[4]) {
+  const int lane = threadIdx.x & 63, ul = lane % MV_U;
+  for (int kb = w * MV_U; kb < kend; kb += MV_W * MV_U) {
+    double lv[MV_U];
+#pragma unroll
+    for (int u = 0; u < MV_U; ++u) lv[u] = gload(Wr + (size_t)min(kb + u, kend - 1) * ld);
+    const double sv = (lane < NC * MV_U) ? gload(my_col + min(kb + ul, kend - 1)) : 0.0;
+#pragma unroll
+    for (int u = 0; u < MV_U; ++u)
+      if (kb + u < kend) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[c] = fma(lv[u], readlane_d(sv, c * MV_U + u), acc[c]);
+      }
+  }
+}
+
 // out[:, c] = Linv * in[:, c] for rows of block rb (grid (nblk_max, nslots))
 // in columns come from `src` (n rows, ld = n, zero beyond n) ; out to V.
 // Column c of the input is src[c * lds + k] for c < ncols_src and src2[k]
 // for c == ncols_src (when src2 is given), so [F | y] go through in one pass.
-// Wave w sums columns k in batches [w U + j W U, w U + j W U + U); the
-// partial sums of the waves are added in a fixed order (deterministic).
+// The partial sums of the waves are added in a fixed order (deterministic).
+// ONE: one input column, written by earlier launches only (scalar unit).
+template <bool ONE>
 __device__ inline void lower_matvec_block(const Slot& S, int rb, const double* __restrict__ src, int lds, int nsrc,
                                           int ncols, double* __restrict__ dst, int ldd, double* __restrict__ part_sq,
                                           const double* __restrict__ src2 = nullptr) {
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i0 = rb * NB, ld = S.npad, n = S.n;
   const int kend = min(i0 + NB, n);  // columns k <= row, and k < n (src is zero beyond n)
   __shared__ double red[MV_W][4][NB];
@@ -681,7 +746,6 @@ __device__ inline void lower_matvec_block(const Slot& S, int rb, const double* _
   double ssq = 0.0;
   for (int c0 = 0; c0 < ncols; c0 += 4) {
     const int nc = min(4, ncols - c0);
-    // columns past nc re-read column c0 (same cache lines) and are dropped
     const double* colp[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -689,26 +753,13 @@ __device__ inline void lower_matvec_block(const Slot& S, int rb, const double* _
       colp[c] = (src2 != nullptr && cs == ncols - 1) ? src2 : src + (size_t)cs * lds;
     }
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    // lane c MV_U + u (< 4 MV_U) fetches input column c at k = kb + u: one
-    // coalesced load per batch instead of 4 MV_U same-address loads, each of
-    // which would move 64 lanes' worth of data; v_readlane broadcasts
-    const int cl = lane / MV_U, ul = lane % MV_U;
-    const double* my_col = colp[cl & 3];
-    for (int kb = w * MV_U; kb < kend; kb += MV_W * MV_U) {
-      double lv[MV_U];
-#pragma unroll
-      for (int u = 0; u < MV_U; ++u) {
-        const int k = min(kb + u, kend - 1);
-        lv[u] = gload(Wr + (size_t)k * ld);
-      }
-      const double sv = (lane < 4 * MV_U) ? gload(my_col + min(kb + ul, kend - 1)) : 0.0;
-#pragma unroll
-      for (int u = 0; u < MV_U; ++u)
-        if (kb + u < kend) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) acc[c] = fma(lv[u], readlane_d(sv, c * MV_U + u), acc[c]);
-        }
-    }
+    const double* my_col = colp[(lane / MV_U) & 3];
+    if constexpr (ONE)
+      acc[0] = lower_matvec_one(Wr, ld, kend, w, colp[0]);
+    else if (nc <= 2)
+      lower_matvec_cols<2>(Wr, ld, kend, w, my_col, acc);
+    else
+      lower_matvec_cols<4>(Wr, ld, kend, w, my_col, acc);
 #pragma unroll
     for (int c = 0; c < 4; ++c) red[w][c][lane] = acc[c];
     __syncthreads();

@@ -414,7 +414,7 @@ __global__ __launch_bounds__(MV_TPB) void k_solve_fy(const Slot* __restrict__ sl
   if (!slot_live(params[b], out[b]) || ts.tile >= S.nblk) return;
   const int rb = ts.tile;
   // [F | y] -> V columns 0 .. p in one pass over this row block of Linv
-  lower_matvec_block(S, rb, S.F, S.n, S.n, S.p + 1, S.V, S.npad, nullptr, S.y);
+  lower_matvec_block<false>(S, rb, S.F, S.n, S.n, S.p + 1, S.V, S.npad, nullptr, S.y);
   // this row block's part of F*'F* and F*'y* (upper triangle and last column
   // of [F* | y*]'[F* | y*], a-major), for k_gls: its columns were just
   // written by this workgroup
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(MV_TPB) void k_solve_e(const Slot* __restrict__ slo
   if (!slot_live(params[b], out[b]) || ts.tile >= S.nblk) return;
   const double* r = S.V + (size_t)(S.p + 1) * S.npad;
   double* e = S.V + (size_t)(S.p + 2) * S.npad;
-  lower_matvec_block(S, ts.tile, r, S.npad, S.n, 1, e, S.npad, S.red + red_sse_off(S.nblk));
+  lower_matvec_block<true>(S, ts.tile, r, S.npad, S.n, 1, e, S.npad, S.red + red_sse_off(S.nblk));
 }
 
 // x = Linv^T E*, and the 1-norms (max column abs sums) of L and Linv
@@ -547,8 +547,7 @@ __global__ __launch_bounds__(MV_TPB) void k_solve_x(const Slot* __restrict__ slo
   // given as input had no panel step: then all of L is read)
   const int lend = (params[b].mode == MODE_FACTOR) ? ld : (ts.tile + 1) * NB;
   // wave w takes the block's columns c0 .. c0 + CW - 1 together: one pass
-  // down the rows with one load of E* and CW coalesced column loads in
-  // flight per row group (the reductions run once per column at the end)
+  // down the rows (the reductions run once per column at the end)
   constexpr int CW = NB / MV_W;  // columns per wave
   const int c0 = ts.tile * NB + CW * w;
   double s[CW], aw[CW];
@@ -557,28 +556,63 @@ __global__ __launch_bounds__(MV_TPB) void k_solve_x(const Slot* __restrict__ slo
     s[q] = 0.0;
     aw[q] = 0.0;
   }
-  for (int i = c0 + lane; i < ld; i += 64) {
+  // the diagonal block's rows, then XU groups of 64 whole rows at a time: XU
+  // (CW + 1) loads in flight per lane, no test per element (n = 4096: 50 ->
+  // 45 us, n = 8192: 128 -> 116)
+  {
+    const int i = ts.tile * NB + lane;
     const double ev = gload(e + i);
-    double wv[CW];
 #pragma unroll
-    for (int q = 0; q < CW; ++q) wv[q] = gload(S.W + (size_t)(c0 + q) * ld + i);
-#pragma unroll
-    for (int q = 0; q < CW; ++q)
+    for (int q = 0; q < CW; ++q) {
+      const double wv = gload(S.W + (size_t)(c0 + q) * ld + i);
       if (i >= c0 + q) {  // the lower triangle only
-        s[q] = fma(wv[q], ev, s[q]);
-        aw[q] += fabs(wv[q]);
+        s[q] = fma(wv, ev, s[q]);
+        aw[q] += fabs(wv);
       }
+    }
   }
+  constexpr int XU = 4;
+  auto rows = [&](int i0, auto utag) __attribute__((always_inline)) {
+    constexpr int U = decltype(utag)::value;
+    double ev[U], wv[U][CW];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      ev[u] = gload(e + i0 + 64 * u + lane);
+#pragma unroll
+      for (int q = 0; q < CW; ++q) wv[u][q] = gload(S.W + (size_t)(c0 + q) * ld + i0 + 64 * u + lane);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int q = 0; q < CW; ++q) {
+        s[q] = fma(wv[u][q], ev[u], s[q]);
+        aw[q] += fabs(wv[u][q]);
+      }
+  };
+  int i0 = (ts.tile + 1) * NB;
+  for (; i0 + 64 * XU <= ld; i0 += 64 * XU) rows(i0, std::integral_constant<int, XU>{});
+  for (; i0 < ld; i0 += 64) rows(i0, std::integral_constant<int, 1>{});
+  // |L|'s column sums: the four columns' loads together
+  double al4[CW];
+#pragma unroll
+  for (int q = 0; q < CW; ++q) al4[q] = 0.0;
+  for (int i = ts.tile * NB + lane; i < lend; i += 64)
+#pragma unroll
+    for (int q = 0; q < CW; ++q) {
+      const double v = fabs(gload(S.A + (size_t)(c0 + q) * ld + i));
+      if (i >= c0 + q) al4[q] += v;
+    }
+  if (lend < ld)
+    // four partial sums per row block (lcol_part in lk_potrf.hip)
+    for (int r = 4 * (ts.tile + 1) + lane; r < 4 * S.nblk; r += 64) {
+      const double* Lp = S.A + (size_t)((r >> 2) * NB + (r & 3)) * ld + c0;
+#pragma unroll
+      for (int q = 0; q < CW; ++q) al4[q] += gload(Lp + q);
+    }
 #pragma unroll
   for (int q = 0; q < CW; ++q) {
     const int c = c0 + q;
-    const double* __restrict__ Ac = S.A + (size_t)c * ld;
-    double al = 0.0;
-    for (int i = c + lane; i < lend; i += 64) al += fabs(gload(Ac + i));
-    if (lend < ld)
-      // four partial sums per row block (lcol_part in lk_potrf.hip)
-      for (int r = 4 * (ts.tile + 1) + lane; r < 4 * S.nblk; r += 64)
-        al += S.A[(size_t)((r >> 2) * NB + (r & 3)) * ld + c];
+    double al = al4[q];
     const double sx = wave_sum(s[q]);
     const double awx = wave_sum(aw[q]);
     al = wave_sum(al);

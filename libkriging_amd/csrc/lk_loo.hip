@@ -159,7 +159,7 @@ __global__ __launch_bounds__(MV_TPB) void k_loo_wv(const Slot* __restrict__ slot
   const Slot S = slots[b];
   if (!slot_live(params[b], out[b]) || !params[b].want_grad || ts.tile >= S.nblk) return;
   const int p = S.p, ld = S.npad;
-  lower_matvec_block(S, ts.tile, S.V + (size_t)v_loo_w(p) * ld, ld, S.n, 1, S.V + (size_t)v_loo_t(p) * ld, ld,
+  lower_matvec_block<true>(S, ts.tile, S.V + (size_t)v_loo_w(p) * ld, ld, S.n, 1, S.V + (size_t)v_loo_t(p) * ld, ld,
                      nullptr);
 }
 
