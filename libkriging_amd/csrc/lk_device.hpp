@@ -414,6 +414,50 @@ __device__ inline void block16_bt(const double* __restrict__ A, int lda, int ai0
   }
 }
 
+// The same with both operands transposed, both through LDS.  aw, bw: this
+// wave's first row and column of the workgroup's 32 x 32.  sAB: 4 * B16_BUF.
+__device__ inline void block16_tt(const double* __restrict__ A, int lda, int ai0, int aw, const double* __restrict__ B,
+                                  int ldb, int bj0, int bw, int kbeg, int kend, double* __restrict__ sAB, d4& acc,
+                                  int tid) {
+  constexpr int D = 16;
+  const int lane = tid & 63, r16 = lane & 15, kq = lane >> 4, nch = (kend - kbeg) / 64;
+  const int sj = tid >> 3, sk = 2 * (tid & 7);
+  const double* Ap = A + (size_t)(ai0 + sj) * lda + kbeg + sk;
+  const double* Bp = B + (size_t)(bj0 + sj) * ldb + kbeg + sk;
+  d2 ra[4], rb[4];
+  auto load = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      ra[q] = gload(reinterpret_cast<const d2*>(Ap + 64 * c + 16 * q));
+      rb[q] = gload(reinterpret_cast<const d2*>(Bp + 64 * c + 16 * q));
+    }
+  };
+  if (nch <= 0) return;
+  load(0);
+  for (int c = 0; c < nch; ++c) {
+    double* bufa = sAB + (c & 1) * 2 * B16_BUF;
+    double* bufb = bufa + B16_BUF;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      bufa[(sk + 16 * q) * B16_S + sj] = ra[q].x;
+      bufa[(sk + 16 * q + 1) * B16_S + sj] = ra[q].y;
+      bufb[(sk + 16 * q) * B16_S + sj] = rb[q].x;
+      bufb[(sk + 16 * q + 1) * B16_S + sj] = rb[q].y;
+    }
+    __syncthreads();
+    if (c + 1 < nch) load(c + 1);
+    double a[D], b[D];
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      a[u] = bufa[(4 * u + kq) * B16_S + aw + r16];
+      b[u] = bufb[(4 * u + kq) * B16_S + bw + r16];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < D; ++u) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(b[u], a[u], acc, 0, 0, 0);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Wide tiles: 128 rows (two 64-row blocks of A) x 64 columns per 256-thread
 // workgroup, both operands plain (i contiguous in memory); wave (wr, wc) owns

@@ -35,16 +35,19 @@ __host__ __device__ inline int tri_n(int t) { return t * (t + 1) / 2; }
 }  // namespace
 
 // ---------------------------------------------------------------------------
-// G' = (R*^-T F*' L^-1)' and diag(B).  grid (nblk_max, nslots), 256 threads;
-// wave w of column block cb handles columns j = 64 cb + w, w + 4, ...; trend
-// columns go four at a time through the rows i >= j of column j of L^-1.
+// G' = (R*^-T F*' L^-1)' and diag(B).  16 columns of L^-1 per workgroup, four
+// per wave; trend columns go four at a time (a constant trend's one alone)
+// through the rows i >= j of column j.  Bound by the loads each CU can issue,
+// so by how many CUs take part: n = 1500, 24 workgroups of 64 columns 67 us,
+// with 16 waves each 57, 96 of 16 columns 18.
+// grid (4 nblk_max, nslots), 256 threads
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(TPB) void k_loo_g(const Slot* __restrict__ slots, const SlotParams* __restrict__ params,
                                                SlotOut* __restrict__ out) {
   const TileSlot ts = tile_slot();
   const int b = ts.slot;
   const Slot S = slots[b];
-  if (!slot_live(params[b], out[b]) || ts.tile >= S.nblk) return;
+  if (!slot_live(params[b], out[b]) || ts.tile >= 4 * S.nblk) return;
   const int p = S.p, n = S.n, ld = S.npad;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const double* __restrict__ rs = S.red + red_rstar_off(S.nblk);  // R* upper, rs[a + c p]
@@ -52,8 +55,8 @@ __global__ __launch_bounds__(TPB) void k_loo_g(const Slot* __restrict__ slots, c
   double* __restrict__ bd = S.V + (size_t)v_loo_s2(p) * ld;
   __shared__ double hbuf[4][PMAX];
   constexpr int XU = 4;
-  for (int cc = w; cc < NB; cc += 4) {
-    const int j = ts.tile * NB + cc;
+  for (int cc = w; cc < NB / 4; cc += 4) {
+    const int j = ts.tile * (NB / 4) + cc;
     if (j >= n) {  // padded column: L^-1 e_j = e_j, G e_j = 0
       if (lane == 0) {
         for (int a = 0; a < p; ++a) Gt[(size_t)a * ld + j] = 0.0;
@@ -68,23 +71,30 @@ __global__ __launch_bounds__(TPB) void k_loo_g(const Slot* __restrict__ slots, c
       const double* fcol[4];
 #pragma unroll
       for (int c = 0; c < 4; ++c) fcol[c] = S.V + (size_t)min(a0 + c, max(p - 1, 0)) * ld;
-      for (int b0 = j; b0 < n; b0 += 64 * XU) {
-        double wv[XU], fv[XU][4];
+      auto sums = [&](auto ftag) __attribute__((always_inline)) {
+        constexpr int NF = decltype(ftag)::value;
+        for (int b0 = j; b0 < n; b0 += 64 * XU) {
+          double wv[XU], fv[XU][NF];
 #pragma unroll
-        for (int u = 0; u < XU; ++u) {
-          const int i = min(b0 + 64 * u + lane, n - 1);
-          wv[u] = gload(Wc + i);
+          for (int u = 0; u < XU; ++u) {
+            const int i = min(b0 + 64 * u + lane, n - 1);
+            wv[u] = gload(Wc + i);
 #pragma unroll
-          for (int c = 0; c < 4; ++c) fv[u][c] = gload(fcol[c] + i);
-        }
-#pragma unroll
-        for (int u = 0; u < XU; ++u)
-          if (b0 + 64 * u + lane < n) {
-            if (a0 == 0) nrm = fma(wv[u], wv[u], nrm);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) h[c] = fma(fv[u][c], wv[u], h[c]);
+            for (int c = 0; c < NF; ++c) fv[u][c] = gload(fcol[c] + i);
           }
-      }
+#pragma unroll
+          for (int u = 0; u < XU; ++u)
+            if (b0 + 64 * u + lane < n) {
+              if (a0 == 0) nrm = fma(wv[u], wv[u], nrm);
+#pragma unroll
+              for (int c = 0; c < NF; ++c) h[c] = fma(fv[u][c], wv[u], h[c]);
+            }
+        }
+      };
+      if (p - a0 > 1)
+        sums(std::integral_constant<int, 4>{});
+      else
+        sums(std::integral_constant<int, 1>{});
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const double v = wave_sum(h[c]);
@@ -277,6 +287,39 @@ __global__ __launch_bounds__(TPB) void k_loo_bs(const Slot* __restrict__ slots, 
       }
 }
 
+// The same, a quarter of a tile per workgroup and 16 x 16 of it per wave (few
+// tiles: see block16_tt).  grid (4 tiles, nslots)
+__global__ __launch_bounds__(TPB) void k_loo_bs_s(const Slot* __restrict__ slots, const SlotParams* __restrict__ params,
+                                                  SlotOut* __restrict__ out) {
+  const TileSlot ts = tile_slot();
+  const int b = ts.slot;
+  const Slot S = slots[b];
+  if (!slot_live(params[b], out[b]) || !params[b].want_grad) return;
+  if ((ts.tile >> 2) >= tri_n(S.nblk)) return;
+  int it, jt;
+  tri_decode(ts.tile >> 2, it, jt);
+  const int p = S.p, ld = S.npad, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int i0 = it * NB + 32 * (ts.tile & 1), j0 = jt * NB + 16 * (ts.tile & 2);
+  const int aw = 16 * (w & 1), bw = 16 * (w >> 1);
+  __shared__ double sAB[4 * B16_BUF];
+  d4 acc = d4{0.0, 0.0, 0.0, 0.0};
+  block16_tt(S.W, ld, i0, aw, S.W, ld, j0, bw, it * NB, S.nblk * NB, sAB, acc, tid);
+  const double* __restrict__ Gt = S.V + (size_t)v_loo_g(p) * ld;
+  const double* __restrict__ sa = S.V + (size_t)v_loo_sa(p) * ld;
+  const int i = i0 + aw + (lane & 15), j = j0 + bw + (lane >> 4);
+  for (int a = 0; a < p; ++a) {
+    const double gi = gload(Gt + (size_t)a * ld + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = fma(-gi, gload(Gt + (size_t)a * ld + j + 4 * e), acc[e]);
+  }
+  const double si = gload(sa + i);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    S.A[(size_t)(j + 4 * e) * ld + i] = acc[e] * gload(sa + j + 4 * e);
+    if (it != jt) S.A[(size_t)i * ld + j + 4 * e] = acc[e] * si;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // C = Bs Bs' tile by tile (full K) and its contraction with dR/dtheta_k:
 // partial_k = sum over the tile's pairs gi > gj of
@@ -441,7 +484,7 @@ hipError_t launch_rinv_store(const Batch& B) {
   return hipGetLastError();
 }
 hipError_t launch_loo_g(const Batch& B) {
-  hipLaunchKernelGGL(k_loo_g, dim3(B.nblk_max, B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params, B.out);
+  hipLaunchKernelGGL(k_loo_g, dim3(4 * B.nblk_max, B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params, B.out);
   return hipGetLastError();
 }
 hipError_t launch_loo_value(const Batch& B) {
@@ -456,9 +499,18 @@ hipError_t launch_loo_bw(const Batch& B) {
   hipLaunchKernelGGL(k_loo_bw, dim3(B.nblk_max, B.nslots), dim3(MV_TPB), 0, B.stream, B.slots, B.params, B.out);
   return hipGetLastError();
 }
+// quarter tiles up to here (64 x 64 tiles in the launch): the whole objective
+// with gradient at n = 1500 (300 tiles) 905 us against 930, n = 1900 (465)
+// 1155 against 1176, n = 2300 (666) 1715 against 1716, n = 3000 2570 against
+// 2516
+constexpr int kBsSmall = 512;
 hipError_t launch_loo_bs(const Batch& B) {
-  hipLaunchKernelGGL(k_loo_bs, dim3(tri_n(B.nblk_max), B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params,
-                     B.out);
+  if (tri_n(B.nblk_max) * B.nslots <= kBsSmall)
+    hipLaunchKernelGGL(k_loo_bs_s, dim3(4 * tri_n(B.nblk_max), B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params,
+                       B.out);
+  else
+    hipLaunchKernelGGL(k_loo_bs, dim3(tri_n(B.nblk_max), B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params,
+                       B.out);
   return hipGetLastError();
 }
 hipError_t launch_loo_adjoint(const Batch& B) {
