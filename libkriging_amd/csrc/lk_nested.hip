@@ -515,18 +515,26 @@ __global__ __launch_bounds__(TPB, 2) void k_nk_pair_few(NkArgs a, int tbase) {
 // (7) per point: KM = cross + diag(Kd + jitter); w = KM^-1 diag(KM) by
 // Cholesky (arma::solve with likely_sympd); on a non-positive pivot, LU with
 // partial pivoting on the same system (the general solver Armadillo falls
-// back to).  One workgroup per point; the factor lives in KF (global, L2).
+// back to).  One workgroup per point.  Bound by the chain of p columns and two
+// substitutions, a few accesses to the factor each: it is in LDS up to
+// NK_PLDS groups (32 groups, 500 points: 90 -> 62 us), in KF (global,
+// L2) beyond.
 // ---------------------------------------------------------------------------
 constexpr int NK_PMAX = 2048;  // groups supported by the solve kernel (LDS vectors)
+constexpr int NK_PLDS = 64;    // 33 KB: four workgroups per CU
 
+template <bool LDS>
 __global__ __launch_bounds__(TPB) void k_nk_solve(NkArgs a) {
   const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int p = a.p;
   const size_t pp = (size_t)p * p;
   double* K = a.KM + (size_t)t * pp;
+  constexpr int PM = LDS ? NK_PLDS : NK_PMAX;
+  __shared__ double sF[LDS ? NK_PLDS * NK_PLDS : 1];
   double* F = a.KF + (size_t)t * pp;
-  __shared__ double kM[NK_PMAX];
-  __shared__ double z[NK_PMAX];
+  if constexpr (LDS) F = sF;
+  __shared__ double kM[PM];
+  __shared__ double z[PM];
   __shared__ double sw[4];
   __shared__ int swi[4];
   __shared__ int spk;
@@ -783,7 +791,10 @@ hipError_t launch_nk_pairs(const NkArgs& args, hipStream_t stream) {
 
 hipError_t launch_nk_solve(const NkArgs& a, hipStream_t stream) {
   if (a.p > NK_PMAX) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_nk_solve, dim3(a.qc), dim3(TPB), 0, stream, a);
+  if (a.p <= NK_PLDS)
+    hipLaunchKernelGGL(k_nk_solve<true>, dim3(a.qc), dim3(TPB), 0, stream, a);
+  else
+    hipLaunchKernelGGL(k_nk_solve<false>, dim3(a.qc), dim3(TPB), 0, stream, a);
   return hipGetLastError();
 }
 

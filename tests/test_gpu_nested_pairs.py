@@ -19,6 +19,8 @@ WIDTHS = [1, 16, 17, 32, 33, 64, 65, 128, 129, 300, 385, 512, 513, 576, 580, 650
     ("exp", 9, [3, 66, 128]),
     ("gauss", 32, [1, 1, 40, 70]),
     ("exp", 1, [5] * 12),
+    ("exp", 3, [3] * 64),  # the largest system solved in LDS
+    ("exp", 3, [3] * 65),
 ])
 def test_pair_widths(kernel, d, sizes):
     import libkriging_amd as lk
