@@ -116,11 +116,11 @@ constexpr int GRAD_STRIDE = 2 * DMAX + 4;
 // R* = chol_upper(F*'F*), p x p column-major, after the adjoint partials
 __host__ __device__ inline int red_rstar_off(int nblk) { return 4 * nblk + nblk * (nblk + 1) / 2 * GRAD_STRIDE; }
 // per diagonal block k, after R*: 64 max|L_kk| max|L_kk^-1|, a bound on
-// cond(L_kk) up to the factor 64 (written by the diagonal-block kernel, read
-// by the panel kernel)
+// cond(L_kk) up to the factor 64 (written by k_potrf_chain, read by
+// k_potrf_rows)
 __host__ __device__ inline int red_cond_off(int nblk) { return red_rstar_off(nblk) + PMAX * PMAX; }
 __host__ __device__ inline size_t red_size(int nblk) { return (size_t)red_cond_off(nblk) + nblk; }
-// Panels whose diagonal block's condition estimate exceeds this get one step
+// Rows whose diagonal block's condition estimate exceeds this get one step
 // of iterative refinement: multiplying by the explicit inverse of an
 // ill-conditioned block is not backward stable, the refined product is.
 constexpr double PANEL_REFINE_COND = 1e4;

@@ -747,6 +747,10 @@ hipError_t launch_potrf_rows(const Batch& B, int k, int nb) {
   const int blocks = B.nblk_max - k - nb;
   if (blocks <= 0) return hipSuccess;
   if (nb < 1 || nb > 2) return hipErrorInvalidValue;
+  // 16-row workgroups while they fit the chip at once (four per CU), else
+  // 64-row ones, which read the square's inverse once for four times the rows:
+  // all rows of a 64 x n = 1024 batch in two streams 340 us with the line at
+  // 1024 workgroups, 346 with 16-row ones throughout, 423 with the line at 256
   const long long groups = 4LL * blocks * B.nslots;
   if (groups <= 1024)
     hipLaunchKernelGGL(k_potrf_rows<1>, dim3(4 * blocks, B.nslots), dim3(TPB), 0, B.stream, B.slots, B.params, B.out,
