@@ -74,7 +74,7 @@ struct ChainLds {
   double L[NB * CS];  // the diagonal block, then its factor (above the diagonal: not meaningful)
   double X[NB * CS];  // its inverse's lower 16 x 16 blocks, by rows: X(i, k) at [i * CS + k]
   double T[NB * CS];  // the tile below it: A, then L
-  double U[NB * CS];  // refinement: the unrefined tile
+  double U[NB * CS];  // refinement: the unrefined tile; then diag_panel's copy of block (0, 0)
   double eye[16 * CS];  // identity, 16 x 16
   double piv[NB];     // pivots; given factor: reciprocals of its diagonal
   float mx[5];
@@ -116,7 +116,9 @@ __device__ inline void diag_tile_update(ChainLds& sh, int rb, int cb, int p, int
 // Panel p by one wave.  Lanes 0-15: rows of the diagonal 16 x 16 block; 16-31:
 // identity rows, becoming L_pp^-T; 32-63: rows of 16-row blocks p + 1 and
 // p + 2 (lanes past the block's end compute values that are dropped).  With
-// `last`, a repetition of panel 0 for block 3's rows alone (lanes 16-31).
+// `last`, a repetition of panel 0 for block 3's rows alone (lanes 16-31); its
+// diagonal rows are read from sh.U, for the first wave overwrites them in
+// sh.L with no barrier between.
 __device__ inline void diag_panel(ChainLds& sh, int p, bool last, int l) {
   const int j0 = 16 * p, gi = l >> 4, r = l & 15;
   int row = j0 + r;
@@ -124,7 +126,7 @@ __device__ inline void diag_panel(ChainLds& sh, int p, bool last, int l) {
   if (last && gi == 1) row = 48 + r;
   const bool ident = gi == 1 && !last;
   const bool keep = last ? gi == 1 : (ident || row < NB);
-  const double* src = ident ? sh.eye + r : sh.L + j0 * CS + min(row, NB - 1);
+  const double* src = ident ? sh.eye + r : (last && gi != 1) ? sh.U + r : sh.L + j0 * CS + min(row, NB - 1);
   double v[16];
 #pragma unroll
   for (int c = 0; c < 16; ++c) v[c] = src[c * CS];
@@ -333,6 +335,10 @@ __device__ inline void u_update(ChainLds& sh, int w, int i, d4& D, int l) {
   if (t.rb < 0) return;
   tile_syrk<16>(D, sh.T, 0, t.rb, t.cb, l);
   tile_put(sh, t.rb, t.cb, D, l);
+  if (i == 0 && w == 0) {  // block (0, 0) again, for diag_panel's repetition
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sh.U[((l >> 4) + 4 * e) * CS + (l & 15)] = D[e];
+  }
 }
 
 // maximum over the wave's lanes of a value that is not negative
@@ -536,6 +542,10 @@ __global__ __launch_bounds__(CH_TPB) void k_potrf_chain(const Slot* __restrict__
     for (int i = tid; i < 16 * 16; i += CH_TPB) sh.eye[(i >> 4) * CS + (i & 15)] = ((i >> 4) == (i & 15)) ? 1.0 : 0.0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) sh.L[(w + 8 * i) * CS + l] = v0[i];
+    if (l < 16) {  // block (0, 0) again, for diag_panel's repetition
+      sh.U[w * CS + l] = v0[0];
+      sh.U[(w + 8) * CS + l] = v0[1];
+    }
   }
   if (given) take_factor(sh, tid);
   __syncthreads();
