@@ -151,7 +151,8 @@ __device__ inline void diag_panel(ChainLds& sh, int p, bool last, int l) {
 }
 
 // The diagonal of panel p (lanes 0-15): the pivots' roots, corrected by one
-// Newton step; sh.bad on a non-positive or NaN pivot
+// Newton step; sh.bad on a non-positive or NaN pivot.  The wave's other lanes
+// read them afterwards.
 __device__ inline void diag_roots(ChainLds& sh, int p, int l) {
   if (l < 16) {
     const int c = 16 * p + l;
@@ -159,6 +160,7 @@ __device__ inline void diag_roots(ChainLds& sh, int p, int l) {
     sh.L[c * CS + c] = fma(fma(-t, t, a), 0.5 * iv, t);
     if (!(a > 0.0)) sh.bad = 1;
   }
+  wave_lds_fence();
 }
 
 // Given factor: X_qq = L_qq^-1 (16 x 16) into sh.X, lane = column

@@ -63,3 +63,11 @@ def test_order_of_waves_does_not_matter(emu, n, make):
     for order in (FORWARD[::-1], [1, 0, 3, 2, 5, 4, 7, 6], [4, 5, 6, 7, 0, 1, 2, 3]):
         assert same(emu(A, order), ref), order
     assert same(emu(A, FORWARD, rb4=True), ref)
+
+
+@pytest.mark.parametrize("n,make", [(64, spd), (128, graded), (192, spd)])
+def test_order_of_lanes_does_not_matter(emu, n, make):
+    A = make(n)
+    ref = emu(A)
+    assert ref[3] == 0
+    assert same(emu(A, lanes_reversed=True), ref)
