@@ -11,8 +11,6 @@
 
 #include <math.h>
 
-#include <type_traits>
-
 #include "lk_device.hpp"
 #include "lk_kernels.h"
 
@@ -77,7 +75,7 @@ struct ChainLds {
   double U[NB * CS];  // refinement: the unrefined tile; then diag_panel's copy of block (0, 0)
   double eye[16 * CS];  // identity, 16 x 16
   double piv[NB];     // pivots; given factor: reciprocals of its diagonal
-  float mx[5];
+  double mx[5];
   int bad;
 };
 
@@ -184,9 +182,9 @@ __device__ inline void given_inverse16(ChainLds& sh, int q, int l) {
     for (int i = 0; i < 16; ++i) sh.X[(o + i) * CS + o + j] = x[i];
 }
 
-__device__ inline float max_abs(const d4& t, float m) {
+__device__ inline double max_abs(const d4& t, double m) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) m = fmaxf(m, fabsf((float)t[e]));
+  for (int e = 0; e < 4; ++e) m = fmax(m, fabs(t[e]));
   return m;
 }
 
@@ -206,7 +204,7 @@ __device__ inline d4 inverse_block(ChainLds& sh, int i, int q, const d4& S, int 
 // row t - 1 (the diagonal one from the panel, the others from the sum of the
 // step before), then the sum of row t.  X[j] holds block (q + j, q).
 // Returns the running maximum of their magnitude.
-__device__ inline float inverse_step(ChainLds& sh, int t, int q, d4 (&X)[3], d4& S, float m, int l) {
+__device__ inline double inverse_step(ChainLds& sh, int t, int q, d4 (&X)[3], d4& S, double m, int l) {
   const int r = l & 15, g = l >> 4;
   if (q > t - 1) return m;
   if (q == t - 1) {
@@ -241,7 +239,7 @@ __device__ inline double* diag_ptr(double* M, int kk, int ld) { return M + (size
 
 // panel p's columns of L (rows from the panel's first on) to memory; the
 // running maximum of their magnitude
-__device__ inline float store_panel(const ChainLds& sh, double* Ab, int ld, int p, float m, int l) {
+__device__ inline double store_panel(const ChainLds& sh, double* Ab, int ld, int p, double m, int l) {
   double v[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) v[i] = sh.L[(16 * p + i) * CS + l];
@@ -251,7 +249,7 @@ __device__ inline float store_panel(const ChainLds& sh, double* Ab, int ld, int 
     for (int i = 0; i < 16; ++i) Ab[(size_t)(16 * p + i) * ld + l] = v[i];
   }
 #pragma unroll
-  for (int i = 0; i < 16; ++i) m = (l >= 16 * p + i) ? fmaxf(m, fabsf((float)v[i])) : m;
+  for (int i = 0; i < 16; ++i) m = (l >= 16 * p + i) ? fmax(m, fabs(v[i])) : m;
   return m;
 }
 // 16 columns (from c0) of T to memory, and their sums of magnitudes over each
@@ -343,35 +341,18 @@ __device__ inline void u_update(ChainLds& sh, int w, int i, d4& D, int l) {
   }
 }
 
-// maximum over the wave's lanes of a value that is not negative
-__device__ inline float wave_max_f(float v) {
-  auto ror = [](float x, auto n) {
-    return __int_as_float(
-        __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + decltype(n)::value, 0xf, 0xf, false));
-  };
-  v = fmaxf(v, ror(v, std::integral_constant<int, 8>{}));
-  v = fmaxf(v, ror(v, std::integral_constant<int, 4>{}));
-  v = fmaxf(v, ror(v, std::integral_constant<int, 2>{}));
-  v = fmaxf(v, ror(v, std::integral_constant<int, 1>{}));
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-
 // Factor of sh.L in place and its inverse's lower 16 x 16 blocks into sh.X,
 // both stored to the diagonal block kk of A and W but for store_rest's part.
 // `given`: sh.L and sh.piv already hold a factor; only the inverse is formed.
 // `behind`: the second block of a square; the rest of its update by T (D,
 // u_tile), T's own stores and the first block's store_rest run beside its
 // first panels.  Every wave passes the same barriers.
-// Returns the condition estimate 64 max|L| max|L^-1| (PANEL_REFINE_COND; the
-// maxima rounded to single precision: it is compared with a power of ten).
+// Returns the condition estimate 64 max|L| max|L^-1| (PANEL_REFINE_COND).
 __device__ inline double diag_block(ChainLds& sh, const Slot& S, int kk, bool given, bool behind, d4 (&D)[3], int w,
                                     int lane) {
   // one loop per role: the addresses and conditions of one role's work stay
   // out of the others' registers (above all out of wave 0's scalar ones)
-  float m = 0.f;  // wave 4: max |L|; waves 5-7: max |L^-1|
+  double m = 0.0;  // wave 4: max |L|; waves 5-7: max |L^-1|
   const int q = w - 5;
   d4 X[3], R;
   if (w == 0) {
@@ -443,26 +424,25 @@ __device__ inline double diag_block(ChainLds& sh, const Slot& S, int kk, bool gi
   if (w == 4) {
     if (!given) diag_roots(sh, 3, l);
     // the last panel of L and the last diagonal block of the inverse
-    float x = 0.f;
+    double x = 0.0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int c = 48 + g + 4 * e;
-      if (r >= g + 4 * e) m = fmaxf(m, fabsf((float)sh.L[c * CS + 48 + r]));
-      x = fmaxf(x, fabsf((float)sh.X[(48 + r) * CS + c]));
+      if (r >= g + 4 * e) m = fmax(m, fabs(sh.L[c * CS + 48 + r]));
+      x = fmax(x, fabs(sh.X[(48 + r) * CS + c]));
     }
-    m = wave_max_f(m);
-    x = wave_max_f(x);
+    m = wave_max(m);
+    x = wave_max(x);
     if (l == 0) {
       sh.mx[0] = m;
       sh.mx[1] = x;
     }
   } else if (w > 4) {
-    m = wave_max_f(max_abs(inverse_block(sh, 3, q, R, l), m));
+    m = wave_max(max_abs(inverse_block(sh, 3, q, R, l), m));
     if (l == 0) sh.mx[w - 3] = m;
   }
   __syncthreads();
-  const double cond = (double)NB * (double)sh.mx[0] *
-                      (double)fmaxf(fmaxf(sh.mx[1], sh.mx[2]), fmaxf(sh.mx[3], sh.mx[4]));
+  const double cond = (double)NB * sh.mx[0] * fmax(fmax(sh.mx[1], sh.mx[2]), fmax(sh.mx[3], sh.mx[4]));
   if (w == 0 && l == 0) S.red[red_cond_off(S.nblk) + kk] = cond;
   return cond;
 }

@@ -71,3 +71,18 @@ def test_order_of_lanes_does_not_matter(emu, n, make):
     ref = emu(A)
     assert ref[3] == 0
     assert same(emu(A, lanes_reversed=True), ref)
+
+
+@pytest.mark.parametrize("exponent", [0, -600, 600])
+@pytest.mark.parametrize("make", [spd, graded])
+def test_condition_estimate_at_any_scale(emu, make, exponent):
+    # 64 max|L_kk| max|L_kk^-1| of what was stored, in 64 bits; a scaling by an
+    # even power of two scales the factor exactly, so the same blocks refine
+    n = 128
+    L0, W0, _, _ = emu(make(n))
+    L, W, cond, st = emu(make(n) * 2.0 ** exponent)
+    assert st == 0
+    assert np.array_equal(L, L0 * 2.0 ** (exponent // 2)) and np.array_equal(W, W0 * 2.0 ** (-exponent // 2))
+    for k in range(n // 64):
+        b = slice(64 * k, 64 * k + 64)
+        assert cond[k] == 64 * np.max(np.abs(L[b, b])) * np.max(np.abs(W[b, b]))
