@@ -17,7 +17,9 @@
 namespace lk {
 
 void hip_check(hipError_t e, const char* what) {
-  if (e != hipSuccess) throw HipError(std::string("HIP error in ") + what + ": " + hipGetErrorString(e));
+  if (e == hipSuccess) return;
+  (void)hipGetLastError();  // reported here, not by the next launch
+  throw HipError(std::string("HIP error in ") + what + ": " + hipGetErrorString(e));
 }
 
 std::string chol_failure_message(int status, int inc, double num_nugget) {
@@ -155,11 +157,28 @@ void Runtime::drop_graphs() {
   graphs_.clear();
 }
 
+// the slot, parameter and result tables, and the graphs, which read them
+void Runtime::free_tables() {
+  drop_graphs();
+  if (d_slots_) hipFree(d_slots_);
+  if (d_params_) hipFree(d_params_);
+  if (d_out_) hipFree(d_out_);
+  if (h_params_) hipHostFree(h_params_);
+  if (h_out_) hipHostFree(h_out_);
+  if (h_slots_pin_) hipHostFree(h_slots_pin_);
+  d_slots_ = nullptr;
+  d_params_ = nullptr;
+  d_out_ = nullptr;
+  h_params_ = nullptr;
+  h_out_ = nullptr;
+  h_slots_pin_ = nullptr;
+  slot_cap_ = 0;
+}
+
 Runtime::~Runtime() {
   hipSetDevice(device_);
   for (auto& e : tev_)
     if (e) hipEventDestroy(e);
-  drop_graphs();
   for (auto& kv : problems_) {
     hipFree(kv.second.X);
     hipFree(kv.second.y);
@@ -167,12 +186,7 @@ Runtime::~Runtime() {
     if (kv.second.owns_M && kv.second.M) hipFree(kv.second.M);
   }
   if (pool_) hipFree(pool_);
-  if (d_slots_) hipFree(d_slots_);
-  if (d_params_) hipFree(d_params_);
-  if (d_out_) hipFree(d_out_);
-  if (h_params_) hipHostFree(h_params_);
-  if (h_out_) hipHostFree(h_out_);
-  if (h_slots_pin_) hipHostFree(h_slots_pin_);
+  free_tables();
   if (fork_) hipEventDestroy(fork_);
   for (auto& e : la_ev_)
     if (e) hipEventDestroy(e);
@@ -541,6 +555,10 @@ void Runtime::ensure_slots(const std::vector<EvalRequest>& reqs) {
   std::vector<size_t> off(ns);
   size_t total = 0;
   int nblk_max = 0, dmax = 0;
+  // from here the slots are laid out anew: a failure on the way leaves no
+  // layout behind, and the next batch starts from none
+  slot_problem_.clear();
+  nslots_ = 0;
   h_slots_.assign(ns, Slot{});
   for (int s = 0; s < ns; ++s) {
     const DeviceProblem& P = problem(slot_prob[s]);
@@ -574,8 +592,10 @@ void Runtime::ensure_slots(const std::vector<EvalRequest>& reqs) {
     h_out_ = np_out_;
     base = scratch_ + t1 + t2 + t3;
   } else if (total > pool_bytes_) {
-    if (pool_) hip_check(hipFree(pool_), "hipFree pool");
+    double* const old = pool_;
     pool_ = nullptr;
+    pool_bytes_ = 0;
+    if (old) hip_check(hipFree(old), "hipFree pool");
     hip_check(alloc(&pool_, total), "hipMalloc slot pool");
     pool_bytes_ = total;
   }
@@ -606,13 +626,7 @@ void Runtime::ensure_slots(const std::vector<EvalRequest>& reqs) {
     S.noise = P.noise;
   }
   if (!noalloc_ && (size_t)ns > slot_cap_) {
-    drop_graphs();  // they read these tables
-    if (h_slots_pin_) hipHostFree(h_slots_pin_);
-    if (d_slots_) hipFree(d_slots_);
-    if (d_params_) hipFree(d_params_);
-    if (d_out_) hipFree(d_out_);
-    if (h_params_) hipHostFree(h_params_);
-    if (h_out_) hipHostFree(h_out_);
+    free_tables();
     const size_t cap = std::max<size_t>(ns, 8);
     hip_check(alloc(&d_slots_, sizeof(Slot) * cap), "hipMalloc slots");
     hip_check(alloc(&d_params_, sizeof(SlotParams) * cap), "hipMalloc params");

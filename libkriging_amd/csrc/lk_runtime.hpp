@@ -321,6 +321,7 @@ class Runtime {
   static constexpr size_t kMaxGraphs = 16;
   std::vector<GraphEntry> graphs_;
   void drop_graphs();
+  void free_tables();
   int last_objective_ = OBJ_LL;
   int timed_stage_ = -1;
   // the batch split into S equal parts on S streams: the latency-bound
