@@ -79,23 +79,22 @@ __global__ __launch_bounds__(TPB) void k_pred_cross(PredictArgs a) {
   }
 }
 
-// C = L^-1 R_on on 64 x 64 tiles, the longest rows first.  Bound by the MFMA:
-// each wave runs the whole tile (16 blocks of 16 x 16 for 8 operand loads a
-// step) over a quarter of the K range, its operands straight from memory into
-// registers four steps ahead, with no LDS and no barrier in the loop; the
-// four sums meet in LDS at the end.  n = 3001, 5003 points: 810 us, 58 TFLOP/s,
-// the MFMA busy 84 % of the time (staged through LDS, a quadrant per wave:
-// 850 .. 890 us and 76 %; 128 x 64 tiles that way: 837 us).
-// grid (columns / 64, npad / 64)
-__global__ __launch_bounds__(TPB, 2) void k_pred_trmm(PredictArgs a) {
-  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r16 = lane & 15, kq = lane >> 4;
-  const int t0 = blockIdx.x * NB, i0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * NB;
-  const int ld = a.groups * a.mpad;
-  __shared__ double sS[2 * NB * LDSS];
-  const int nst = (i0 + NB) / 4, s0 = nst * w / 4, s1 = nst * (w + 1) / 4;
-  const double* Pl = a.Linv + (size_t)kq * a.npad + i0 + r16;
-  const double* Ql = a.Ron + (size_t)kq * ld + t0 + r16;
+// ---------------------------------------------------------------------------
+// A 64 x 64 tile: sum_k P(i0 + row, k) Q(j0 + col, k) over [0, 4 nst), P and Q
+// with rows contiguous (P[k * ldp + row]).  Each wave runs the whole tile (16
+// blocks of 16 x 16 for 8 operand loads a step) over a quarter of the K range,
+// its operands straight from memory into registers four steps ahead, with no
+// LDS and no barrier in the loop; the four sums s_w meet in LDS as (s_0 + s_2)
+// + (s_1 + s_3), the order of tile32_sum too: an element has the same bits in
+// either.  v[r]: element (w + 4 r, lane).  sS: 2 NB LDSS doubles.
+// ---------------------------------------------------------------------------
+template <bool NEG>
+__device__ inline void tile64(const double* __restrict__ P, int ldp, int i0, const double* __restrict__ Q, int ldq,
+                              int j0, int nst, double* __restrict__ sS, double (&v)[16], int tid) {
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, kq = lane >> 4;
+  const int s0 = nst * w / 4, s1 = nst * (w + 1) / 4;
+  const double* Pl = P + (size_t)kq * ldp + i0 + r16;
+  const double* Ql = Q + (size_t)kq * ldq + j0 + r16;
   d4 acc[4][4];
 #pragma unroll
   for (int x = 0; x < 4; ++x)
@@ -107,8 +106,8 @@ __global__ __launch_bounds__(TPB, 2) void k_pred_trmm(PredictArgs a) {
     const size_t k = 4 * (size_t)min(s, s1 - 1);
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
-      p[u][x] = gload(Pl + k * a.npad + 16 * x);
-      q[u][x] = gload(Ql + k * ld + 16 * x);
+      p[u][x] = gload(Pl + k * ldp + 16 * x);
+      q[u][x] = gload(Ql + k * ldq + 16 * x);
     }
   };
 #pragma unroll
@@ -125,7 +124,7 @@ __global__ __launch_bounds__(TPB, 2) void k_pred_trmm(PredictArgs a) {
         for (int x = 0; x < 4; ++x)
 #pragma unroll
           for (int y = 0; y < 4; ++y)
-            acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(p[u][x], q[u][y], acc[x][y], 0, 0, 0);
+            acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(NEG ? -p[u][x] : p[u][x], q[u][y], acc[x][y], 0, 0, 0);
       }
       load(u, s + u + D);
     }
@@ -157,8 +156,24 @@ __global__ __launch_bounds__(TPB, 2) void k_pred_trmm(PredictArgs a) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int o = (w + 4 * r) * LDSS + lane;
-    a.C[(size_t)(i0 + w + 4 * r) * ld + t0 + lane] = sS[o] + sS[o + NB * LDSS];
+    v[r] = sS[o] + sS[o + NB * LDSS];
   }
+}
+
+// C = L^-1 R_on on 64 x 64 tiles, the longest rows first.  Bound by the MFMA:
+// n = 3001, 5003 points: 810 us, 58 TFLOP/s, the MFMA busy 84 % of the time
+// (staged through LDS, a quadrant per wave: 850 .. 890 us and 76 %; 128 x 64
+// tiles that way: 837 us).
+// grid (columns / 64, npad / 64)
+__global__ __launch_bounds__(TPB, 2) void k_pred_trmm(PredictArgs a) {
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int t0 = blockIdx.x * NB, i0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * NB;
+  const int ld = a.groups * a.mpad;
+  __shared__ double sS[2 * NB * LDSS];
+  double v[16];
+  tile64<false>(a.Linv, a.npad, i0, a.Ron, ld, t0, (i0 + NB) / 4, sS, v, tid);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) a.C[(size_t)(i0 + w + 4 * r) * ld + t0 + lane] = v[r];
 }
 
 // ---------------------------------------------------------------------------
@@ -223,15 +238,16 @@ __device__ inline void tile32(const double* __restrict__ P, int ldp, int i0, con
 }
 __device__ inline double tile32_sum(const double* sS, int row, int col) {
   const double* s = sS + row * T32_S + col;
-  return (s[0] + s[T32 * T32_S]) + (s[2 * T32 * T32_S] + s[3 * T32 * T32_S]);
+  return (s[0] + s[2 * T32 * T32_S]) + (s[T32 * T32_S] + s[3 * T32 * T32_S]);
 }
 
-// grid (columns / 32, npad / 32)
+// K ends with the 64-row block, as in k_pred_trmm: the quarters are the same,
+// and L^-1 is zero beyond the diagonal.  grid (columns / 32, npad / 32)
 __global__ __launch_bounds__(TPB) void k_pred_trmm32(PredictArgs a) {
   const int tid = threadIdx.x, t0 = blockIdx.x * T32, i0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * T32;
   const int ld = a.groups * a.mpad;
   __shared__ double sS[4 * T32 * T32_S];
-  tile32<false>(a.Linv, a.npad, i0, a.Ron, ld, t0, i0 + T32, sS, tid);
+  tile32<false>(a.Linv, a.npad, i0, a.Ron, ld, t0, (i0 / NB + 1) * NB, sS, tid);
   const int col = tid & 31;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -394,51 +410,38 @@ __device__ inline void pred_stage_points(const PredictArgs& a, double* sXi, doub
 }
 
 template <int DT>
-__global__ __launch_bounds__(TPB) void k_pred_cov(PredictArgs a) {
+__global__ __launch_bounds__(TPB, 2) void k_pred_cov(PredictArgs a) {
   int ti, tj;
   tri_decode(blockIdx.x, ti, tj);
   const int i0 = ti * NB, j0 = tj * NB;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wr = w >> 1, wc = w & 1;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = a.m, ld = a.groups * a.mpad;
-  __shared__ double sbuf[4 * KC * LDSS];
-  d4 acc[2][2];
-  acc_zero(acc);
-  tile_mainloop<false, false, true>(a.C, ld, i0, a.C, ld, j0, 0, a.npad, sbuf, acc, tid, lane, wr, wc);
-  double* sXi = sbuf;
-  double* sXj = sbuf + DT * NB;
+  __shared__ double sS[2 * NB * LDSS];
+  double v[16];
+  tile64<true>(a.C, ld, j0, a.C, ld, i0, a.npad / 4, sS, v, tid);  // rows j, columns i
+  static_assert(2 * DMAX * NB <= 2 * NB * LDSS && NB * (NB + 1) <= 2 * NB * LDSS, "what follows in sS");
+  double* sXi = sS;
+  double* sXj = sS + DT * NB;
+  __syncthreads();  // every wave has read its sums
   pred_stage_points<DT>(a, sXi, sXj, NB, i0, j0, tid);
   __syncthreads();
+  const int gi = i0 + lane;
 #pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int r = acc_row(lane, wr, bi), c = acc_col(lane, wc, bj, e);
-        const int gi = i0 + r, gj = j0 + c;
-        if (gi >= m || gj >= m) continue;
-        const double v = pred_sigma<DT>(a, acc[bi][bj][e], sXi, sXj, NB, r, c, gi, gj);
-        a.cov[(size_t)gj * m + gi] = v;
-        acc[bi][bj][e] = v;
-      }
+  for (int r = 0; r < 16; ++r) {
+    const int c = w + 4 * r, gj = j0 + c;
+    if (gi >= m || gj >= m) continue;
+    v[r] = pred_sigma<DT>(a, v[r], sXi, sXj, NB, lane, c, gi, gj);
+    a.cov[(size_t)gj * m + gi] = v[r];
+  }
   if (ti == tj) return;
-  // the transpose of an off-diagonal tile, staged through LDS so that its
-  // columns are stored with 64 consecutive lanes (coalesced)
-  static_assert(4 * KC * LDSS >= NB * (NB + 1), "a 64 x 65 tile fits the staging buffer");
-  double* sT = sbuf;
+  // the transpose of an off-diagonal tile, through LDS: stored in rows too
   __syncthreads();  // every wave is done with sXi / sXj
 #pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        sT[acc_row(lane, wr, bi) * (NB + 1) + acc_col(lane, wc, bj, e)] = acc[bi][bj][e];
+  for (int r = 0; r < 16; ++r) sS[lane * (NB + 1) + w + 4 * r] = v[r];
   __syncthreads();
-  const int gj = j0 + lane;
-  for (int r = w * (NB / 4); r < (w + 1) * (NB / 4); ++r) {
-    const int gi = i0 + r;
-    if (gi < m && gj < m) a.cov[(size_t)gi * m + gj] = sT[r * (NB + 1) + lane];
+  for (int r = 0; r < 16; ++r) {
+    const int row = w + 4 * r;
+    if (i0 + row < m && j0 + lane < m) a.cov[(size_t)(i0 + row) * m + j0 + lane] = sS[row * (NB + 1) + lane];
   }
 }
 
