@@ -297,13 +297,11 @@ struct NkArgs {
 };
 hipError_t launch_nk_prepare(const NkArgs& a, hipStream_t stream);  // C, U, M, Kd, R_g^-1 k_g
 constexpr int NK_QT = 512;         // points per workgroup of the pair kernel at its widest
-// up to here its form for few points: a whole prediction at 30 points takes
-// 0.80 .. 1.0 times the wide form's time (n = 900 .. 20000), at 60 points 1.03
-// .. 1.15 times
+// up to here its form for few points: a whole prediction at 32 points takes
+// 0.74 .. 0.96 times the wide form's time (n = 900 .. 20000)
 constexpr int NK_FEW = 32;
-constexpr int NK_WGS = 2048;       // workgroups to aim at, many points
-constexpr int NK_WGS_FEW = 3072;   // and few
-int nk_pair_slices(int npairs, int qc, int max_tiles);
+constexpr int NK_WGS = 2048;       // workgroups to aim at
+int nk_pair_slices(int npairs, int max_tiles);
 hipError_t launch_nk_pairs(const NkArgs& a, hipStream_t stream);    // off-diagonal KM
 hipError_t launch_nk_solve(const NkArgs& a, hipStream_t stream);    // per-point aggregation
 hipError_t launch_nk_alpha(const NkArgs& a, const double* r, hipStream_t stream);  // alpha = Linv' r

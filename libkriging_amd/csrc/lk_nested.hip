@@ -409,106 +409,121 @@ __global__ __launch_bounds__(512, 2) void k_nk_pair(NkArgs a, int tbase) {
 
 // (6b) few points (<= 32): a value of R serves so few points that the time is
 // its generation, so each wave generates its own operands in the MFMA's
-// register layout (lane = row r16, column kq), four independent values at a
-// time, with no LDS and no barrier; the four waves take the rows b in
-// turn and their parts are added at the end.  A whole prediction, n = 20000
-// in 32 groups: 0.80 ms at 16 points against 1.03 through (6a) and 2.06 when
-// every call was padded to 128 points.  grid (npairs, slices)
+// register layout (lane = row a r16, row b kq), four independent values a lane
+// at a time.  The four waves take 16 of the 64 rows a each; group j's
+// coordinates are in LDS, FB rows at a time, so that the loop has no barrier.
+// A tile's products meet in LDS, where one wave per 16 points weights and adds
+// them in (6a)'s order: the same sums, bit for bit.  A whole prediction, n =
+// 20000 in 32 groups: 0.61 ms at 16 points, 0.87 through (6a); n = 3000 in 6
+// groups 131 us and 145.  (The rows b over the waves, whose sums are not
+// (6a)'s: 0.65 ms and 128 us.  The coordinates from memory, four times the
+// loads of that: 1.08 ms.  The values through LDS, a barrier per chunk: 0.66.)
+// grid (npairs, slices)
 template <int DT, int KT, int NBJ>
-__global__ __launch_bounds__(TPB, 2) void k_nk_pair_few(NkArgs a, int tbase) {
+__global__ __launch_bounds__(TPB, 3) void k_nk_pair_few(NkArgs a, int tbase) {
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, kq = lane >> 4;
   const int2 pr = a.pairs[blockIdx.x];
   const NkGroup Gi = a.groups[pr.x], Gj = a.groups[pr.y];
   const int d = a.d, ld = a.qpad;
-  const int nti = Gi.npad / NB;
+  const int nti = Gi.npad / NB, nb = (Gj.n + NK_PKC - 1) / NK_PKC * NK_PKC;
   const int tile0 = nti * (int)blockIdx.y / a.nslice, tile1 = nti * ((int)blockIdx.y + 1) / a.nslice;
-  // K-steps of 4 rows b: wave w's are s0 .. s1 - 1 (rows beyond n: W_j = 0)
-  const int nst = (Gj.n + 3) / 4, s0 = nst * w / 4, s1 = nst * (w + 1) / 4;
+  constexpr int FB = DT > NK_DR ? NB : 256;  // rows b in LDS
+  constexpr int DX = DT > NK_DR ? 1 : DT;
+  __shared__ double sB[FB * DT];  // row b: its coordinates
   __shared__ double sX[DT > NK_DR ? DT * NB : 1];
-  __shared__ double red[4][16 * NBJ];
-  double part[NBJ];
-#pragma unroll
-  for (int bj = 0; bj < NBJ; ++bj) part[bj] = 0.0;
+  __shared__ d4 sAcc[4][NBJ][64];
   const unsigned lo = 8u * (kq * ld + r16);  // row kq, point r16
   const double* Wj = a.C + (size_t)Gj.off * ld + tbase;
-  const double* Xb = a.Xg + Gj.off;
+  double part = 0.0;
+  int have = -1;  // first of the rows in sB
   for (int tile = tile0; tile < tile1; ++tile) {
     const double* X = a.Xg + Gi.off + tile * NB;
-    if constexpr (DT > NK_DR) {
+    double xa[DX];
+    if constexpr (DT <= NK_DR) {
+#pragma unroll
+      for (int k = 0; k < DT; ++k) xa[k] = nk_load(X + (size_t)min(k, d - 1) * a.Npad + 16 * w, 8u * r16);
+    } else {
       __syncthreads();
       for (int q = tid; q < d * NB; q += TPB) sX[q] = X[(size_t)(q / NB) * a.Npad + q % NB];
       __syncthreads();
     }
-    double xa[DT > NK_DR ? 1 : DT][4];
-    if constexpr (DT <= NK_DR) {
+    d4 acc[NBJ];
 #pragma unroll
-      for (int k = 0; k < DT; ++k)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          xa[k][q] = nk_load(X + (size_t)min(k, d - 1) * a.Npad + 16 * q, 8u * r16);
-    }
-    d4 acc[4][NBJ];
-#pragma unroll
-    for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-      for (int bj = 0; bj < NBJ; ++bj) acc[bi][bj] = d4{0.0, 0.0, 0.0, 0.0};
-    double xb[DT > NK_DR ? 1 : DT], bv[NBJ];
-    auto load_step = [&](int s) __attribute__((always_inline)) {
-      if constexpr (DT <= NK_DR) {
-#pragma unroll
-        for (int k = 0; k < DT; ++k) xb[k] = nk_load(Xb + (size_t)min(k, d - 1) * a.Npad + 4 * s, 8u * kq);
+    for (int bj = 0; bj < NBJ; ++bj) acc[bj] = d4{0.0, 0.0, 0.0, 0.0};
+    for (int s0 = 0; s0 < nb; s0 += FB) {
+      if (have != s0) {
+        __syncthreads();  // every wave is done with the rows before
+        for (int q = tid; q < DT * FB; q += TPB) {
+          const int k = q / FB, b = q % FB;
+          if (k < d && s0 + b < Gj.npad) sB[b * DT + k] = a.Xg[(size_t)k * a.Npad + Gj.off + s0 + b];
+        }
+        have = s0;
+        __syncthreads();
       }
+      const int cend = min(FB, nb - s0);
+      double x[DX][4];
+      auto load_x = [&](int b) __attribute__((always_inline)) {
+        if constexpr (DT <= NK_DR) {
 #pragma unroll
-      for (int bj = 0; bj < NBJ; ++bj) bv[bj] = nk_load(Wj + (size_t)(4 * s) * ld + 16 * bj, lo);
-    };
-    if (s0 < s1) load_step(s0);
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int k = 0; k < DT; ++k) x[k][q] = sB[(b + 4 * q + kq) * DT + k];
+        }
+      };
+      load_x(0);
 #pragma unroll 1
-    for (int s = s0; s < s1; ++s) {
-      double av[4], b[NBJ], x[DT > NK_DR ? 1 : DT];
-      if constexpr (DT <= NK_DR) {
+      for (int b = 0; b < cend; b += NK_PKC) {
+        double av[4], bv[4][NBJ];
 #pragma unroll
-        for (int k = 0; k < DT; ++k) x[k] = xb[k];
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int bj = 0; bj < NBJ; ++bj) bv[s][bj] = nk_load(Wj + (size_t)(s0 + b + 4 * s) * ld + 16 * bj, lo);
+        __builtin_amdgcn_sched_barrier(0);  // they arrive while the values are made
+        nk_values<DT, KT, 4>(
+            d, a.itheta,
+            [&](int k, int q) {
+              if constexpr (DT > NK_DR)
+                return sB[(b + 4 * q + kq) * DT + k];
+              else
+                return x[k][q];
+            },
+            [&](int k) {
+              if constexpr (DT > NK_DR)
+                return sX[k * NB + 16 * w + r16];
+              else
+                return xa[k];
+            },
+            av);
+        load_x(min(b + NK_PKC, cend - NK_PKC));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int bj = 0; bj < NBJ; ++bj)
+            acc[bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s], bv[s][bj], acc[bj], 0, 0, 0);
       }
-#pragma unroll
-      for (int bj = 0; bj < NBJ; ++bj) b[bj] = bv[bj];
-      load_step(min(s + 1, s1 - 1));
-      __builtin_amdgcn_sched_barrier(0);  // the next step's loads fly during this one
-      if constexpr (DT > NK_DR)
-        nk_values<DT, KT, 4>(
-            d, a.itheta, [&](int k, int q) { return sX[k * NB + 16 * q + r16]; },
-            [&](int k) { return nk_load(Xb + (size_t)k * a.Npad + 4 * s, 8u * kq); }, av);
-      else
-        nk_values<DT, KT, 4>(
-            d, a.itheta, [&](int k, int q) { return xa[k][q]; }, [&](int k) { return x[k]; }, av);
-#pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < NBJ; ++bj)
-          acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[bi], b[bj], acc[bi][bj], 0, 0, 0);
     }
-    const double* Wi = a.C + ((size_t)Gi.off + nk_fresh(tile) * NB) * ld + tbase;
+    __syncthreads();  // the tile before has been added
 #pragma unroll
-    for (int bj = 0; bj < NBJ; ++bj) {
+    for (int bj = 0; bj < NBJ; ++bj) sAcc[w][bj][lane] = acc[bj];
+    __syncthreads();
+    if (w < NBJ) {
+      const double* Wi = a.C + ((size_t)Gi.off + nk_fresh(tile) * NB) * ld + tbase + 16 * w;
       double wv[16];
 #pragma unroll
-      for (int q = 0; q < 16; ++q) wv[q] = nk_load(Wi + (size_t)(4 * q) * ld + 16 * bj, lo);
+      for (int q = 0; q < 16; ++q) wv[q] = nk_load(Wi + (size_t)(4 * q) * ld, lo);
 #pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
+      for (int bi = 0; bi < 4; ++bi) {
+        const d4 s = sAcc[bi][w][lane];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) part[bj] = fma(acc[bi][bj][e], wv[4 * bi + e], part[bj]);
-      __builtin_amdgcn_sched_barrier(0);
+        for (int e = 0; e < 4; ++e) part = fma(s[e], wv[4 * bi + e], part);
+      }
     }
   }
-#pragma unroll
-  for (int bj = 0; bj < NBJ; ++bj) {
-    const double v = nk_fold(part[bj]);
-    if (kq == 0) red[w][16 * bj + r16] = v;
-  }
-  __syncthreads();
-  const int t = tbase + tid;
-  if (tid < 16 * NBJ && t < a.qc)
-    a.U[((size_t)blockIdx.y * a.npairs + blockIdx.x) * ld + t] = (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
+  const int t = tbase + 16 * w + r16;
+  const double v = nk_fold(part);
+  if (w < NBJ && kq == 0 && t < a.qc) a.U[((size_t)blockIdx.y * a.npairs + blockIdx.x) * ld + t] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -726,16 +741,16 @@ hipError_t launch_nk_prepare(const NkArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Slices of group i's row tiles, so that few pairs still cover the chip and
-// the last workgroups are a small part of the time.  Aims, measured at 496
-// pairs and 500 points: 2048 workgroups of 512 threads, one per CU at a time
-// (pair kernel 3.77 ms; 3.82 for 1024, 4.02 for 4096, where the start of
-// each shows); 3072 of the short 256-thread ones
-int nk_pair_slices(int npairs, int qc, int max_tiles) {
+// Slices of group i's row tiles, so that few pairs still cover the chip.  A
+// point's sum is that of its slices in order, so their number depends on the
+// pairs alone and never on the points: NK_WGS workgroups where 512 points or
+// fewer are one launch of it (pair kernel at 496 pairs and 500 points 3.77 ms;
+// 3.82 for 1024, 4.02 for 4096, where the start of each workgroup shows); with
+// more points fewer, longer workgroups gained nothing (1000 points 7.96 ms a
+// prediction against 8.29, 8192 points 61.7 against 61.4)
+int nk_pair_slices(int npairs, int max_tiles) {
   if (npairs <= 0) return 1;
-  const int have = qc <= NK_FEW ? npairs : npairs * ((qc + NK_QT - 1) / NK_QT);
-  const int want = qc <= NK_FEW ? NK_WGS_FEW : NK_WGS;
-  return std::max(1, std::min(max_tiles, (want + have - 1) / have));
+  return std::max(1, std::min(max_tiles, (NK_WGS + npairs - 1) / npairs));
 }
 
 hipError_t launch_nk_pairs(const NkArgs& args, hipStream_t stream) {

@@ -543,11 +543,11 @@ void NestedKriging::predict_poe(const double* Xn, int m, bool want_stdev, double
 void NestedKriging::predict_nk(const double* Xn, int m, bool want_stdev, double* mean, double* stdev) {
   const int p = (int)groups_.size(), d = d_;
   hip_check(hipSetDevice(device_), "hipSetDevice");
-  // U's rows also hold the pairs' sums, nslice per pair (at most as many as
-  // the smallest chunk is cut into)
+  // U's rows also hold the pairs' sums, nslice per pair
   int max_tiles = 1;
   for (int np : gpad_) max_tiles = std::max(max_tiles, np / NB);
-  const size_t u_rows = std::max((size_t)Npad_, (size_t)nk_pair_slices(npairs_, 1, max_tiles) * npairs_);
+  const int nslice = nk_pair_slices(npairs_, max_tiles);
+  const size_t u_rows = std::max((size_t)Npad_, (size_t)nslice * npairs_);
   // chunk: explicit, else as many points as fit in ~8 GiB of workspace
   int qc = chunk_;
   if (qc <= 0) {
@@ -615,7 +615,7 @@ void NestedKriging::predict_nk(const double* Xn, int m, bool want_stdev, double*
       a.p = p;
       a.qc = mc;
       a.qpad = (mc + NB - 1) / NB * NB;
-      a.nslice = nk_pair_slices(npairs_, mc, max_tiles);
+      a.nslice = nslice;
       a.kernel = kernel_id(kernel_);
       a.npairs = npairs_;
       hip_check(launch_nk_prepare(a, st), "nk prepare");
