@@ -86,3 +86,12 @@ def test_condition_estimate_at_any_scale(emu, make, exponent):
     for k in range(n // 64):
         b = slice(64 * k, 64 * k + 64)
         assert cond[k] == 64 * np.max(np.abs(L[b, b])) * np.max(np.abs(W[b, b]))
+
+
+@pytest.mark.parametrize("make", [spd, graded])
+def test_rows_of_16_and_of_64(emu, make):
+    # two block columns per square and three row blocks below the first
+    A = make(320)
+    ref = emu(A)
+    assert ref[3] == 0
+    assert same(emu(A, FORWARD[::-1], lanes_reversed=True, rb4=True), ref)
