@@ -220,7 +220,13 @@ int lk_kriging_fit_parameters(void* ptr, const double* y, int n, const double* X
                               int is_nugget_estim);
 /* libkriging_c.h:60-71 (Kriging::predict, Kriging.cpp:2241-2285): mean,
  * stdev, the m x m covariance (at most 32768 points per call) and the
- * m x d derivatives of mean and stdev, column-major */
+ * m x d derivatives of mean and stdev, column-major.  A point's results are
+ * the same, bit for bit, whatever other points the call has.  Predictions
+ * (and lk_nested_kriging_predict's) work in device memory that the device's
+ * runtime keeps for the next ones: at most 2 GiB, and 64 MiB pinned on the
+ * host, until the last model is deleted or an allocation of this library
+ * needs it; another user of the device in the process does not get it back
+ * before. */
 int lk_kriging_predict(void* ptr, const double* X_n, int m, int d, int return_stdev, int return_cov, int return_deriv,
                        double* mean_out, double* stdev_out, double* cov_out, double* mean_deriv_out,
                        double* stdev_deriv_out);
@@ -394,7 +400,8 @@ double lk_nested_kriging_get_beta0(void* ptr);
  * lk_nested_kriging_submodel returns a borrowed lk_kriging_* handle of
  * submodel i (valid until the next fit or delete; never delete it);
  * lk_nested_kriging_set_predict_chunk is NestedKriging::set_predict_chunk
- * (0 = sized from a device-memory budget); lk_nested_kriging_predict_fallbacks
+ * (0 = sized from a device-memory budget; the NK values do not depend on it,
+ * nor on the other points of the call); lk_nested_kriging_predict_fallbacks
  * counts the points of the last NK predict whose aggregation system was not
  * positive definite (solved by LU, or by the pseudo-inverse when singular). */
 void* lk_nested_kriging_new(const char* kernel, const char* aggregation, const char* partition, int seed);

@@ -981,78 +981,76 @@ void Kriging::predict(const double* Xn, int m, bool want_stdev, double* mean, do
   double* const xn = up + ncoef;
   for (int a = 0; a < p; ++a) up[a] = beta_[a];
   for (int q = 0; q < p * p; ++q) up[p + q] = Rstar_[q];
-  {
-    const bool nug = noise_ == NoiseModel::Nugget;
-    const double var_scale = nug ? sigma2_ / alpha_ : sigma2_;
-    const double vs = var_scale * scaleY_ * scaleY_;
-    const double* const hdm = host_out + 2 * (size_t)chunk;
-    const double* const hdv = hdm + nder;
-    for (int s0 = 0; s0 < m; s0 += chunk) {
-      const int mc = std::min(chunk, m - s0);
-      for (int k = 0; k < d; ++k)
-        for (int j = 0; j < mc; ++j) xn[j + (size_t)k * mc] = (Xn[s0 + j + (size_t)k * m] - centerX_[k]) / scaleX_[k];
-      hip_check(hipMemcpyAsync(dup, up, sizeof(double) * (ncoef + (size_t)mc * d), hipMemcpyHostToDevice,
+  const bool nug = noise_ == NoiseModel::Nugget;
+  const double var_scale = nug ? sigma2_ / alpha_ : sigma2_;
+  const double vs = var_scale * scaleY_ * scaleY_;
+  const double* const hdm = host_out + 2 * (size_t)chunk;
+  const double* const hdv = hdm + nder;
+  for (int s0 = 0; s0 < m; s0 += chunk) {
+    const int mc = std::min(chunk, m - s0);
+    for (int k = 0; k < d; ++k)
+      for (int j = 0; j < mc; ++j) xn[j + (size_t)k * mc] = (Xn[s0 + j + (size_t)k * m] - centerX_[k]) / scaleX_[k];
+    hip_check(hipMemcpyAsync(dup, up, sizeof(double) * (ncoef + (size_t)mc * d), hipMemcpyHostToDevice,
+                             rt_->stream()),
+              "upload Xn");
+    PredictArgs a{};
+    a.X = rt_->problem(problem_).X;
+    a.Linv = d_Linv_;
+    a.MZ = d_vec_;
+    a.coef = dup;
+    a.Xn = dup + ncoef;
+    a.Ron = dRon;
+    a.C = dC;
+    a.out = dout;
+    a.ecirc = dEc;
+    a.cov = dCov;
+    a.nn_factor = nug ? alpha_ : 1.0;
+    a.dmean = dout + 2 * (size_t)chunk;
+    a.dvar = a.dmean + nder;
+    for (int k = 0; k < DMAX; ++k) a.itheta[k] = (k < d) ? 1.0 / theta_[k] : 1.0;
+    a.factor = nug ? alpha_ : 1.0;
+    a.n = n_;
+    a.d = d;
+    a.npad = npad_;
+    a.p = p;
+    a.m = mc;
+    a.mpad = (mc + NB - 1) / NB * NB;
+    a.groups = groups;
+    a.kernel = kernel_id(kernel_);
+    a.linear_trend = regmodel_ == RegModel::Linear;
+    a.want_var = want_stdev ? 1 : 0;
+    hip_check(launch_predict(a, rt_->stream()), "predict");
+    if (want_deriv) hip_check(launch_predict_deriv(a, rt_->stream()), "predict deriv");
+    if (want_cov) hip_check(launch_predict_cov(a, rt_->stream()), "predict cov");
+    // the variances' derivatives, last, only when they were asked for
+    const size_t nd = !want_deriv ? 2 * (size_t)mc : ndown - (want_stdev ? 0 : nder);
+    hip_check(hipMemcpyAsync(host_out, dout, sizeof(double) * nd, hipMemcpyDeviceToHost, rt_->stream()), "download");
+    if (want_cov && cov != nullptr)
+      hip_check(hipMemcpyAsync(stage_cov ? hcov : cov, dCov, sizeof(double) * ncov, hipMemcpyDeviceToHost,
                                rt_->stream()),
-                "upload Xn");
-      PredictArgs a{};
-      a.X = rt_->problem(problem_).X;
-      a.Linv = d_Linv_;
-      a.MZ = d_vec_;
-      a.coef = dup;
-      a.Xn = dup + ncoef;
-      a.Ron = dRon;
-      a.C = dC;
-      a.out = dout;
-      a.ecirc = dEc;
-      a.cov = dCov;
-      a.nn_factor = nug ? alpha_ : 1.0;
-      a.dmean = dout + 2 * (size_t)chunk;
-      a.dvar = a.dmean + nder;
-      for (int k = 0; k < DMAX; ++k) a.itheta[k] = (k < d) ? 1.0 / theta_[k] : 1.0;
-      a.factor = nug ? alpha_ : 1.0;
-      a.n = n_;
-      a.d = d;
-      a.npad = npad_;
-      a.p = p;
-      a.m = mc;
-      a.mpad = (mc + NB - 1) / NB * NB;
-      a.groups = groups;
-      a.kernel = kernel_id(kernel_);
-      a.linear_trend = regmodel_ == RegModel::Linear;
-      a.want_var = want_stdev ? 1 : 0;
-      hip_check(launch_predict(a, rt_->stream()), "predict");
-      if (want_deriv) hip_check(launch_predict_deriv(a, rt_->stream()), "predict deriv");
-      if (want_cov) hip_check(launch_predict_cov(a, rt_->stream()), "predict cov");
-      // the variances' derivatives, last, only when they were asked for
-      const size_t nd = !want_deriv ? 2 * (size_t)mc : ndown - (want_stdev ? 0 : nder);
-      hip_check(hipMemcpyAsync(host_out, dout, sizeof(double) * nd, hipMemcpyDeviceToHost, rt_->stream()), "download");
-      if (want_cov && cov != nullptr)
-        hip_check(hipMemcpyAsync(stage_cov ? hcov : cov, dCov, sizeof(double) * ncov, hipMemcpyDeviceToHost,
-                                 rt_->stream()),
-                  "download");
-      hip_check(hipStreamSynchronize(rt_->stream()), "sync");
-      for (int j = 0; j < mc; ++j) {
-        mean[s0 + j] = centerY_ + scaleY_ * host_out[j];
-        if (want_stdev && stdev != nullptr) stdev[s0 + j] = std::sqrt(host_out[mc + j] * vs);
-      }
-      if (want_deriv) {
-        // chain rule of the normalisation (KrigingImpl.cpp:289-293), then
-        // d stdev = d var / (2 stdev)
-        for (int k = 0; k < d; ++k)
-          for (int j = 0; j < mc; ++j) {
-            if (mean_deriv != nullptr) mean_deriv[s0 + j + (size_t)k * m] = hdm[j + (size_t)k * mc] * scaleY_ / scaleX_[k];
-            if (stdev_deriv != nullptr) {
-              const double sd = std::sqrt(host_out[mc + j] * vs);
-              const double dv = want_stdev ? hdv[j + (size_t)k * mc] * vs / scaleX_[k] : 0.0;
-              stdev_deriv[s0 + j + (size_t)k * m] = dv / (2.0 * (want_stdev ? sd : 0.0));
-            }
+                "download");
+    hip_check(hipStreamSynchronize(rt_->stream()), "sync");
+    for (int j = 0; j < mc; ++j) {
+      mean[s0 + j] = centerY_ + scaleY_ * host_out[j];
+      if (want_stdev && stdev != nullptr) stdev[s0 + j] = std::sqrt(host_out[mc + j] * vs);
+    }
+    if (want_deriv) {
+      // chain rule of the normalisation (KrigingImpl.cpp:289-293), then
+      // d stdev = d var / (2 stdev)
+      for (int k = 0; k < d; ++k)
+        for (int j = 0; j < mc; ++j) {
+          if (mean_deriv != nullptr) mean_deriv[s0 + j + (size_t)k * m] = hdm[j + (size_t)k * mc] * scaleY_ / scaleX_[k];
+          if (stdev_deriv != nullptr) {
+            const double sd = std::sqrt(host_out[mc + j] * vs);
+            const double dv = want_stdev ? hdv[j + (size_t)k * mc] * vs / scaleX_[k] : 0.0;
+            stdev_deriv[s0 + j + (size_t)k * m] = dv / (2.0 * (want_stdev ? sd : 0.0));
           }
-      }
+        }
     }
-    if (want_cov && cov != nullptr) {
-      const double* c = stage_cov ? hcov : cov;
-      for (size_t q = 0; q < ncov; ++q) cov[q] = c[q] * vs;
-    }
+  }
+  if (want_cov && cov != nullptr) {
+    const double* c = stage_cov ? hcov : cov;
+    for (size_t q = 0; q < ncov; ++q) cov[q] = c[q] * vs;
   }
   lease.finished();
 }

@@ -582,80 +582,78 @@ void NestedKriging::predict_nk(const double* Xn, int m, bool want_stdev, double*
   double* const xc = reinterpret_cast<double*>(lease.pin());
   double* const hout = xc + (size_t)qc * d;
   const int* const hinfo = reinterpret_cast<const int*>(hout + 2 * (size_t)qc);
-  {
-    hipStream_t st = rt_->stream();
-    for (int s0 = 0; s0 < m; s0 += qc) {
-      const int mc = std::min(qc, m - s0);
-      for (int k = 0; k < d; ++k)
-        for (int t = 0; t < mc; ++t) xc[t + (size_t)k * mc] = Xn[s0 + t + (size_t)k * m];
-      hip_check(hipMemcpyAsync(dXc, xc, sizeof(double) * (size_t)mc * d, hipMemcpyHostToDevice, st), "upload");
-      NkArgs a{};
-      a.Xg = d_Xg_;
-      a.Linv = d_Linv_;
-      a.alpha = d_alpha_;
-      a.groups = (const NkGroup*)d_groups_;
-      a.tile_group = d_tile_group_;
-      a.pairs = (const int2*)d_pairs_;
-      a.Xc = dXc;
-      a.C = dC;
-      a.U = dU;
-      a.M = dM;
-      a.Kd = dKd;
-      a.KM = dKM;
-      a.KF = dKF;
-      a.out = dout;
-      a.info = dinfo;
-      for (int k = 0; k < d; ++k) a.theta[k] = theta_[k];
-      for (int k = 0; k < DMAX; ++k) a.itheta[k] = (k < d) ? 1.0 / theta_[k] : 1.0;
-      a.beta0 = beta0_;
-      a.sigma2 = sigma2_;
-      a.jitter = NK_JITTER;
-      a.Npad = Npad_;
-      a.d = d;
-      a.p = p;
-      a.qc = mc;
-      a.qpad = (mc + NB - 1) / NB * NB;
-      a.nslice = nslice;
-      a.kernel = kernel_id(kernel_);
-      a.npairs = npairs_;
-      hip_check(launch_nk_prepare(a, st), "nk prepare");
-      if (time_pairs_) hip_check(hipEventRecord(pev_[0], st), "event record");
-      hip_check(launch_nk_pairs(a, st), "nk pairs");
-      if (time_pairs_) hip_check(hipEventRecord(pev_[1], st), "event record");
-      hip_check(launch_nk_solve(a, st), "nk solve");
-      hip_check(hipMemcpyAsync(hout, dout, down_bytes, hipMemcpyDeviceToHost, st), "download");
-      hip_check(hipStreamSynchronize(st), "sync");
-      if (time_pairs_) {
-        float ms = 0.f;
-        hip_check(hipEventElapsedTime(&ms, pev_[0], pev_[1]), "event elapsed");
-        pair_ms_ += ms;
-        pair_points_ += mc;
-        ++pair_launches_;
-      }
-      for (int t = 0; t < mc; ++t) {
-        double mu = hout[t], var = hout[mc + t];
-        if (hinfo[t] != 0) ++fallbacks_;
-        if (hinfo[t] == 2) {
-          // singular KM: w = pinv(KM) kM (NestedKriging.cpp:457-458)
-          std::vector<double> K(pp), kM(p), Mv(p);
-          hip_check(hipMemcpy(K.data(), dKM + (size_t)t * pp, sizeof(double) * pp, hipMemcpyDeviceToHost), "download");
-          hip_check(hipMemcpy(Mv.data(), dM + (size_t)t * p, sizeof(double) * p, hipMemcpyDeviceToHost), "download");
-          for (int i = 0; i < p; ++i) {
-            for (int j = 0; j < i; ++j) K[(size_t)j * p + i] = K[(size_t)i * p + j];  // symmatu
-            kM[i] = K[(size_t)i * p + i];
-          }
-          const std::vector<double> w = sym_pinv_solve(K, kM, p);
-          double sm = 0.0, sv = 0.0;
-          for (int i = 0; i < p; ++i) {
-            sm += w[i] * (Mv[i] - beta0_);
-            sv += w[i] * kM[i];
-          }
-          mu = beta0_ + sm;
-          var = sigma2_ * std::max(0.0, 1.0 - sv);
+  hipStream_t st = rt_->stream();
+  for (int s0 = 0; s0 < m; s0 += qc) {
+    const int mc = std::min(qc, m - s0);
+    for (int k = 0; k < d; ++k)
+      for (int t = 0; t < mc; ++t) xc[t + (size_t)k * mc] = Xn[s0 + t + (size_t)k * m];
+    hip_check(hipMemcpyAsync(dXc, xc, sizeof(double) * (size_t)mc * d, hipMemcpyHostToDevice, st), "upload");
+    NkArgs a{};
+    a.Xg = d_Xg_;
+    a.Linv = d_Linv_;
+    a.alpha = d_alpha_;
+    a.groups = (const NkGroup*)d_groups_;
+    a.tile_group = d_tile_group_;
+    a.pairs = (const int2*)d_pairs_;
+    a.Xc = dXc;
+    a.C = dC;
+    a.U = dU;
+    a.M = dM;
+    a.Kd = dKd;
+    a.KM = dKM;
+    a.KF = dKF;
+    a.out = dout;
+    a.info = dinfo;
+    for (int k = 0; k < d; ++k) a.theta[k] = theta_[k];
+    for (int k = 0; k < DMAX; ++k) a.itheta[k] = (k < d) ? 1.0 / theta_[k] : 1.0;
+    a.beta0 = beta0_;
+    a.sigma2 = sigma2_;
+    a.jitter = NK_JITTER;
+    a.Npad = Npad_;
+    a.d = d;
+    a.p = p;
+    a.qc = mc;
+    a.qpad = (mc + NB - 1) / NB * NB;
+    a.nslice = nslice;
+    a.kernel = kernel_id(kernel_);
+    a.npairs = npairs_;
+    hip_check(launch_nk_prepare(a, st), "nk prepare");
+    if (time_pairs_) hip_check(hipEventRecord(pev_[0], st), "event record");
+    hip_check(launch_nk_pairs(a, st), "nk pairs");
+    if (time_pairs_) hip_check(hipEventRecord(pev_[1], st), "event record");
+    hip_check(launch_nk_solve(a, st), "nk solve");
+    hip_check(hipMemcpyAsync(hout, dout, down_bytes, hipMemcpyDeviceToHost, st), "download");
+    hip_check(hipStreamSynchronize(st), "sync");
+    if (time_pairs_) {
+      float ms = 0.f;
+      hip_check(hipEventElapsedTime(&ms, pev_[0], pev_[1]), "event elapsed");
+      pair_ms_ += ms;
+      pair_points_ += mc;
+      ++pair_launches_;
+    }
+    for (int t = 0; t < mc; ++t) {
+      double mu = hout[t], var = hout[mc + t];
+      if (hinfo[t] != 0) ++fallbacks_;
+      if (hinfo[t] == 2) {
+        // singular KM: w = pinv(KM) kM (NestedKriging.cpp:457-458)
+        std::vector<double> K(pp), kM(p), Mv(p);
+        hip_check(hipMemcpy(K.data(), dKM + (size_t)t * pp, sizeof(double) * pp, hipMemcpyDeviceToHost), "download");
+        hip_check(hipMemcpy(Mv.data(), dM + (size_t)t * p, sizeof(double) * p, hipMemcpyDeviceToHost), "download");
+        for (int i = 0; i < p; ++i) {
+          for (int j = 0; j < i; ++j) K[(size_t)j * p + i] = K[(size_t)i * p + j];  // symmatu
+          kM[i] = K[(size_t)i * p + i];
         }
-        mean[s0 + t] = mu;
-        if (want_stdev && stdev != nullptr) stdev[s0 + t] = std::sqrt(var);
+        const std::vector<double> w = sym_pinv_solve(K, kM, p);
+        double sm = 0.0, sv = 0.0;
+        for (int i = 0; i < p; ++i) {
+          sm += w[i] * (Mv[i] - beta0_);
+          sv += w[i] * kM[i];
+        }
+        mu = beta0_ + sm;
+        var = sigma2_ * std::max(0.0, 1.0 - sv);
       }
+      mean[s0 + t] = mu;
+      if (want_stdev && stdev != nullptr) stdev[s0 + t] = std::sqrt(var);
     }
   }
   lease.finished();
