@@ -20,22 +20,36 @@ __global__ __launch_bounds__(TPB) void k_copy(const double2* __restrict__ src, d
   for (size_t i = blockIdx.x * (size_t)TPB + threadIdx.x; i < n; i += (size_t)gridDim.x * TPB) dst[i] = src[i];
 }
 
-// Every wave runs `iters` rounds of CH independent V_MFMA_F64_16X16X4_F64
-// accumulation chains on register operands (no memory traffic in the loop);
-// each thread stores one sum so the chains stay live.  Thread 0 of each
-// workgroup records the shader-clock and constant-rate counters around the
-// loop: stamps[4 b ..] = clock start, clock end, wall start, wall end.
+// Every wave runs `iters` rounds (a multiple of 4) of CH independent
+// V_MFMA_F64_16X16X4_F64 accumulation chains on register operands from `in`
+// (8 TPB values; no memory traffic in the loop); each thread stores one sum so
+// the chains stay live.  Thread 0 of each workgroup records the shader-clock
+// and constant-rate counters around the loop: stamps[4 b ..] = clock start,
+// clock end, wall start, wall end.  Four waves per SIMD asked for: with one,
+// the compiler keeps the accumulators in the other register file and moves
+// them there and back around every instruction, and those moves bound the loop
+// (49 TFLOP/s).
 template <int CH>
-__global__ __launch_bounds__(TPB) void k_mfma_probe(int iters, double* __restrict__ out,
-                                                    unsigned long long* __restrict__ stamps) {
-  const unsigned long long c0 = clock64(), w0 = wall_clock64();
+__global__ __launch_bounds__(TPB, 4) void k_mfma_probe(const double* __restrict__ in, int iters,
+                                                       double* __restrict__ out,
+                                                       unsigned long long* __restrict__ stamps) {
   d4 acc[CH];
 #pragma unroll
   for (int c = 0; c < CH; ++c) acc[c] = d4{0.0, 0.0, 0.0, 0.0};
-  const double a = 1.0 + 1e-12 * threadIdx.x, b = 1.0 - 1e-12 * threadIdx.x;
-  for (int it = 0; it < iters; ++it) {
+  double a[4], b[4];
 #pragma unroll
-    for (int c = 0; c < CH; ++c) acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[c], 0, 0, 0);
+  for (int i = 0; i < 4; ++i) {
+    a[i] = in[threadIdx.x + TPB * i];
+    b[i] = in[threadIdx.x + TPB * (4 + i)];
+  }
+  const unsigned long long c0 = clock64(), w0 = wall_clock64();
+#pragma unroll 1
+  for (int it = 0; it < iters; it += 4) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+        acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[(c + i) & 3], b[i], acc[c], 0, 0, 0);
   }
   double s = 0.0;
 #pragma unroll
@@ -119,20 +133,31 @@ int lkprobe_device_copy(int device, size_t bytes, int reps, double* ms_out) {
 int lkprobe_mfma(int device, int blocks, int iters, int chains, double* ms_out, double* tflops_out,
                  double* clock_mhz_out) {
   return guarded([&] {
-    if (blocks <= 0 || iters <= 0 || !(chains == 1 || chains == 2 || chains == 4 || chains == 8))
-      throw std::invalid_argument("blocks, iters > 0 and chains in {1, 2, 4, 8}");
+    if (blocks <= 0 || iters <= 0 || iters % 4 != 0 || !(chains == 1 || chains == 2 || chains == 4 || chains == 8))
+      throw std::invalid_argument("blocks > 0, iters a positive multiple of 4 and chains in {1, 2, 4, 8}");
     check(hipSetDevice(device), "hipSetDevice");
     int wall_khz = 0;
     check(hipDeviceGetAttribute(&wall_khz, hipDeviceAttributeWallClockRate, device), "wall clock rate");
+    // operands with every bit in use, as in a product (on constants the clock
+    // is higher)
+    std::vector<double> operands(8 * TPB);
+    uint64_t x = 1;
+    for (double& v : operands) {
+      x = x * 6364136223846793005ull + 1442695040888963407ull;
+      v = (double)(int64_t)x * 0x1p-63;
+    }
+    DevBuf in(sizeof(double) * operands.size());
+    check(hipMemcpy(in.p, operands.data(), sizeof(double) * operands.size(), hipMemcpyHostToDevice), "upload");
     DevBuf out(sizeof(double) * (size_t)blocks * TPB), st(sizeof(unsigned long long) * 4 * (size_t)blocks);
     auto launch = [&] {
+      const double* i = (const double*)in.p;
       double* o = (double*)out.p;
       unsigned long long* s = (unsigned long long*)st.p;
       switch (chains) {
-        case 1: hipLaunchKernelGGL(k_mfma_probe<1>, dim3(blocks), dim3(TPB), 0, 0, iters, o, s); break;
-        case 2: hipLaunchKernelGGL(k_mfma_probe<2>, dim3(blocks), dim3(TPB), 0, 0, iters, o, s); break;
-        case 4: hipLaunchKernelGGL(k_mfma_probe<4>, dim3(blocks), dim3(TPB), 0, 0, iters, o, s); break;
-        default: hipLaunchKernelGGL(k_mfma_probe<8>, dim3(blocks), dim3(TPB), 0, 0, iters, o, s); break;
+        case 1: hipLaunchKernelGGL(k_mfma_probe<1>, dim3(blocks), dim3(TPB), 0, 0, i, iters, o, s); break;
+        case 2: hipLaunchKernelGGL(k_mfma_probe<2>, dim3(blocks), dim3(TPB), 0, 0, i, iters, o, s); break;
+        case 4: hipLaunchKernelGGL(k_mfma_probe<4>, dim3(blocks), dim3(TPB), 0, 0, i, iters, o, s); break;
+        default: hipLaunchKernelGGL(k_mfma_probe<8>, dim3(blocks), dim3(TPB), 0, 0, i, iters, o, s); break;
       }
       check(hipGetLastError(), "k_mfma_probe");
     };
