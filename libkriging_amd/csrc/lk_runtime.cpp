@@ -895,8 +895,7 @@ Batch Runtime::part_batch(const Part& q, hipStream_t s) const {
 }
 
 // launches of the S parts, interleaved, between a fork from and a join back
-// to the main stream (also valid inside a stream capture, which the other
-// streams then join)
+// to the main stream
 void Runtime::issue_split(const std::vector<Step>* parts, int S) {
   hip_check(hipEventRecord(fork_, stream_), "fork record");
   for (int q = 1; q < S; ++q) hip_check(hipStreamWaitEvent(xstream_[q - 1], fork_, 0), "fork wait");
@@ -909,6 +908,70 @@ void Runtime::issue_split(const std::vector<Step>* parts, int S) {
     hip_check(hipEventRecord(join_[q - 1], xstream_[q - 1]), "join record");
     hip_check(hipStreamWaitEvent(stream_, join_[q - 1], 0), "join wait");
   }
+}
+
+// The captured steps of one part: made on first use, then kept.  A graph holds
+// its launches' grids and the addresses of the tables they read; which design a
+// slot evaluates and where it works are in the tables.  So one graph serves
+// every batch that is cut alike: a program that goes from one design to another
+// of its size captures nothing again (n = 200: 90 us, 64 x n = 1024: 150 us).
+// `timed`: the steps between which the timing events are recorded.
+hipGraphExec_t Runtime::graph_for(const Part& q, const std::function<std::vector<Step>()>& make_steps, bool want_grad,
+                                  int objective, const std::pair<size_t, size_t>* timed) {
+  GraphKey key;
+  key.tables[0] = d_slots_;
+  key.tables[1] = d_params_;
+  key.tables[2] = d_out_;
+  key.tables[3] = h_params_;
+  key.tables[4] = h_out_;
+  key.objective = objective;
+  key.want_grad = want_grad;
+  key.timed_stage = timed != nullptr ? timed_stage_ : -1;
+  key.part = {q.first, q.count, q.nblk_max, q.dmax, q.panel_blocks, q.wide};
+  auto it = std::find_if(graphs_.begin(), graphs_.end(), [&](const GraphEntry& g) { return g.key == key; });
+  if (it != graphs_.end()) {
+    std::rotate(graphs_.begin(), it, it + 1);  // most recently used first
+    return graphs_.front().exec;
+  }
+  const std::vector<Step> steps = make_steps();
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec = nullptr;
+  if (timed == nullptr) {
+    graph = capture(steps, 0, steps.size());
+  } else {
+    // events captured from a stream are not timeable here, so the timed
+    // stage sits between explicit event-record nodes of a parent graph
+    // whose other nodes are the captured segments before and after it
+    hip_check(hipGraphCreate(&graph, 0), "graph create");
+    hipGraphNode_t prev = nullptr, node = nullptr;
+    auto add_child = [&](size_t a, size_t b) {
+      if (a >= b) return;
+      hipGraph_t child = capture(steps, a, b);
+      hip_check(hipGraphAddChildGraphNode(&node, graph, prev ? &prev : nullptr, prev ? 1 : 0, child),
+                "add child graph");
+      hip_check(hipGraphDestroy(child), "graph destroy");
+      prev = node;
+    };
+    auto add_event = [&](hipEvent_t e) {
+      hip_check(hipGraphAddEventRecordNode(&node, graph, prev ? &prev : nullptr, prev ? 1 : 0, e),
+                "add event node");
+      prev = node;
+    };
+    add_child(0, timed->first);
+    add_event(tev_[0]);
+    add_child(timed->first, timed->second);
+    add_event(tev_[1]);
+    add_child(timed->second, steps.size());
+  }
+  const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+  hipGraphDestroy(graph);
+  hip_check(ie, "graph instantiate");
+  while (graphs_.size() >= kMaxGraphs) {
+    hipGraphExecDestroy(graphs_.back().exec);
+    graphs_.pop_back();
+  }
+  graphs_.insert(graphs_.begin(), GraphEntry{key, exec});
+  return exec;
 }
 
 void Runtime::run_pipeline(bool want_grad, BenchMap* bench, int objective) {
@@ -926,12 +989,6 @@ void Runtime::run_pipeline(bool want_grad, BenchMap* bench, int objective) {
   const int S = (int)plan.size();
   const bool split = S > 1;
   last_parts_ = S;
-  std::vector<Step> part[kMaxStreams];
-  if (split) {
-    for (int q = 0; q < S; ++q)
-      part[q] = pipeline_steps(part_batch(plan[q], q == 0 ? stream_ : xstream_[q - 1]), want_grad, objective,
-                               plan[q].panel_blocks, plan[q].wide);
-  }
   if (bench != nullptr) {
     // uncaptured run with one event pair around the whole pipeline
     hipEvent_t e0, e1;
@@ -948,76 +1005,39 @@ void Runtime::run_pipeline(bool want_grad, BenchMap* bench, int objective) {
     hipEventDestroy(e1);
   } else if (use_graph && !noalloc_ && !la) {
     if (objective < 0 || objective >= OBJ_COUNT) throw std::invalid_argument("unknown objective");
-    // A graph holds its launches' grids and the addresses of the tables they
-    // read; which design a slot evaluates and where it works are in the
-    // tables.  So one graph serves every batch that is cut into the same
-    // parts: a program that goes from one design to another of its size
-    // captures nothing again (n = 200: 90 us, 64 x n = 1024: 150 us).
-    GraphKey key;
-    key.tables[0] = d_slots_;
-    key.tables[1] = d_params_;
-    key.tables[2] = d_out_;
-    key.tables[3] = h_params_;
-    key.tables[4] = h_out_;
-    key.objective = objective;
-    key.want_grad = want_grad;
-    key.timed_stage = timed ? timed_stage_ : -1;
-    for (const Part& q : plan)
-      for (int v : {q.first, q.count, q.nblk_max, q.dmax, q.panel_blocks, q.wide}) key.parts.push_back(v);
-    auto it = std::find_if(graphs_.begin(), graphs_.end(), [&](const GraphEntry& g) { return g.key == key; });
-    if (it != graphs_.end()) {
-      std::rotate(graphs_.begin(), it, it + 1);  // most recently used first
+    if (!split) {
+      hip_check(hipGraphLaunch(graph_for(plan[0], [&] { return steps; }, want_grad, objective, timed ? &rng : nullptr),
+                               stream_),
+                "graph launch");
     } else {
-      hipGraph_t graph = nullptr;
-      hipGraphExec_t exec = nullptr;
-      if (split) {
-        hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "begin capture");
-        try {
-          issue_split(part, S);
-        } catch (...) {
-          hipStreamEndCapture(stream_, &graph);
-          if (graph) hipGraphDestroy(graph);
-          throw;
-        }
-        hip_check(hipStreamEndCapture(stream_, &graph), "end capture");
-      } else if (!timed) {
-        graph = capture(steps, 0, steps.size());
-      } else {
-        // events captured from a stream are not timeable here, so the timed
-        // stage sits between explicit event-record nodes of a parent graph
-        // whose other nodes are the captured segments before and after it
-        hip_check(hipGraphCreate(&graph, 0), "graph create");
-        hipGraphNode_t prev = nullptr, node = nullptr;
-        auto add_child = [&](size_t a, size_t b) {
-          if (a >= b) return;
-          hipGraph_t child = capture(steps, a, b);
-          hip_check(hipGraphAddChildGraphNode(&node, graph, prev ? &prev : nullptr, prev ? 1 : 0, child),
-                    "add child graph");
-          hip_check(hipGraphDestroy(child), "graph destroy");
-          prev = node;
-        };
-        auto add_event = [&](hipEvent_t e) {
-          hip_check(hipGraphAddEventRecordNode(&node, graph, prev ? &prev : nullptr, prev ? 1 : 0, e),
-                    "add event node");
-          prev = node;
-        };
-        add_child(0, rng.first);
-        add_event(tev_[0]);
-        add_child(rng.first, rng.second);
-        add_event(tev_[1]);
-        add_child(rng.second, steps.size());
+      // a linear graph per part, launched on the context's own streams: the
+      // branches of one graph run on streams that the graph creates for
+      // itself, and of several such graphs every second one had its branch on
+      // the hardware queue of its launch stream (48 x n = 900 in two parts:
+      // 1.63 ms, 2.26 as a context's second shape)
+      hipGraphExec_t exec[kMaxStreams];
+      for (int q = 0; q < S; ++q)
+        exec[q] = graph_for(
+            plan[q],
+            [&] {
+              return pipeline_steps(part_batch(plan[q], stream_), want_grad, objective, plan[q].panel_blocks,
+                                    plan[q].wide);
+            },
+            want_grad, objective, nullptr);
+      hip_check(hipEventRecord(fork_, stream_), "fork record");
+      for (int q = S - 1; q >= 0; --q) {  // the largest matrices first
+        const hipStream_t st = q == 0 ? stream_ : xstream_[q - 1];
+        if (q > 0) hip_check(hipStreamWaitEvent(st, fork_, 0), "fork wait");
+        hip_check(hipGraphLaunch(exec[q], st), "graph launch");
+        if (q > 0) hip_check(hipEventRecord(join_[q - 1], st), "join record");
       }
-      const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-      hipGraphDestroy(graph);
-      hip_check(ie, "graph instantiate");
-      while (graphs_.size() >= kMaxGraphs) {
-        hipGraphExecDestroy(graphs_.back().exec);
-        graphs_.pop_back();
-      }
-      graphs_.insert(graphs_.begin(), GraphEntry{key, exec});
+      for (int q = 1; q < S; ++q) hip_check(hipStreamWaitEvent(stream_, join_[q - 1], 0), "join wait");
     }
-    hip_check(hipGraphLaunch(graphs_.front().exec, stream_), "graph launch");
   } else if (split) {
+    std::vector<Step> part[kMaxStreams];
+    for (int q = 0; q < S; ++q)
+      part[q] = pipeline_steps(part_batch(plan[q], q == 0 ? stream_ : xstream_[q - 1]), want_grad, objective,
+                               plan[q].panel_blocks, plan[q].wide);
     issue_split(part, S);
   } else {
     run_steps(steps, 0, rng.first);

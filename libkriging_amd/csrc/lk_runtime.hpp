@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cstdint>
 #include <functional>
 #include <map>
@@ -307,10 +308,10 @@ class Runtime {
   // captured pipelines, most recently used first (at most kMaxGraphs)
   struct GraphKey {
     const void* tables[5] = {};  // slot, parameter and result tables, device and pinned
-    std::vector<int> parts;      // the parts' slot ranges, extents and launch parameters
+    std::array<int, 6> part{};   // its slot range, extents and launch parameters
     int objective = 0, want_grad = 0, timed_stage = -1;
     bool operator==(const GraphKey& o) const {
-      return std::equal(tables, tables + 5, o.tables) && parts == o.parts && objective == o.objective &&
+      return std::equal(tables, tables + 5, o.tables) && part == o.part && objective == o.objective &&
              want_grad == o.want_grad && timed_stage == o.timed_stage;
     }
   };
@@ -318,8 +319,10 @@ class Runtime {
     GraphKey key;
     hipGraphExec_t exec = nullptr;
   };
-  static constexpr size_t kMaxGraphs = 16;
+  static constexpr size_t kMaxGraphs = 32;
   std::vector<GraphEntry> graphs_;
+  hipGraphExec_t graph_for(const Part& q, const std::function<std::vector<Step>()>& make_steps, bool want_grad,
+                           int objective, const std::pair<size_t, size_t>* timed);
   void drop_graphs();
   void free_tables();
   int last_objective_ = OBJ_LL;

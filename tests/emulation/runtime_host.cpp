@@ -12,6 +12,10 @@ namespace {
 std::map<char*, size_t> live;
 int errors = 0, countdown = -1;  // allocations that still succeed (-1: all)
 hipError_t last = hipSuccess;    // until it is asked for
+intptr_t handles = 0;            // streams and graphs made
+bool capturing = false;
+int captures = 0, events_captured = 0;
+std::vector<hipStream_t> launched;  // streams of the graph launches
 
 hipError_t take(void** p, size_t bytes) {
   if (countdown == 0) return last = hipErrorOutOfMemory;
@@ -57,20 +61,20 @@ hipError_t hipEventCreate(hipEvent_t* e) { return *e = (hipEvent_t)1, hipSuccess
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float* f, hipEvent_t, hipEvent_t) { return *f = 0, hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return events_captured += capturing, hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = (hipStream_t)1, hipSuccess; }
-hipError_t hipExtStreamCreateWithCUMask(hipStream_t* s, uint32_t, const uint32_t*) { return *s = (hipStream_t)1, hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = (hipStream_t)++handles, hipSuccess; }
+hipError_t hipExtStreamCreateWithCUMask(hipStream_t* s, uint32_t, const uint32_t*) { return *s = (hipStream_t)++handles, hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
-hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { return *g = (hipGraph_t)1, hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return events_captured += capturing, hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return ++captures, capturing = true, hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { return capturing = false, *g = (hipGraph_t)1, hipSuccess; }
 hipError_t hipGraphCreate(hipGraph_t* g, unsigned) { return *g = (hipGraph_t)1, hipSuccess; }
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
 hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) { return *e = (hipGraphExec_t)1, hipSuccess; }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t s) { return launched.push_back(s), hipSuccess; }
 hipError_t hipGraphAddChildGraphNode(hipGraphNode_t*, hipGraph_t, const hipGraphNode_t*, size_t, hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphAddEventRecordNode(hipGraphNode_t*, hipGraph_t, const hipGraphNode_t*, size_t, hipEvent_t) { return hipSuccess; }
 }
@@ -113,6 +117,23 @@ hipError_t launch_block_assemble(const BlockAssembleArgs&, hipStream_t) { return
 hipError_t launch_trmm_lower(const double*, const double*, double*, int, int, hipStream_t) { return hipSuccess; }
 }  // namespace lk
 
+// n-point designs of one dimension, evaluated in batches of one design
+struct Bench {
+  lk::Runtime rt{0};
+  std::vector<double> x = std::vector<double>(300, 0.5), g = std::vector<double>(1, 0.3);
+  int design(int n) { return rt.add_problem(x.data(), n, 1, x.data(), x.data(), 1, 0, 0); }
+  void batch(int id, int items) {
+    std::vector<lk::EvalRequest> r(items);
+    for (auto& q : r) {
+      q.problem = id;
+      q.gamma = g.data();
+      q.gamma_n = 1;
+    }
+    std::vector<lk::EvalResult> res;
+    rt.evaluate(r, true, res);
+  }
+};
+
 // A batch, then one that needs a larger pool and larger tables and whose
 // allocation number `fail` (from 0) fails, then the first batch, another that
 // fits the old pool, and the large one.  Returns the accesses to and frees of
@@ -121,21 +142,10 @@ hipError_t launch_trmm_lower(const double*, const double*, double*, int, int, hi
 static int failed_growth(int fail) {
   bool threw = false;
   {
-    lk::Runtime rt(0);
-    rt.use_graph = false;
-    std::vector<double> x(300, 0.5), g(1, 0.3);
-    const int a = rt.add_problem(x.data(), 100, 1, x.data(), x.data(), 1, 0, 0);
-    const int b = rt.add_problem(x.data(), 60, 1, x.data(), x.data(), 1, 0, 0);
-    auto batch = [&](int id, int items) {
-      std::vector<lk::EvalRequest> r(items);
-      for (auto& q : r) {
-        q.problem = id;
-        q.gamma = g.data();
-        q.gamma_n = 1;
-      }
-      std::vector<lk::EvalResult> res;
-      rt.evaluate(r, true, res);
-    };
+    Bench t;
+    t.rt.use_graph = false;
+    const int a = t.design(100), b = t.design(60);
+    auto batch = [&](int id, int items) { t.batch(id, items); };
     batch(a, 1);
     countdown = fail;
     try {
@@ -152,7 +162,31 @@ static int failed_growth(int fail) {
   return threw ? errors + 1000 * (int)live.size() : -1;
 }
 
+// Graphs of batches in parts: "captures events-in-captures launches
+// distinct-streams" after a batch in four parts, after the same again, and
+// after another design in two
+static void split_batches() {
+  Bench t;
+  auto report = [&] {
+    std::sort(launched.begin(), launched.end());
+    const int streams = int(std::unique(launched.begin(), launched.end()) - launched.begin());
+    std::printf("%d %d %d %d\n", captures, events_captured, (int)launched.size(), streams);
+    launched.clear();
+    captures = 0;
+  };
+  const int a = t.design(100), b = t.design(200);
+  t.batch(a, 32);
+  report();
+  t.batch(a, 32);
+  report();
+  t.batch(b, 16);
+  report();
+}
+
 int main(int, char** argv) {
-  std::printf("%d\n", failed_growth(std::atoi(argv[1])));
+  if (std::string(argv[1]) == "split")
+    split_batches();
+  else
+    std::printf("%d\n", failed_growth(std::atoi(argv[1])));
   return 0;
 }
