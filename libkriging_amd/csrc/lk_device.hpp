@@ -714,7 +714,9 @@ __device__ inline double sload(const double* p) { return *(const __attribute__((
 // column: read by the scalar unit, an operand of the FMA.  Batches of 16, the
 // next one's loads in flight (n = 8192: 106 -> 81 us, n = 4096: 45 -> 31; with
 // four columns always computed from broadcast lanes the loop was bound by
-// its instructions).
+// its instructions).  In batches too: 64 x n = 1024 55.7 -> 51.0 us, 32 slots
+// 28.8 -> 26.0, 16 x n = 2048 61 -> 53 (the same batches of 16 by lane
+// broadcasts: 51.6 .. 53.9, 26.0 .. 26.9, 54 .. 58).
 __device__ inline double lower_matvec_one(const double* __restrict__ Wr, int ld, int kend, int w,
                                           const double* __restrict__ col) {
   constexpr int U = 16, STEP = MV_W * U;
